@@ -124,7 +124,10 @@ int swe_hip_eval_rhs32(swe_hip_ctx *ctx, int member, const float *K, float *F);
 #define SWE_HIP_KERNEL_AUTO 0   /* single state: RESIDENT up to 256 nodes
                                    per compute unit (with a
                                    Hilbert device order unless another is
-                                   asked for), else PAIR with a 31-point
+                                   asked for), in fast mode its streaming
+                                   form beyond that as far as a tile's rows
+                                   fit the LDS (about 4000 nodes per compute
+                                   unit), else PAIR with a 31-point
                                    stencil, else QUADW (FP32: see below)     */
 #define SWE_HIP_KERNEL_QUAD 1   /* FP32 single state: 4 lanes per node
                                    splitting the stencil slots (fast mode)   */
@@ -152,7 +155,8 @@ int swe_hip_eval_rhs32(swe_hip_ctx *ctx, int member, const float *K, float *F);
                                    nodes keeping the tile's weights,
                                    positions, geometry, H and D in registers
                                    and waiting, before every stage, for the
-                                   tiles it exchanges rows with; same
+                                   tiles it exchanges rows with (fast mode:
+                                   stencil sums on the matrix cores); same
                                    arithmetic as PAIR (FP32: LANE), bitwise
                                    in both modes.  A wait
                                    that times out (the state is then
@@ -176,8 +180,9 @@ int swe_hip_eval_rhs32(swe_hip_ctx *ctx, int member, const float *K, float *F);
  * partial sums added across the group (fast mode only).  RESIDENT = the
  * resident whole-step kernel with one lane per node (both modes).  AUTO =
  * RESIDENT up to 256 nodes per compute unit, else LANE in exact
- * mode, and in fast mode PAIR up to 262144 nodes (one lane per node would
- * leave the chip under-filled), LANE above.  QUADW is an FP64 mapping. */
+ * mode, and in fast mode the resident kernel's streaming form with the sums
+ * of PAIR up to 262144 nodes, of LANE above (PAIR and LANE themselves where
+ * it does not fit).  QUADW is an FP64 mapping. */
 #define SWE_HIP_ORDER_HOST 0    /* device node order = the caller's (RCM)    */
 #define SWE_HIP_ORDER_MORTON 1  /* device node order = 3-D Morton curve      */
 #define SWE_HIP_ORDER_HILBERT 2 /* device node order = 3-D Hilbert curve     */

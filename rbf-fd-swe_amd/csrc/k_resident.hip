@@ -1,126 +1,36 @@
-// Whole RK4 steps of one single-state mesh in one cooperative launch: each
-// workgroup owns one tile of consecutive nodes for the whole launch and
-// keeps everything static about them -- 31 x 4 weights, stencil positions,
-// geometry -- and its running H and D in registers; per stage it waits for
-// the tiles it exchanges rows with, copies its tile's distinct neighbour
-// states into LDS, evaluates the stencil sums, the RHS and the stage update
-// of its nodes, publishes their new state and its own stage count.  The
-// static stencil data (1252 of the 1388 bytes a node costs one stage launch
-// of the stage kernels) is read once per launch instead of once per stage.
+// Whole RK4 steps of one single-state mesh in one cooperative launch, exact
+// mode (fast mode: k_units.hip, k_units32.hip, whose matrix instructions fuse
+// every multiply-add): each workgroup owns one tile of consecutive nodes for
+// the whole launch and keeps everything static about them -- 31 x 4 weights,
+// stencil positions, geometry -- and its running H and D in registers; per
+// stage it waits for the tiles it exchanges rows with, copies its tile's
+// distinct neighbour states into LDS, evaluates the stencil sums, the RHS and
+// the stage update of its nodes, publishes their new state and its own stage
+// count.  The static stencil data (1252 of the 1388 bytes a node costs one
+// stage launch of the stage kernels) is read once per launch instead of once
+// per stage.
 //
 // Same sums, same order and same stage arithmetic as k_stage_pair and
-// k_stage_ptile (bitwise in exact mode and in fast mode); the RK stages and
-// constants of RK_substep (rk4_rbffd_swe.c:30-72) and the fused stage
-// kernels: stage 0 gathers H and writes Ka, stage 1 Ka -> Kb, stage 2
-// Kb -> Ka, stage 3 Ka -> H.
+// k_stage_ptile, bitwise; the RK stages and constants of RK_substep
+// (rk4_rbffd_swe.c:30-72) and the fused stage kernels: stage 0 gathers H and
+// writes Ka, stage 1 Ka -> Kb, stage 2 Kb -> Ka, stage 3 Ka -> H.
 //
-// Cross-workgroup visibility: the L2 caches of the 8 XCDs are not coherent
-// with each other, so every state access another workgroup depends on is
-// agent-coherent (direct-to-LDS loads and buffer stores with the sc1 cache
-// policy; the published states are small and live in the last-level
-// cache), and the
-// stage counts are agent-scope atomics written after the state stores
-// have completed.  Every wait is bounded (spin_limit polls): a workgroup
-// that exceeds it raises the abort flag, which every waiting workgroup
-// sees, and all of them leave the kernel; the host reports the launch as
-// failed.
-#include "swe_ctx.h"
+// The exchange between workgroups is res_sync.h's.
+#include "res_sync.h"
 
 #include <algorithm>
 
 namespace swe {
 
-// Synchronisation state (unsigned words), zeroed before the first launch of
-// a context and when the counts near 2^31: word 0 is the abort flag, then
-// one 128-byte line per tile holding the number of stages the tile has
-// completed, counted on across launches.  Instead of a grid-wide barrier a
-// tile waits, before each stage, for the tiles it exchanges rows with (the
-// owners of the rows it reads and the tiles that read its rows): they have
-// then finished the previous stage, so the rows it reads are final and
-// nobody still reads the buffer it is about to overwrite.  Neighbouring
-// tiles are at most one stage apart and no wait depends on a later stage.
-constexpr int kResLine = 32;
-
 struct DevResident {
+    DevResSync y;
     double *H, *Ka, *Kb;
-    unsigned *sync;     // [1 + ntiles][kResLine]
-    unsigned *host_abort;   // pinned host word, set on a time-out
-    const int *nbrs;    // [ntiles][kResMaxNbrs] tiles to wait for, -1 padded
     double c[4];        // K = H + c F (dt/2, dt/2, dt); stage 3: H += c D (dt/6)
     double dcoef[4];    // D += dcoef F (0: D = F, 2, 2, 1)
     int nsteps;
     int bytes;          // bytes of each state buffer (buffer-resource bound)
     int lds_rows;       // row halves the LDS holds (2 x the largest tile's rows)
-    unsigned stage0;    // stages completed before this launch
-    unsigned spin_limit;
 };
-
-__device__ __forceinline__ unsigned ld_agent(const unsigned *p)
-{
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-__device__ __forceinline__ void st_agent(unsigned *p, unsigned v)
-{
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// Wave 0 polls the neighbour tiles' stage counts (one per lane) until every
-// one has reached `need`; false once any wait in the grid was aborted.
-__device__ bool res_wait(const DevResident &r, int tile, unsigned need)
-{
-    __shared__ int ok;
-    if (threadIdx.x < 64) {
-        const int u = r.nbrs[tile * kResMaxNbrs + (int)threadIdx.x];
-        const unsigned *f = r.sync + (long)(1 + (u >= 0 ? u : tile)) * kResLine;
-        int good = 1;
-        unsigned polls = 0;
-        while (!__all(u < 0 || ld_agent(f) >= need)) {
-            if (++polls > r.spin_limit || ld_agent(r.sync)) {
-                if (threadIdx.x == 0) {
-                    st_agent(r.sync, 1u);
-                    __hip_atomic_store(r.host_abort, 1u, __ATOMIC_RELAXED,
-                                       __HIP_MEMORY_SCOPE_SYSTEM);
-                }
-                good = 0;
-                break;
-            }
-            __builtin_amdgcn_s_sleep(1);
-        }
-        if (threadIdx.x == 0)
-            ok = good;
-    }
-    __syncthreads();
-    return ok != 0;
-}
-
-// Every wave's state stores are complete, then the tile's count moves on.
-__device__ __forceinline__ void res_publish(const DevResident &r, int tile, unsigned done)
-{
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-    if (threadIdx.x == 0)
-        st_agent(r.sync + (long)(1 + tile) * kResLine, done);
-}
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t state_rsrc(const double *p, int bytes)
-{
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<double *>(p), (short)0, bytes,
-                                             0x00020000);
-}
-
-constexpr int kSc1 = 16;   // cache policy: agent-coherent access
-
-typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-
-// 16 bytes per lane from global memory straight into LDS, agent-coherent
-// (global_load_lds_dwordx4 ... sc1): lane l's bytes land at lds + 16 l, lds
-// being wave-uniform; the wave's vmcnt counts the load until they are there.
-__device__ __forceinline__ void dma16_sc1(const void *src, void *lds)
-{
-    __builtin_amdgcn_global_load_lds(src, (__attribute__((address_space(3))) void *)lds, 16, 0,
-                                     kSc1);
-}
 
 // Copies rows [0, count) of 16 bytes from byte offsets offs[] of `base`
 // into rows[], one direct-to-LDS load per wave and 64 rows, then waits for
@@ -145,7 +55,7 @@ __device__ __forceinline__ void store_sc1(__amdgpu_buffer_rsrc_t r, int off_byte
     __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), r, off_bytes, 0, kSc1);
 }
 
-template <bool EXACT, int NNBR>
+template <int NNBR>
 __global__ __launch_bounds__(64 * kResMaxWaves) void k_steps_resident(DevMesh m, DevTiles tl,
                                                                       DevResident r)
 {
@@ -189,7 +99,7 @@ __global__ __launch_bounds__(64 * kResMaxWaves) void k_steps_resident(DevMesh m,
     double2 H = *reinterpret_cast<const double2 *>(r.H + 4L * node + 2 * k);
     double2 D = make_double2(0.0, 0.0);
     double2 K = H;   // the state the next stage gathers, this lane's part
-    unsigned stage = r.stage0;
+    unsigned stage = r.y.stage0;
     bool alive = true;
 
     for (int step = 0; step < r.nsteps && alive; ++step) {
@@ -199,7 +109,7 @@ __global__ __launch_bounds__(64 * kResMaxWaves) void k_steps_resident(DevMesh m,
                 return;
             const double *src = s == 0 ? r.H : (s == 2 ? r.Kb : r.Ka);
             double *out = s == 0 ? r.Ka : (s == 1 ? r.Kb : (s == 2 ? r.Ka : r.H));
-            if (!(alive = res_wait(r, tile, stage)))   // also: offsets written, rows free
+            if (!(alive = res_wait(r.y, tile, stage)))   // also: offsets written, rows free
                 return;
             copy_rows_sc1(src, offs, rows, 2 * ucount);
             __syncthreads();
@@ -211,10 +121,10 @@ __global__ __launch_bounds__(64 * kResMaxWaves) void k_steps_resident(DevMesh m,
                 const int pos = (int)((j & 1) ? (wv >> 16) : (wv & 0xffffu));
                 const double2 sv = rows[2 * pos + k];
                 const double o0 = pair_swap(w[j].x), o1 = pair_swap(w[j].y);
-                a0 = madd<EXACT>(a0, w[j].x, sv.x); a1 = madd<EXACT>(a1, w[j].y, sv.x);
-                a2 = madd<EXACT>(a2, o0, sv.x);     a3 = madd<EXACT>(a3, o1, sv.x);
-                b0 = madd<EXACT>(b0, w[j].x, sv.y); b1 = madd<EXACT>(b1, w[j].y, sv.y);
-                b2 = madd<EXACT>(b2, o0, sv.y);     b3 = madd<EXACT>(b3, o1, sv.y);
+                a0 = madd<true>(a0, w[j].x, sv.x); a1 = madd<true>(a1, w[j].y, sv.x);
+                a2 = madd<true>(a2, o0, sv.x);     a3 = madd<true>(a3, o1, sv.x);
+                b0 = madd<true>(b0, w[j].x, sv.y); b1 = madd<true>(b1, w[j].y, sv.y);
+                b2 = madd<true>(b2, o0, sv.y);     b3 = madd<true>(b3, o1, sv.y);
             });
             const double ax = k ? a2 : a0, ay = k ? a3 : a1, az = k ? a0 : a2, al = k ? a1 : a3;
             const double bx = k ? b2 : b0, by = k ? b3 : b1, bz = k ? b0 : b2, bl = k ? b1 : b3;
@@ -247,40 +157,36 @@ __global__ __launch_bounds__(64 * kResMaxWaves) void k_steps_resident(DevMesh m,
             // the stage update of stage_update_pair, on registers
             if constexpr (s == 0) {
                 D = make_double2(f0, f1);
-                K = make_double2(axpy<EXACT>(H.x, r.c[0], f0), axpy<EXACT>(H.y, r.c[0], f1));
+                K = make_double2(axpy<true>(H.x, r.c[0], f0), axpy<true>(H.y, r.c[0], f1));
             } else if constexpr (s == 1 || s == 2) {
-                D = make_double2(axpy<EXACT>(D.x, r.dcoef[s], f0), axpy<EXACT>(D.y, r.dcoef[s], f1));
-                K = make_double2(axpy<EXACT>(H.x, r.c[s], f0), axpy<EXACT>(H.y, r.c[s], f1));
+                D = make_double2(axpy<true>(D.x, r.dcoef[s], f0), axpy<true>(D.y, r.dcoef[s], f1));
+                K = make_double2(axpy<true>(H.x, r.c[s], f0), axpy<true>(H.y, r.c[s], f1));
             } else {
-                const double d0 = axpy<EXACT>(D.x, r.dcoef[3], f0);
-                const double d1 = axpy<EXACT>(D.y, r.dcoef[3], f1);
-                H = make_double2(axpy<EXACT>(H.x, r.c[3], d0), axpy<EXACT>(H.y, r.c[3], d1));
+                const double d0 = axpy<true>(D.x, r.dcoef[3], f0);
+                const double d1 = axpy<true>(D.y, r.dcoef[3], f1);
+                H = make_double2(axpy<true>(H.x, r.c[3], d0), axpy<true>(H.y, r.c[3], d1));
                 K = H;
             }
             if (live)
                 store_sc1(state_rsrc(out, r.bytes), e, K);
-            res_publish(r, tile, ++stage);
+            res_publish(r.y, tile, ++stage);
         });
     }
 }
 
 // FP32 (the reference's RUN_32BIT type), one lane per node: the sums,
-// RHS and stage update of k_stage_lane32 (bitwise equal to it in both
-// modes, and in exact mode to the reference's FP32 build), the tile's rows
+// RHS and stage update of k_stage_lane32 (bitwise equal to it and to the
+// reference's FP32 build), the tile's rows
 // as 16-byte float4 in LDS, the same neighbour waits.
 struct DevResident32 {
+    DevResSync y;
     float *H, *Ka, *Kb;
-    unsigned *sync;
-    unsigned *host_abort;
-    const int *nbrs;
     float c[3];         // K = H + c F: (float)(dt/2.0), (float)(dt/2.0), dt
     double c6;          // stage 3: H += (dt/6.0) D in double
     float dcoef[4];     // D += dcoef F (0: D = F, 2, 2, 1)
     int nsteps;
     int bytes;
     int lds_rows;       // rows the LDS holds (the largest tile's)
-    unsigned stage0;
-    unsigned spin_limit;
 };
 
 __device__ __forceinline__ void store_sc1_f4(__amdgpu_buffer_rsrc_t r, int off_bytes, float4 v)
@@ -288,12 +194,7 @@ __device__ __forceinline__ void store_sc1_f4(__amdgpu_buffer_rsrc_t r, int off_b
     __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), r, off_bytes, 0, kSc1);
 }
 
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t state_rsrc32(const float *p, int bytes)
-{
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(p), (short)0, bytes, 0x00020000);
-}
-
-template <bool EXACT, int NNBR>
+template <int NNBR>
 __global__ __launch_bounds__(64 * kResMaxWaves) void k_steps_resident32(DevMesh32 m, DevTiles tl,
                                                                         DevResident32 r)
 {
@@ -335,13 +236,8 @@ __global__ __launch_bounds__(64 * kResMaxWaves) void k_steps_resident32(DevMesh3
     float4 H = *reinterpret_cast<const float4 *>(r.H + 4L * node);
     float4 D = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     float4 K = H;
-    unsigned stage = r.stage0;
+    unsigned stage = r.y.stage0;
     bool alive = true;
-    DevResident sync_view{};   // the fields res_wait and res_publish read
-    sync_view.sync = r.sync;
-    sync_view.host_abort = r.host_abort;
-    sync_view.nbrs = r.nbrs;
-    sync_view.spin_limit = r.spin_limit;
 
     for (int step = 0; step < r.nsteps && alive; ++step) {
         static_for<4>([&](auto sc) {
@@ -350,7 +246,7 @@ __global__ __launch_bounds__(64 * kResMaxWaves) void k_steps_resident32(DevMesh3
                 return;
             const float *src = s == 0 ? r.H : (s == 2 ? r.Kb : r.Ka);
             float *out = s == 0 ? r.Ka : (s == 1 ? r.Kb : (s == 2 ? r.Ka : r.H));
-            if (!(alive = res_wait(sync_view, tile, stage)))   // also: offsets written, rows free
+            if (!(alive = res_wait(r.y, tile, stage)))   // also: offsets written, rows free
                 return;
             copy_rows_sc1(src, offs, rows32, ucount);
             __syncthreads();
@@ -360,39 +256,39 @@ __global__ __launch_bounds__(64 * kResMaxWaves) void k_steps_resident32(DevMesh3
                 const unsigned pv = pw[j >> 1];
                 const float4 sv = rows32[(j & 1) ? (pv >> 16) : (pv & 0xffffu)];
                 const float4 wj = w[j];
-                S.dudx = madd32<EXACT>(S.dudx, wj.x, sv.x); S.dvdx = madd32<EXACT>(S.dvdx, wj.x, sv.y);
-                S.dwdx = madd32<EXACT>(S.dwdx, wj.x, sv.z); S.dhdx = madd32<EXACT>(S.dhdx, wj.x, sv.w);
-                S.dudy = madd32<EXACT>(S.dudy, wj.y, sv.x); S.dvdy = madd32<EXACT>(S.dvdy, wj.y, sv.y);
-                S.dwdy = madd32<EXACT>(S.dwdy, wj.y, sv.z); S.dhdy = madd32<EXACT>(S.dhdy, wj.y, sv.w);
-                S.dudz = madd32<EXACT>(S.dudz, wj.z, sv.x); S.dvdz = madd32<EXACT>(S.dvdz, wj.z, sv.y);
-                S.dwdz = madd32<EXACT>(S.dwdz, wj.z, sv.z); S.dhdz = madd32<EXACT>(S.dhdz, wj.z, sv.w);
-                S.lu = madd32<EXACT>(S.lu, wj.w, sv.x); S.lv = madd32<EXACT>(S.lv, wj.w, sv.y);
-                S.lw = madd32<EXACT>(S.lw, wj.w, sv.z); S.lh = madd32<EXACT>(S.lh, wj.w, sv.w);
+                S.dudx = madd32<true>(S.dudx, wj.x, sv.x); S.dvdx = madd32<true>(S.dvdx, wj.x, sv.y);
+                S.dwdx = madd32<true>(S.dwdx, wj.x, sv.z); S.dhdx = madd32<true>(S.dhdx, wj.x, sv.w);
+                S.dudy = madd32<true>(S.dudy, wj.y, sv.x); S.dvdy = madd32<true>(S.dvdy, wj.y, sv.y);
+                S.dwdy = madd32<true>(S.dwdy, wj.y, sv.z); S.dhdy = madd32<true>(S.dhdy, wj.y, sv.w);
+                S.dudz = madd32<true>(S.dudz, wj.z, sv.x); S.dvdz = madd32<true>(S.dvdz, wj.z, sv.y);
+                S.dwdz = madd32<true>(S.dwdz, wj.z, sv.z); S.dhdz = madd32<true>(S.dhdz, wj.z, sv.w);
+                S.lu = madd32<true>(S.lu, wj.w, sv.x); S.lv = madd32<true>(S.lv, wj.w, sv.y);
+                S.lw = madd32<true>(S.lw, wj.w, sv.z); S.lh = madd32<true>(S.lh, wj.w, sv.w);
             });
             float F[4];
             rhs_point32(S, K.x, K.y, K.z, K.w, g, m.gh0, F);
             // the stage update of stage_update32, on registers
             if constexpr (s == 0) {
                 D = make_float4(F[0], F[1], F[2], F[3]);
-                K = make_float4(axpy32<EXACT>(H.x, r.c[0], F[0]), axpy32<EXACT>(H.y, r.c[0], F[1]),
-                                axpy32<EXACT>(H.z, r.c[0], F[2]), axpy32<EXACT>(H.w, r.c[0], F[3]));
+                K = make_float4(axpy32<true>(H.x, r.c[0], F[0]), axpy32<true>(H.y, r.c[0], F[1]),
+                                axpy32<true>(H.z, r.c[0], F[2]), axpy32<true>(H.w, r.c[0], F[3]));
             } else {
-                D = make_float4(axpy32<EXACT>(D.x, r.dcoef[s], F[0]),
-                                axpy32<EXACT>(D.y, r.dcoef[s], F[1]),
-                                axpy32<EXACT>(D.z, r.dcoef[s], F[2]),
-                                axpy32<EXACT>(D.w, r.dcoef[s], F[3]));
+                D = make_float4(axpy32<true>(D.x, r.dcoef[s], F[0]),
+                                axpy32<true>(D.y, r.dcoef[s], F[1]),
+                                axpy32<true>(D.z, r.dcoef[s], F[2]),
+                                axpy32<true>(D.w, r.dcoef[s], F[3]));
                 if constexpr (s == 3) {
-                    H = make_float4(update_h32<EXACT>(H.x, r.c6, D.x), update_h32<EXACT>(H.y, r.c6, D.y),
-                                    update_h32<EXACT>(H.z, r.c6, D.z), update_h32<EXACT>(H.w, r.c6, D.w));
+                    H = make_float4(update_h32<true>(H.x, r.c6, D.x), update_h32<true>(H.y, r.c6, D.y),
+                                    update_h32<true>(H.z, r.c6, D.z), update_h32<true>(H.w, r.c6, D.w));
                     K = H;
                 } else {
-                    K = make_float4(axpy32<EXACT>(H.x, r.c[s], F[0]), axpy32<EXACT>(H.y, r.c[s], F[1]),
-                                    axpy32<EXACT>(H.z, r.c[s], F[2]), axpy32<EXACT>(H.w, r.c[s], F[3]));
+                    K = make_float4(axpy32<true>(H.x, r.c[s], F[0]), axpy32<true>(H.y, r.c[s], F[1]),
+                                    axpy32<true>(H.z, r.c[s], F[2]), axpy32<true>(H.w, r.c[s], F[3]));
                 }
             }
             if (live)
-                store_sc1_f4(state_rsrc32(out, r.bytes), e, K);
-            res_publish(sync_view, tile, ++stage);
+                store_sc1_f4(state_rsrc(out, r.bytes), e, K);
+            res_publish(r.y, tile, ++stage);
         });
     }
 }
@@ -404,46 +300,41 @@ __global__ void k_res_clear(unsigned *p, int words)
         p[i] = 0u;
 }
 
-namespace {
-
-template <bool EX>
-void *resident_kernel(bool fp32)
+static void *resident_kernel(bool fp32)
 {
-    return fp32 ? reinterpret_cast<void *>(&k_steps_resident32<EX, 31>)
-                : reinterpret_cast<void *>(&k_steps_resident<EX, 31>);
+    return fp32 ? reinterpret_cast<void *>(&k_steps_resident32<31>)
+                : reinterpret_cast<void *>(&k_steps_resident<31>);
 }
-
-}  // namespace
 
 long resident_sync_bytes(int ntiles) { return (1L + ntiles) * kResLine * sizeof(unsigned); }
 
-// LDS budget of both kernel instances and a check that one workgroup per
+// LDS budget of the kernel and a check that one workgroup per
 // tile can be resident at once (the cooperative launch needs it).  The
 // budget is a property of the kernel, shared by every context: it is set to
 // what the largest tile any context may build needs (kResMaxRows rows), so
 // that a context created later never lowers it below an earlier one's use.
 int resident_prepare(swe_hip_ctx *c, std::string *err)
 {
+    if (c->units.ntiles > 0)
+        return units_prepare(c, err);
     const int lds_max = kResMaxRows * (c->fp32 ? (int)(sizeof(float4) + sizeof(int))
                                                : 2 * (int)(sizeof(double2) + sizeof(int)));
     if (c->res_lds > lds_max) {
         *err = "resident kernel: LDS budget";
         return SWE_HIP_EDEVICE;
     }
-    for (bool ex : {false, true}) {
-        void *fn = ex ? resident_kernel<true>(c->fp32) : resident_kernel<false>(c->fp32);
-        if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, lds_max)
-            != hipSuccess) {
-            *err = "resident kernel: LDS budget";
-            return SWE_HIP_EDEVICE;
-        }
-        int per_cu = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, c->res_block, c->res_lds)
-                != hipSuccess
-            || (long)per_cu * c->ncu < c->tiles.ntiles) {
-            *err = "resident kernel: the launch cannot be co-resident on this device";
-            return SWE_HIP_EDEVICE;
-        }
+    void *fn = resident_kernel(c->fp32);
+    if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, lds_max)
+        != hipSuccess) {
+        *err = "resident kernel: LDS budget";
+        return SWE_HIP_EDEVICE;
+    }
+    int per_cu = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, c->res_block, c->res_lds)
+            != hipSuccess
+        || (long)per_cu * c->ncu < c->tiles.ntiles) {
+        *err = "resident kernel: the launch cannot be co-resident on this device";
+        return SWE_HIP_EDEVICE;
     }
     return 0;
 }
@@ -486,23 +377,29 @@ int resident_launch(swe_hip_ctx *c, int nsteps, std::string *err)
 {
     const long long stages = 4LL * nsteps;
     if (c->res_stages == 0 || c->res_stages + stages > (1LL << 31)) {
-        const int words = (int)(resident_sync_bytes(c->tiles.ntiles) / sizeof(unsigned));
+        const int words = (int)(resident_sync_bytes(resident_tiles(c)) / sizeof(unsigned));
         k_res_clear<<<(words + 255) / 256, 256, 0, c->stream>>>(
             reinterpret_cast<unsigned *>(c->d_res_sync), words);
         c->res_stages = 0;
     }
+    DevResSync y{};
+    y.sync = reinterpret_cast<unsigned *>(c->d_res_sync);
+    y.host_abort = c->d_res_abort;
+    y.nbrs = c->d_res_nbrs;
+    y.stage0 = (unsigned)c->res_stages;
+    y.spin_limit = c->res_spin;
     DevTiles tl = tiles_of(c, 1);
-    void *fn = exact(c) ? resident_kernel<true>(c->fp32) : resident_kernel<false>(c->fp32);
+    void *fn = resident_kernel(c->fp32);
     hipError_t e = hipSuccess;
-    if (c->fp32) {
+    if (c->units.ntiles > 0) {
+        e = units_launch(c, nsteps, y);
+    } else if (c->fp32) {
         DevMesh32 m = mesh32_of(c);
         DevResident32 r{};
+        r.y = y;
         r.H = c->f_H;
         r.Ka = c->f_Ka;
         r.Kb = c->f_Kb;
-        r.sync = reinterpret_cast<unsigned *>(c->d_res_sync);
-        r.host_abort = c->d_res_abort;
-        r.nbrs = c->d_res_nbrs;
         // the constants of the FP32 stage kernels (rk4_rbffd_swe.c:123-186)
         const float dt = (float)c->dt;
         r.c[0] = (float)(dt / 2.0); r.c[1] = (float)(dt / 2.0); r.c[2] = dt;
@@ -510,29 +407,23 @@ int resident_launch(swe_hip_ctx *c, int nsteps, std::string *err)
         r.dcoef[0] = 0.0f; r.dcoef[1] = 2.0f; r.dcoef[2] = 2.0f; r.dcoef[3] = 1.0f;
         r.nsteps = nsteps;
         r.bytes = (int)(state_count(c) * (long)sizeof(float));
-        r.spin_limit = c->res_spin;
         r.lds_rows = c->tiles.umax_used;
-        r.stage0 = (unsigned)c->res_stages;
         void *args[] = {&m, &tl, &r};
         e = hipLaunchCooperativeKernel(fn, dim3(c->tiles.ntiles), dim3(c->res_block), args,
                                        (unsigned)c->res_lds, c->stream);
     } else {
         DevMesh m = mesh_of(c);
         DevResident r{};
+        r.y = y;
         r.H = c->d_H;
         r.Ka = c->d_Ka;
         r.Kb = c->d_Kb;
-        r.sync = reinterpret_cast<unsigned *>(c->d_res_sync);
-        r.host_abort = c->d_res_abort;
-        r.nbrs = c->d_res_nbrs;
         const double dt = c->dt;
         r.c[0] = dt / 2.0; r.c[1] = dt / 2.0; r.c[2] = dt; r.c[3] = dt / 6.0;
         r.dcoef[0] = 0.0; r.dcoef[1] = 2.0; r.dcoef[2] = 2.0; r.dcoef[3] = 1.0;
         r.nsteps = nsteps;
         r.bytes = (int)(state_count(c) * (long)sizeof(double));
-        r.spin_limit = c->res_spin;
         r.lds_rows = 2 * c->tiles.umax_used;
-        r.stage0 = (unsigned)c->res_stages;
         void *args[] = {&m, &tl, &r};
         e = hipLaunchCooperativeKernel(fn, dim3(c->tiles.ntiles), dim3(c->res_block), args,
                                        (unsigned)c->res_lds, c->stream);

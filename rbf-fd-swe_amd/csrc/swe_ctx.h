@@ -27,6 +27,13 @@ constexpr int kGraphCount = 4;         // captured step graphs per context
 constexpr int kResMaxWaves = 8;
 constexpr int kResMaxRows = 2560;
 constexpr int kResAutoMinNodes = 1;       // SWE_HIP_KERNEL_AUTO picks it from here
+constexpr int kUnitsMaxLds = 160 * 1024 - 64;   // dynamic LDS of k_steps_units
+// Nodes per compute unit up to which AUTO tries the streaming form of the unit
+// kernels (their own LDS check decides: ~4600 FP64 rows of 32 bytes).  Beyond
+// 256 nodes per unit it beats the stage kernels at every size measured (us per
+// stage, FP64: N = 163842 19.4 against 32.6, 655362 180 against 197; FP32: 7.5
+// against 19.7, 78 against 110).
+constexpr int kUnitsMaxPerCu = 4096;
 constexpr int kResMaxNbrs = 64;           // tiles one tile exchanges rows with (one wave)
 constexpr int kResAutoMinSteps = 4;       // AUTO contexts: shorter calls replay stage graphs
 
@@ -65,6 +72,7 @@ struct SweMesh {
     int order = SWE_HIP_ORDER_HOST;
     int sblk = 0;                 // stencil layout: 0 slot-major, 16 node blocks
     std::vector<int> perm;        // device node -> host node (empty: identity)
+    std::vector<double> h_xyz;    // node coordinates, device order, [3][n]
     std::vector<int> h_nbr;       // host copy of nbr, device order, [nnbr][n]
 };
 
@@ -79,6 +87,22 @@ struct SweTiles {
     int *d_ulist_tile = nullptr;             // [ntiles][kTmemStride] (member-lane kernel)
     double *d_wts_node = nullptr;            // [n][32][4] (member-lane kernel)
     double *d_geo_node = nullptr;            // [n][32] (member-lane kernel)
+};
+
+// Unit records of the matrix-core resident kernel (k_units.hip): tiles of
+// consecutive nodes along a space-filling curve, cut into units of 16.
+struct SweUnits {
+    int ntiles = 0;               // 0: not built
+    int units = 0, rows = 0;      // most units and rows of one tile
+    int waves = 0, lds = 0;       // waves per workgroup, dynamic LDS bytes
+    int mode = 0;                 // UnitMode (units.h)
+    int chains = 1;               // FP32: partial sums per stencil sum, as split32's lanes
+    int pos = 0, geo = 0;         // units whose positions, geometry the LDS holds
+    long long bytes = 0;          // counted in the context's bytes too
+    void *d_wrec = nullptr, *d_grec = nullptr, *d_hd = nullptr;
+    uint4 *d_prec = nullptr;
+    int *d_tile_start = nullptr, *d_unit_start = nullptr, *d_ustart = nullptr;
+    int *d_ulist = nullptr, *d_own_row = nullptr, *d_perm = nullptr;
 };
 
 struct swe_hip_ctx {
@@ -108,6 +132,7 @@ struct swe_hip_ctx {
     SweTiles tiles;              // LDS-staged ensemble kernel (ntiles == 0: unused)
     hipGraphExec_t graphs[swe::kGraphCount] = {};   // 64, 16, 4 and 1 RK steps
     // resident whole-step kernel (kernel == SWE_HIP_KERNEL_RESIDENT)
+    SweUnits units;                   // its matrix-core form (FP64, fast mode)
     int res_block = 0, res_lds = 0;   // threads per workgroup, dynamic LDS bytes
     void *d_res_sync = nullptr;       // abort word + per-tile stage counts
     unsigned *h_res_abort = nullptr;  // pinned: wait time-out flag of the resident launches
@@ -124,6 +149,14 @@ struct swe_hip_ctx {
 };
 
 namespace swe {
+
+struct DevResSync;   // res_sync.h
+
+// Tiles (workgroups) of a context's resident launches.
+inline int resident_tiles(const swe_hip_ctx *c)
+{
+    return c->units.ntiles > 0 ? c->units.ntiles : c->tiles.ntiles;
+}
 
 inline bool exact(const swe_hip_ctx *c) { return (c->flags & SWE_HIP_EXACT) != 0; }
 
@@ -162,6 +195,14 @@ long resident_sync_bytes(int ntiles);
 int resident_prepare(swe_hip_ctx *c, std::string *err);
 int resident_steps(swe_hip_ctx *c, int nsteps, std::string *err);
 int resident_check(swe_hip_ctx *c, std::string *err);
+
+// The matrix-core resident kernel: unit records in a kernel order of its own
+// with each tile's list of tiles it reads rows from, the co-residency check,
+// one launch of n steps.
+int units_build(swe_hip_ctx *c, std::vector<std::vector<int>> *nbr_tiles, std::string *err);
+int units_prepare(swe_hip_ctx *c, std::string *err);
+hipError_t units_launch(swe_hip_ctx *c, int nsteps, const DevResSync &y);
+void units_free(swe_hip_ctx *c);
 
 // Looks up this device's no-allocation scratch address (swe_noalloc.hip);
 // the device must be current.  On failure *err says why.

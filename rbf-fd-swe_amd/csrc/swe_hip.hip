@@ -13,6 +13,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <numeric>
 #include <string>
 #include <vector>
 
@@ -316,6 +317,7 @@ void free_ctx(swe_hip_ctx *c)
                     c->tiles.d_wts_node, c->tiles.d_geo_node, c->d_res_sync, c->d_res_nbrs};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
+    units_free(c);
     if (c->h_res_abort) (void)hipHostFree(c->h_res_abort);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     release_mesh(c->mesh);
@@ -546,6 +548,7 @@ int build_mesh(const swe_hip_static *s, int device, int order, int sblk, bool fp
         release_mesh(m);
         return rc;
     }
+    m->h_xyz.assign(geo.begin() + (size_t)G_X * n, geo.begin() + (size_t)(G_X + 3) * n);
     m->perm = std::move(perm);
     m->h_nbr = std::move(nbr);
     *out = m;
@@ -583,15 +586,17 @@ __global__ void k_pack_tile_nodes(DevMesh m, int n, const unsigned short *lidx_n
     geo_node[t] = g;
 }
 
-int build_tiles(swe_hip_ctx *c, int tmax, int umax, std::vector<int> *h_tstart = nullptr,
-                std::vector<int> *h_ustart = nullptr, std::vector<int> *h_ulist = nullptr)
+// Cuts the device node order into tiles: first nodes, offsets of the row
+// lists and the lists themselves (distinct stencil nodes, ascending).
+int cut_tiles(const swe_hip_ctx *c, int tmax, int umax, std::vector<int> &tstart,
+              std::vector<int> &ustart, std::vector<int> &ulist)
 {
     const int n = c->n, W = c->nnbr;
     const std::vector<int> &nbr = c->mesh->h_nbr;
-    std::vector<int> tstart{0}, ustart{0}, ulist;
-    std::vector<unsigned short> lidx((size_t)W * n), lidx_node((size_t)32 * n, 0);
-    std::vector<int> mark(n, -1), pos(n, 0);
-    std::vector<int> cur;
+    tstart.assign(1, 0);
+    ustart.assign(1, 0);
+    ulist.clear();
+    std::vector<int> mark(n, -1), cur;
     int tile = 0, node = 0;
     while (node < n) {
         cur.clear();
@@ -616,9 +621,31 @@ int build_tiles(swe_hip_ctx *c, int tmax, int umax, std::vector<int> *h_tstart =
             ++node;
         }
         std::sort(cur.begin(), cur.end());
-        for (int k = 0; k < (int)cur.size(); ++k)
-            pos[cur[k]] = k;
-        for (int i = first; i < node; ++i) {
+        ulist.insert(ulist.end(), cur.begin(), cur.end());
+        tstart.push_back(node);
+        ustart.push_back((int)ulist.size());
+        ++tile;
+    }
+    return 0;
+}
+
+int build_tiles(swe_hip_ctx *c, int tmax, int umax, std::vector<int> *h_tstart = nullptr,
+                std::vector<int> *h_ustart = nullptr, std::vector<int> *h_ulist = nullptr)
+{
+    const int n = c->n, W = c->nnbr;
+    const std::vector<int> &nbr = c->mesh->h_nbr;
+    std::vector<int> tstart, ustart, ulist;
+    if (int rc = cut_tiles(c, tmax, umax, tstart, ustart, ulist))
+        return rc;
+    const int tile = (int)tstart.size() - 1;
+    std::vector<unsigned short> lidx((size_t)W * n), lidx_node((size_t)32 * n, 0);
+    std::vector<int> mark(n, -1), pos(n, 0);
+    for (int t = 0; t < tile; ++t) {
+        for (int k = ustart[t]; k < ustart[t + 1]; ++k) {
+            mark[ulist[k]] = t;
+            pos[ulist[k]] = k - ustart[t];
+        }
+        for (int i = tstart[t]; i < tstart[t + 1]; ++i) {
             for (int j = 0; j < W; ++j) {
                 const unsigned short l = (unsigned short)pos[nbr[(size_t)j * n + i]];
                 lidx[(size_t)j * n + i] = l;
@@ -628,12 +655,8 @@ int build_tiles(swe_hip_ctx *c, int tmax, int umax, std::vector<int> *h_tstart =
             // spare slot 31: the node's own row in its tile (0xffff if its
             // stencil does not contain it)
             if (W < 32)
-                lidx_node[(size_t)32 * i + 31] = mark[i] == tile ? (unsigned short)pos[i] : 0xffff;
+                lidx_node[(size_t)32 * i + 31] = mark[i] == t ? (unsigned short)pos[i] : 0xffff;
         }
-        ulist.insert(ulist.end(), cur.begin(), cur.end());
-        tstart.push_back(node);
-        ustart.push_back((int)ulist.size());
-        ++tile;
     }
     // fixed-stride copy for the member-lane kernel (tiles of <= kTmemRows rows)
     std::vector<int> ulist_tile;
@@ -688,39 +711,55 @@ int build_tiles(swe_hip_ctx *c, int tmax, int umax, std::vector<int> *h_tstart =
     return rc;
 }
 
-// Resident kernel: for every tile, the tiles it must wait for before a
-// stage -- owners of the rows it reads and tiles that read its rows.
-int resident_neighbours(swe_hip_ctx *c, const std::vector<int> &tstart,
-                        const std::vector<int> &ustart, const std::vector<int> &ulist)
+// Resident kernels: for every tile, the tiles it must wait for before a
+// stage -- owners of the rows it reads (reads[t]) and tiles that read its
+// rows -- at a stride of kResMaxNbrs, -1 padded.
+int resident_neighbours(const std::vector<std::vector<int>> &reads, std::vector<int> *flat)
 {
-    const int nt = (int)tstart.size() - 1;
-    std::vector<int> owner(c->n);
+    const int nt = (int)reads.size();
+    std::vector<std::vector<int>> nb = reads;
     for (int t = 0; t < nt; ++t)
-        for (int i = tstart[t]; i < tstart[t + 1]; ++i)
-            owner[i] = t;
-    std::vector<std::vector<int>> nb(nt);
-    for (int t = 0; t < nt; ++t)
-        for (int k = ustart[t]; k < ustart[t + 1]; ++k) {
-            const int u = owner[ulist[k]];
-            if (u != t) {
-                nb[t].push_back(u);
-                nb[u].push_back(t);
-            }
-        }
-    std::vector<int> flat((size_t)nt * kResMaxNbrs, -1);
+        for (int u : reads[t])
+            nb[u].push_back(t);
+    if (flat)
+        flat->assign((size_t)nt * kResMaxNbrs, -1);
     for (int t = 0; t < nt; ++t) {
         std::sort(nb[t].begin(), nb[t].end());
         nb[t].erase(std::unique(nb[t].begin(), nb[t].end()), nb[t].end());
         if ((int)nb[t].size() > kResMaxNbrs)
             return fail(SWE_HIP_EINVAL, "the resident kernel's tiles exchange rows with more than "
                                         + std::to_string(kResMaxNbrs) + " other tiles");
-        std::copy(nb[t].begin(), nb[t].end(), flat.begin() + (size_t)t * kResMaxNbrs);
+        if (flat)
+            std::copy(nb[t].begin(), nb[t].end(), flat->begin() + (size_t)t * kResMaxNbrs);
     }
+    return 0;
+}
+
+int upload_waits(swe_hip_ctx *c, const std::vector<int> &flat)
+{
     int rc = dev_alloc(&c->bytes, (void **)&c->d_res_nbrs, sizeof(int) * flat.size());
     if (!rc && hipMemcpy(c->d_res_nbrs, flat.data(), sizeof(int) * flat.size(),
                          hipMemcpyHostToDevice) != hipSuccess)
         rc = fail(SWE_HIP_EDEVICE, "resident kernel: neighbour upload");
     return rc;
+}
+
+// The tiles each tile of build_tiles reads rows from.
+std::vector<std::vector<int>> tile_reads(int n, const std::vector<int> &tstart,
+                                         const std::vector<int> &ustart,
+                                         const std::vector<int> &ulist)
+{
+    const int nt = (int)tstart.size() - 1;
+    std::vector<int> owner(n);
+    for (int t = 0; t < nt; ++t)
+        for (int i = tstart[t]; i < tstart[t + 1]; ++i)
+            owner[i] = t;
+    std::vector<std::vector<int>> reads(nt);
+    for (int t = 0; t < nt; ++t)
+        for (int k = ustart[t]; k < ustart[t + 1]; ++k)
+            if (owner[ulist[k]] != t)
+                reads[t].push_back(owner[ulist[k]]);
+    return reads;
 }
 
 }  // namespace
@@ -938,7 +977,8 @@ int swe_hip_create_ex(const swe_hip_static *s, const swe_hip_options *o, swe_hip
     if (o->kernel == SWE_HIP_KERNEL_AUTO) {
         c->kernel = m->nnbr == 31 ? SWE_HIP_KERNEL_PAIR : SWE_HIP_KERNEL_QUADW;
         if (!fp32 && o->members == 1 && !o->tiled && m->nnbr == 31 && m->n >= kResAutoMinNodes
-            && m->n <= 32 * kResMaxWaves * c->ncu) {
+            && (m->n <= 32 * kResMaxWaves * c->ncu
+                || (!(o->flags & SWE_HIP_EXACT) && m->n <= kUnitsMaxPerCu * c->ncu))) {
             c->kernel = SWE_HIP_KERNEL_RESIDENT;
             c->res_auto = true;
         }
@@ -961,13 +1001,18 @@ int swe_hip_create_ex(const swe_hip_static *s, const swe_hip_options *o, swe_hip
         // the resident kernel (both modes; its single stages are the lane
         // kernel's) over the same node range as in FP64
         if (o->kernel == SWE_HIP_KERNEL_AUTO && m->nnbr == 31 && m->n >= kResAutoMinNodes
-            && m->n <= 32 * kResMaxWaves * c->ncu) {
+            && (m->n <= 32 * kResMaxWaves * c->ncu
+                || (!(o->flags & SWE_HIP_EXACT) && m->n <= kUnitsMaxPerCu * c->ncu))) {
             k = SWE_HIP_KERNEL_RESIDENT;
             c->res_auto = true;
         }
         c->kernel = k;
         c->split32 = k == SWE_HIP_KERNEL_PAIR ? 2 : k == SWE_HIP_KERNEL_QUAD ? 4
                    : k == SWE_HIP_KERNEL_OCT ? 8 : 1;
+        // the single stages (drop-in substeps, RHS) of an AUTO context beyond
+        // the lane-per-node resident kernel's sizes keep two lanes per node
+        if (c->res_auto && m->n > 32 * kResMaxWaves * c->ncu && fast_auto == SWE_HIP_KERNEL_PAIR)
+            c->split32 = 2;
     }
     c->prefetch = o->prefetch;
     c->tile_nodes = o->tile_nodes;
@@ -1003,6 +1048,36 @@ int swe_hip_create_ex(const swe_hip_static *s, const swe_hip_options *o, swe_hip
         rc = build_tiles(c, c->tile_nodes, 4 * c->tile_nodes);
     }
     if (!rc && c->kernel == SWE_HIP_KERNEL_RESIDENT) {
+        if (!exact(c)) {
+            std::string why;
+            std::vector<std::vector<int>> reads;
+            if (c->nnbr != 31 || (!c->res_auto && c->n > 32 * kResMaxWaves * c->ncu))
+                rc = fail(SWE_HIP_EINVAL, "the resident kernel takes 31-point stencils and at "
+                                          "most " + std::to_string(32 * kResMaxWaves)
+                                          + " nodes per compute unit");
+            else {
+                // a caller that names the kernel keeps its node order: tiles
+                // of that order must fit the scheme, though the units are cut
+                // from an order of their own
+                std::vector<int> ts, us, ul;
+                const int tmax = (c->n + c->ncu - 1) / c->ncu;
+                if (!c->res_auto)
+                    rc = cut_tiles(c, tmax, kResMaxRows, ts, us, ul);
+                if (!rc && (int)ts.size() - 1 > c->ncu)
+                    rc = fail(SWE_HIP_EINVAL,
+                              "the resident kernel's tiles exceed one per compute unit");
+                if (!rc && !c->res_auto)
+                    rc = resident_neighbours(tile_reads(c->n, ts, us, ul), nullptr);
+                if (!rc)
+                    if (int e = units_build(c, &reads, &why))
+                        rc = fail(e, why);
+            }
+            std::vector<int> waits;
+            if (!rc)
+                rc = resident_neighbours(reads, &waits);
+            if (!rc)
+                rc = upload_waits(c, waits);
+        } else {
         // one tile of <= ceil(n / CUs) consecutive nodes per compute unit;
         // two lanes per node in FP64, one in FP32
         const int tmax = (c->n + c->ncu - 1) / c->ncu;
@@ -1018,13 +1093,18 @@ int swe_hip_create_ex(const swe_hip_static *s, const swe_hip_options *o, swe_hip
         }
         if (!rc && c->tiles.ntiles > c->ncu)
             rc = fail(SWE_HIP_EINVAL, "the resident kernel's tiles exceed one per compute unit");
+        std::vector<int> waits;
         if (!rc)
-            rc = resident_neighbours(c, ts, us, ul);
-        if (!rc) {
+            rc = resident_neighbours(tile_reads(c->n, ts, us, ul), &waits);
+        if (!rc)
+            rc = upload_waits(c, waits);
+        if (!rc)
             c->res_lds = c->tiles.umax_used * (fp32 ? (int)(sizeof(float4) + sizeof(int))
                                                     : 2 * (int)(sizeof(double2) + sizeof(int)));
+        }
+        if (!rc) {
             rc = dev_alloc(&c->bytes, &c->d_res_sync,
-                           (size_t)resident_sync_bytes(c->tiles.ntiles));
+                           (size_t)resident_sync_bytes(resident_tiles(c)));
         }
         if (!rc)
             check(hipHostMalloc((void **)&c->h_res_abort, sizeof(unsigned)), "hipHostMalloc");
@@ -1048,10 +1128,14 @@ int swe_hip_create_ex(const swe_hip_static *s, const swe_hip_options *o, swe_hip
         }
         // AUTO: a mesh whose tiles do not fit the resident scheme (too many
         // rows or neighbouring tiles, e.g. long bands of a caller's node
-        // order) or that cannot be co-resident runs the stage kernels
-        if (rc == SWE_HIP_EINVAL && c->res_auto) {
+        // order), that cannot be co-resident or whose unit records the device
+        // has no memory for runs the stage kernels
+        if ((rc == SWE_HIP_EINVAL || (rc == SWE_HIP_ENOMEM && c->units.ntiles > 0))
+            && c->res_auto) {
+            (void)hipGetLastError();
             c->res_auto = false;
             c->tiles.ntiles = 0;
+            units_free(c);
             if (fp32) {
                 c->kernel = (o->flags & SWE_HIP_EXACT) || c->n > 262144 ? SWE_HIP_KERNEL_LANE
                                                                          : SWE_HIP_KERNEL_PAIR;
@@ -1558,8 +1642,11 @@ int swe_hip_rk_steps(swe_hip_ctx *c, int nsteps)
         return fail(SWE_HIP_EINVAL, "rk_steps: bad ctx or nsteps");
     HIPCHK(hipSetDevice(c->dev));
     // a resident context chosen by AUTO replays the stage graphs for calls
-    // too short to repay a launch (same arithmetic, bitwise)
-    if (c->kernel == SWE_HIP_KERNEL_RESIDENT && (!c->res_auto || nsteps >= kResAutoMinSteps)) {
+    // too short to repay a launch (same arithmetic, bitwise); above 256 nodes
+    // per compute unit one step already does
+    if (c->kernel == SWE_HIP_KERNEL_RESIDENT
+        && (!c->res_auto || nsteps >= kResAutoMinSteps
+            || c->n > 32 * kResMaxWaves * c->ncu)) {
         std::string why;
         const long long before = c->res_stages;
         int rc = resident_steps(c, nsteps, &why);
@@ -1569,8 +1656,8 @@ int swe_hip_rk_steps(swe_hip_ctx *c, int nsteps)
             // (e.g. compute units reserved by another process): the stage
             // kernels from here on
             c->res_auto = false;
-            c->kernel = c->fp32 ? SWE_HIP_KERNEL_LANE : SWE_HIP_KERNEL_PAIR;
-            c->split32 = 1;
+            c->kernel = c->fp32 ? (c->split32 == 2 ? SWE_HIP_KERNEL_PAIR : SWE_HIP_KERNEL_LANE)
+                                : SWE_HIP_KERNEL_PAIR;
             (void)hipGetLastError();
         } else if (rc) {
             return fail(rc, why);

@@ -226,6 +226,16 @@ __device__ __forceinline__ double quad_bcast(double v)
     return __hiloint2double(hi, lo);
 }
 
+// Lane k of every aligned group of 4 lanes takes lane Pk's value.
+template <int P0, int P1, int P2, int P3>
+__device__ __forceinline__ double quad_perm(double v)
+{
+    constexpr int ctrl = P0 | P1 << 2 | P2 << 4 | P3 << 6;
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), ctrl, 0xF, 0xF, false);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), ctrl, 0xF, 0xF, false);
+    return __hiloint2double(hi, lo);
+}
+
 template <int K>
 __device__ __forceinline__ int quad_bcast_i(int v)
 {

@@ -1,0 +1,314 @@
+// Host side of the matrix-core resident kernels: the kernel order, the tiles
+// and their row lists, the launch.
+#include "units.h"
+
+#include <algorithm>
+#include <atomic>
+#include <cmath>
+#include <new>
+#include <numeric>
+#include <system_error>
+#include <thread>
+
+namespace swe {
+
+namespace {
+
+template <typename T>
+int upload(swe_hip_ctx *c, T **dst, const std::vector<T> &v, std::string *err)
+{
+    const size_t bytes = sizeof(T) * v.size();
+    if (hipMalloc((void **)dst, bytes ? bytes : 8) != hipSuccess) {
+        *err = "unit tables: hipMalloc";
+        return SWE_HIP_ENOMEM;
+    }
+    c->bytes += (long long)bytes;
+    c->units.bytes += (long long)bytes;
+    if (hipMemcpy(*dst, v.data(), bytes, hipMemcpyHostToDevice) != hipSuccess) {
+        *err = "unit tables: upload";
+        return SWE_HIP_EDEVICE;
+    }
+    return 0;
+}
+
+// Place of (node of the unit, slot) in a unit's 512 row numbers: FP64 [group of
+// 4 nodes][slot & 3][node][slot / 4], FP32 [slot / 8][node][slot & 7].
+int prec_at(bool fp32, int m, int slot)
+{
+    return fp32 ? (slot >> 3) * 128 + m * 8 + (slot & 7)
+                : (m >> 2) * 128 + ((slot & 3) * 4 + (m & 3)) * 8 + (slot >> 2);
+}
+
+// Runs the tasks on host threads of their own (in line where no thread can be
+// had); an exception in any (out of memory) is thrown again once all are done.
+template <typename F>
+void in_parallel(int tasks, F f)
+{
+    std::atomic<bool> failed{false};
+    auto guarded = [&](int k) {
+        try {
+            f(k);
+        } catch (...) {
+            failed = true;
+        }
+    };
+    std::vector<std::thread> th(tasks > 1 ? tasks - 1 : 0);
+    for (int k = 1; k < tasks; ++k) {
+        try {
+            th[k - 1] = std::thread(guarded, k);
+        } catch (const std::system_error &) {
+            guarded(k);
+        }
+    }
+    guarded(0);
+    for (std::thread &t : th)
+        if (t.joinable())
+            t.join();
+    if (failed)
+        throw std::bad_alloc();
+}
+
+// f(first, last) over [0, n) in up to 8 ranges.
+template <typename F>
+void parallel_ranges(int n, F f)
+{
+    const int nt = std::max(1, std::min({n, 8, (int)std::thread::hardware_concurrency()}));
+    in_parallel(nt, [&](int k) { f((int)((long)n * k / nt), (int)((long)n * (k + 1) / nt)); });
+}
+
+}  // namespace
+
+void units_free(swe_hip_ctx *c)
+{
+    SweUnits &u = c->units;
+    void *ptrs[] = {u.d_wrec, u.d_prec, u.d_grec, u.d_tile_start, u.d_unit_start, u.d_ustart,
+                    u.d_ulist, u.d_own_row, u.d_perm, u.d_hd};
+    for (void *p : ptrs)
+        if (p)
+            (void)hipFree(p);
+    c->bytes -= u.bytes;
+    u = SweUnits{};
+}
+
+namespace {
+
+// Reorders ids[first, last) so that consecutive chunks of `chunk` nodes are
+// compact on the sphere: recursive bisection along the longest principal
+// axis, the left part always whole chunks.  Against a Hilbert curve through
+// the nodes a tile reads fewer rows from fewer tiles (N = 40962, 161-node
+// tiles: at most 352 rows and 10 tiles against 565 and 18; N = 163842: 1006
+// and 10 against 1487 and 17).
+void bisect(const double *xyz, int n, std::vector<int> &ids, int first, int last, int chunk)
+{
+    const int count = last - first, parts = (count + chunk - 1) / chunk;
+    if (parts < 2)
+        return;
+    double mean[3] = {0.0, 0.0, 0.0}, cov[3][3] = {};
+    for (int i = first; i < last; ++i)
+        for (int d = 0; d < 3; ++d)
+            mean[d] += xyz[(size_t)d * n + ids[i]] / count;
+    for (int i = first; i < last; ++i) {
+        double r[3];
+        for (int d = 0; d < 3; ++d)
+            r[d] = xyz[(size_t)d * n + ids[i]] - mean[d];
+        for (int d = 0; d < 3; ++d)
+            for (int e = 0; e < 3; ++e)
+                cov[d][e] += r[d] * r[e];
+    }
+    double v[3] = {1.0, 0.7, 0.4};   // power iteration: the split only needs a long axis
+    for (int it = 0; it < 24; ++it) {
+        double t[3], len = 0.0;
+        for (int d = 0; d < 3; ++d) {
+            t[d] = cov[d][0] * v[0] + cov[d][1] * v[1] + cov[d][2] * v[2];
+            len += t[d] * t[d];
+        }
+        if (!(len > 0.0) || !std::isfinite(len))
+            break;
+        len = std::sqrt(len);
+        for (int d = 0; d < 3; ++d)
+            v[d] = t[d] / len;
+    }
+    std::vector<std::pair<double, int>> key(count);
+    for (int i = 0; i < count; ++i) {
+        const int id = ids[first + i];
+        const double k = xyz[id] * v[0] + xyz[(size_t)n + id] * v[1] + xyz[2 * (size_t)n + id] * v[2];
+        key[i] = {k == k ? k : 0.0, id};   // a NaN coordinate must not break the order
+    }
+    const int left = parts / 2 * chunk;
+    std::nth_element(key.begin(), key.begin() + left, key.end());
+    for (int i = 0; i < count; ++i)
+        ids[first + i] = key[i].second;
+    key = {};
+    auto half = [&](int k) {
+        bisect(xyz, n, ids, k ? first + left : first, k ? last : first + left, chunk);
+    };
+    if (count > 16384) {
+        in_parallel(2, half);
+    } else {
+        half(0);
+        half(1);
+    }
+}
+
+}  // namespace
+
+static int build(swe_hip_ctx *c, std::vector<std::vector<int>> *nbr_tiles, std::string *err)
+{
+    const int n = c->n, W = c->nnbr;
+    SweUnits &u = c->units;
+    const int tmax = std::max(16, (n + c->ncu - 1) / c->ncu);
+    const int nt = (n + tmax - 1) / tmax;
+    const std::vector<int> &nbr = c->mesh->h_nbr;
+    // kernel order: compact tiles of compact units
+    const double *xyz = c->mesh->h_xyz.data();
+    std::vector<int> perm(n), inv(n);
+    std::iota(perm.begin(), perm.end(), 0);
+    bisect(xyz, n, perm, 0, n, tmax);
+    parallel_ranges(nt, [&](int a, int b) {
+        for (int t = a; t < b; ++t)
+            bisect(xyz, n, perm, t * tmax, std::min(n, (t + 1) * tmax), 16);
+    });
+    for (int i = 0; i < n; ++i)
+        inv[perm[i]] = i;
+    std::vector<int> tstart(nt + 1), ustart(nt + 1, 0), unit_start(nt + 1, 0), own_row(nt);
+    for (int t = 0; t <= nt; ++t)
+        tstart[t] = std::min(n, t * tmax);
+    for (int t = 0; t < nt; ++t)
+        unit_start[t + 1] = unit_start[t] + (tstart[t + 1] - tstart[t] + 15) / 16;
+    const int units = unit_start[nt];
+    // distinct rows of each tile (its own nodes among them), ascending
+    std::vector<std::vector<int>> list(nt);
+    std::vector<uint4> precq((size_t)units * 64);
+    unsigned short *prec = reinterpret_cast<unsigned short *>(precq.data());
+    nbr_tiles->assign(nt, {});
+    parallel_ranges(nt, [&](int a, int b) {
+        std::vector<int> mark(n, -1), where(n);
+        for (int t = a; t < b; ++t) {
+            std::vector<int> &l = list[t];
+            for (int i = tstart[t]; i < tstart[t + 1]; ++i) {
+                mark[i] = t;
+                l.push_back(i);
+            }
+            for (int i = tstart[t]; i < tstart[t + 1]; ++i)
+                for (int s = 0; s < W; ++s) {
+                    const int q = inv[nbr[(size_t)s * n + perm[i]]];
+                    if (mark[q] != t) {
+                        mark[q] = t;
+                        l.push_back(q);
+                    }
+                }
+            std::sort(l.begin(), l.end());
+            for (int k = 0; k < (int)l.size(); ++k) {
+                where[l[k]] = k;
+                const int o = l[k] / tmax;
+                if (o != t && ((*nbr_tiles)[t].empty() || (*nbr_tiles)[t].back() != o))
+                    (*nbr_tiles)[t].push_back(o);
+            }
+            own_row[t] = where[tstart[t]];
+            for (int i = tstart[t]; i < tstart[t + 1]; ++i) {
+                const int m = i - tstart[t];
+                unsigned short *p = &prec[(size_t)(unit_start[t] + m / 16) * 512];
+                for (int slot = 0; slot < W; ++slot)
+                    p[prec_at(c->fp32, m & 15, slot)] =
+                        (unsigned short)where[inv[nbr[(size_t)slot * n + perm[i]]]];
+            }
+        }
+    });
+    int rows = 0;
+    for (int t = 0; t < nt; ++t) {
+        ustart[t + 1] = ustart[t] + (int)list[t].size();
+        rows = std::max(rows, (int)list[t].size());
+    }
+    std::vector<int> ulist;
+    ulist.reserve(ustart[nt]);
+    for (int t = 0; t < nt; ++t)
+        ulist.insert(ulist.end(), list[t].begin(), list[t].end());
+    // FP64 slots past the stencil read the zero row after the last
+    if (!c->fp32)
+        for (int k = 0; k < units; ++k)
+            for (int slot = W; slot < 32; ++slot)
+                for (int m = 0; m < 16; ++m)
+                    prec[(size_t)k * 512 + prec_at(false, m, slot)] = (unsigned short)rows;
+    u.chains = c->fp32 && c->split32 == 2 ? 2 : 1;
+    u.ntiles = nt;
+    u.units = (tmax + 15) / 16;
+    u.rows = rows;
+    u.waves = std::min(8, std::max(4, u.units));
+    if (!(c->fp32 ? units_plan32(u) : units_plan64(u)) || rows > 65534) {
+        *err = "unit kernel: a tile's rows do not fit the LDS";
+        return SWE_HIP_EINVAL;
+    }
+    std::vector<int> unit_tile(units);
+    for (int t = 0; t < nt; ++t)
+        std::fill(unit_tile.begin() + unit_start[t], unit_tile.begin() + unit_start[t + 1], t);
+    int *d_unit_tile = nullptr;
+    int rc = upload(c, &u.d_tile_start, tstart, err);
+    if (!rc) rc = upload(c, &u.d_unit_start, unit_start, err);
+    if (!rc) rc = upload(c, &u.d_ustart, ustart, err);
+    if (!rc) rc = upload(c, &u.d_ulist, ulist, err);
+    if (!rc) rc = upload(c, &u.d_own_row, own_row, err);
+    if (!rc) rc = upload(c, &u.d_perm, perm, err);
+    if (!rc) rc = upload(c, &u.d_prec, precq, err);
+    if (!rc) rc = upload(c, &d_unit_tile, unit_tile, err);
+    if (!rc) {
+        rc = c->fp32 ? units_pack32(c, units, d_unit_tile) : units_pack64(c, units, d_unit_tile);
+        if (rc)
+            *err = "unit records: allocation or pack kernel";
+    }
+    if (d_unit_tile) {
+        (void)hipFree(d_unit_tile);
+        c->bytes -= (long long)(sizeof(int) * unit_tile.size());
+        u.bytes -= (long long)(sizeof(int) * unit_tile.size());
+    }
+    return rc;
+}
+
+int units_build(swe_hip_ctx *c, std::vector<std::vector<int>> *nbr_tiles, std::string *err)
+{
+    try {
+        return build(c, nbr_tiles, err);
+    } catch (const std::bad_alloc &) {
+        *err = "unit tables: out of host memory";
+        return SWE_HIP_ENOMEM;
+    }
+}
+
+void units_tables(const swe_hip_ctx *c, int nsteps, const DevResSync &y, DevUnits *p)
+{
+    const SweUnits &u = c->units;
+    p->y = y;
+    p->tile_start = u.d_tile_start;
+    p->unit_start = u.d_unit_start;
+    p->ustart = u.d_ustart;
+    p->ulist = u.d_ulist;
+    p->own_row = u.d_own_row;
+    p->perm = u.d_perm;
+    p->prec = u.d_prec;
+    p->nsteps = nsteps;
+    p->bytes = (int)(state_count(c) * (long)(c->fp32 ? sizeof(float) : sizeof(double)));
+    p->lds_rows = u.rows;
+    p->lds_pos = u.pos;
+    p->lds_geo = u.geo;
+}
+
+int units_prepare(swe_hip_ctx *c, std::string *err)
+{
+    void *fn = c->fp32 ? units_kernel32(c->units) : units_kernel64(c->units);
+    int per_cu = 0;
+    if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, kUnitsMaxLds)
+            != hipSuccess
+        || hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, 64 * c->units.waves,
+                                                        c->units.lds) != hipSuccess
+        || (long)per_cu * c->ncu < c->units.ntiles) {
+        *err = "unit kernel: the launch cannot be co-resident on this device";
+        return SWE_HIP_EDEVICE;
+    }
+    return 0;
+}
+
+hipError_t units_launch(swe_hip_ctx *c, int nsteps, const DevResSync &y)
+{
+    return c->fp32 ? units_launch32(c, nsteps, y) : units_launch64(c, nsteps, y);
+}
+
+}  // namespace swe
