@@ -259,9 +259,11 @@ int swe_hip_set_state(swe_hip_ctx *ctx, int member, const double *H);
 /* Read-back (main.c:379-380): member slot -> host state layout. */
 int swe_hip_get_state(swe_hip_ctx *ctx, int member, double *H);
 
-/* Exactly RK_substep / RK_substep_ocl for every member: eval_RHS into F,
- * then copy/update_D and eval_K/update_H as separate kernels with the
- * reference's constants (dt/2.0, 2.0, 1.0, dt/6.0).  substep_id 0..3. */
+/* Exactly RK_substep / RK_substep_ocl for every member, with the reference's
+ * constants (dt/2.0, 2.0, 1.0, dt/6.0).  substep_id 0..3.  With timing on
+ * (swe_hip_set_timing), eval_RHS into F, then copy/update_D and
+ * eval_K/update_H as separate kernels; otherwise one fused kernel with the
+ * same arithmetic, bitwise. */
 int swe_hip_rk_substep(swe_hip_ctx *ctx, int substep_id);
 
 /* Fast path: nsteps full RK4 steps (4 fused stage kernels per step, the RHS

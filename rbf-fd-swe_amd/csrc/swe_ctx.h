@@ -127,6 +127,7 @@ struct swe_hip_ctx {
     // FP32 contexts (SWE_HIP_FP32): the same buffers in float, d_* unused
     bool fp32 = false;
     float *f_H = nullptr, *f_Ka = nullptr, *f_Kb = nullptr, *f_D = nullptr, *f_F = nullptr;
+    bool k_in_b = false;         // drop-in substeps: K is in Kb, not Ka
     double *d_stage = nullptr;   // [n*4] staging for member upload/read-back
     int *d_active = nullptr;     // member slots advanced by the ensemble kernel
     SweTiles tiles;              // LDS-staged ensemble kernel (ntiles == 0: unused)

@@ -170,63 +170,49 @@ constexpr int kGraphSteps[kGraphCount] = {64, 16, 4, 1};
 
 namespace {
 
-// Fused stage s of one RK step: gathers from H (s=0), Ka (s=1), Kb (s=2),
-// Ka (s=3); writes Ka, Kb, Ka, H.
-// FP32 stage s of one RK step: the same buffers and constants in float;
-// stage 3 keeps dt/6.0 in double (update_H, rk4_rbffd_swe.c:86-121).
-void launch_fused32(const swe_hip_ctx *c, int s)
+// Fused stage s of one RK step on caller-given K buffers: gathers from H
+// (s = 0) or kin, writes kout, in stage 3 H.  FP32: the same in float; stage 3
+// keeps dt/6.0 in double (update_H, rk4_rbffd_swe.c:86-121).
+template <typename T>
+void launch_fused_k(const swe_hip_ctx *c, int s, const T *kin, T *kout, bool keep_d)
 {
-    DevStage32 st{};
-    st.h = c->f_H;
-    st.d = c->f_D;
-    const float dt = (float)c->dt;
-    switch (s) {
-    case 0:
-        st.src = c->f_H; st.out = c->f_Ka; st.c = (float)(dt / 2.0); st.dcoef = 0.0f;
-        break;
-    case 1:
-        st.src = c->f_Ka; st.out = c->f_Kb; st.c = (float)(dt / 2.0); st.dcoef = 2.0f;
-        break;
-    case 2:
-        st.src = c->f_Kb; st.out = c->f_Ka; st.c = dt; st.dcoef = 2.0f;
-        break;
-    default:
-        st.src = c->f_Ka; st.out = c->f_H; st.c6 = dt / 6.0; st.dcoef = 1.0f;
-        break;
+    if constexpr (sizeof(T) == sizeof(float)) {
+        const float dt = (float)c->dt;
+        DevStage32 st{};
+        st.h = c->f_H;
+        st.d = c->f_D;
+        st.keep_d = keep_d;
+        st.src = s == 0 ? c->f_H : kin;
+        st.out = s == 3 ? c->f_H : kout;
+        st.c = s == 2 ? dt : (float)(dt / 2.0);
+        st.c6 = dt / 6.0;
+        st.dcoef = s == 0 ? 0.0f : (s == 3 ? 1.0f : 2.0f);
+        launch_fp32_stage(c, s, st);
+    } else {
+        const double dt = c->dt;
+        DevStage st{};
+        st.members = c->B;
+        st.active = c->d_active;
+        st.h = c->d_H;
+        st.d = c->d_D;
+        st.keep_d = keep_d;
+        st.src = s == 0 ? c->d_H : kin;
+        st.out = s == 3 ? c->d_H : kout;
+        st.c = s == 3 ? dt / 6.0 : (s == 2 ? dt : dt / 2.0);
+        st.dcoef = s == 0 ? 0.0 : (s == 3 ? 1.0 : 2.0);
+        launch_stage(c, s, st);
     }
-    launch_fp32_stage(c, s, st);
 }
 
+// Fused stage s of a whole step: gathers from H (s=0), Ka (s=1), Kb (s=2),
+// Ka (s=3); writes Ka, Kb, Ka, H.
 void launch_fused(const swe_hip_ctx *c, int s)
 {
-    if (c->fp32) {
-        launch_fused32(c, s);
-        return;
-    }
-    DevStage st{};
-    st.members = c->B;
-    st.active = c->d_active;
-    st.h = c->d_H;
-    st.d = c->d_D;
-    const double dt = c->dt;
-    switch (s) {
-    case 0:
-        st.src = c->d_H; st.out = c->d_Ka; st.c = dt / 2.0; st.dcoef = 0.0;
-        launch_stage(c, ST_0, st);
-        break;
-    case 1:
-        st.src = c->d_Ka; st.out = c->d_Kb; st.c = dt / 2.0; st.dcoef = 2.0;
-        launch_stage(c, ST_1, st);
-        break;
-    case 2:
-        st.src = c->d_Kb; st.out = c->d_Ka; st.c = dt; st.dcoef = 2.0;
-        launch_stage(c, ST_2, st);
-        break;
-    default:
-        st.src = c->d_Ka; st.out = c->d_H; st.c = dt / 6.0; st.dcoef = 1.0;
-        launch_stage(c, ST_3, st);
-        break;
-    }
+    if (c->fp32)
+        launch_fused_k<float>(c, s, s == 2 ? c->f_Kb : c->f_Ka, s == 1 ? c->f_Kb : c->f_Ka, false);
+    else
+        launch_fused_k<double>(c, s, s == 2 ? c->d_Kb : c->d_Ka, s == 1 ? c->d_Kb : c->d_Ka,
+                               false);
 }
 
 void launch_rhs(const swe_hip_ctx *c, const double *src, double *F)
@@ -1519,10 +1505,10 @@ int swe_hip_eval_rhs32(swe_hip_ctx *c, int member, const float *K, float *F)
                                     "only, member 0)");
     int rc = ensure_F(c);
     if (!rc)
-        rc = to_device32(c, K, c->f_Kb);
+        rc = to_device32(c, K, c->k_in_b ? c->f_Ka : c->f_Kb);   // not the substeps' K
     if (rc)
         return rc;
-    launch_rhs32(c, c->f_Kb, c->f_F);
+    launch_rhs32(c, c->k_in_b ? c->f_Ka : c->f_Kb, c->f_F);
     rc = check_launch("eval_RHS kernel (FP32)");
     if (rc)
         return rc;
@@ -1538,7 +1524,7 @@ static int rk_substep32(swe_hip_ctx *c, int s)
     const int eb = elementwise_blocks(cnt);
     const float dt = (float)c->dt;
     const bool ex = exact(c);
-    float *H = c->f_H, *K = c->f_Ka, *F = c->f_F, *D = c->f_D;
+    float *H = c->f_H, *K = c->k_in_b ? c->f_Kb : c->f_Ka, *F = c->f_F, *D = c->f_D;
     hipStream_t q = c->stream;
     int rc = timed(c, &c->acc.t_eval_rhs, "eval_RHS kernel (FP32)",
                    [&] { launch_rhs32(c, s == 0 ? H : K, F); });
@@ -1580,10 +1566,11 @@ int swe_hip_eval_rhs(swe_hip_ctx *c, int member, const double *K, double *F)
     int rc = ensure_F(c);
     if (rc)
         return rc;
-    rc = to_device_member(c, member, K, c->d_Kb);
+    double *in = c->k_in_b ? c->d_Ka : c->d_Kb;   // not the substeps' K
+    rc = to_device_member(c, member, K, in);
     if (rc)
         return rc;
-    launch_rhs(c, c->d_Kb, c->d_F);
+    launch_rhs(c, in, c->d_F);
     rc = check_launch("eval_RHS kernel");
     if (rc)
         return rc;
@@ -1595,6 +1582,22 @@ int swe_hip_rk_substep(swe_hip_ctx *c, int s)
     if (!c || s < 0 || s > 3)
         return fail(SWE_HIP_EINVAL, "rk_substep: bad ctx or substep_id");
     HIPCHK(hipSetDevice(c->dev));
+    // Without timers one fused launch replaces the three: F stays in
+    // registers, K goes to the other K buffer (a stage never writes the array
+    // it gathers from), D is kept after stage 3 as the reference keeps it.
+    // Same arithmetic, bitwise.  N = 2562: 5.0 + 2.0 + 2.0 us of kernels and
+    // two launch gaps against 4.6 us.
+    if (!c->timing) {
+        if (c->fp32)
+            launch_fused_k<float>(c, s, c->k_in_b ? c->f_Kb : c->f_Ka,
+                                  c->k_in_b ? c->f_Ka : c->f_Kb, true);
+        else
+            launch_fused_k<double>(c, s, c->k_in_b ? c->d_Kb : c->d_Ka,
+                                   c->k_in_b ? c->d_Ka : c->d_Kb, true);
+        if (s < 3)
+            c->k_in_b = !c->k_in_b;
+        return check_launch("substep kernel");
+    }
     if (int rc0 = ensure_F(c))
         return rc0;
     if (c->fp32)
@@ -1603,7 +1606,7 @@ int swe_hip_rk_substep(swe_hip_ctx *c, int s)
     const int eb = elementwise_blocks(cnt);
     const double dt = c->dt;
     const bool ex = exact(c);
-    double *H = c->d_H, *K = c->d_Ka, *F = c->d_F, *D = c->d_D;
+    double *H = c->d_H, *K = c->k_in_b ? c->d_Kb : c->d_Ka, *F = c->d_F, *D = c->d_D;
     hipStream_t q = c->stream;
     int rc = timed(c, &c->acc.t_eval_rhs, "eval_RHS kernel",
                    [&] { launch_rhs(c, s == 0 ? H : K, F); });
@@ -1662,8 +1665,21 @@ int swe_hip_rk_steps(swe_hip_ctx *c, int nsteps)
         } else if (rc) {
             return fail(rc, why);
         } else {
+            if (nsteps > 0)
+                c->k_in_b = false;
             return 0;
         }
+    }
+    if (nsteps > 0)
+        c->k_in_b = false;   // stage 2 leaves K in Ka
+    // an AUTO context comes here for at most kResAutoMinSteps - 1 steps: plain
+    // launches, without the captures (N = 642, one step with its state in and
+    // out: 52 us against 61 by graph, 77 against 518 on the first call)
+    if (c->res_auto) {
+        for (int i = 0; i < nsteps; ++i)
+            for (int s = 0; s < 4; ++s)
+                launch_fused(c, s);
+        return check_launch("stage kernels");
     }
     // every graph is captured on the first call, so no later (timed) call
     // pays for a capture

@@ -70,6 +70,7 @@ struct DevStage {
     double *out;        // next K, H (stage 3) or F (ST_RHS)
     double c;           // K = H + c*F (dt/2, dt/2, dt); stage 3: H += c*D (dt/6)
     double dcoef;       // D += dcoef*F (2, 2, 1)
+    int keep_d;         // stage 3 stores D too (drop-in substeps)
     const int *active;  // ensemble: member slots [0, *active) are advanced
     int members;        // B: state stride of a (node, var) row
     int nblk;           // grid.x, a multiple of 8
@@ -166,7 +167,8 @@ __device__ __forceinline__ void rhs_point(const Sums &S, double u, double v, dou
 //   stage 0: D = F;             K = H + (dt/2)*F
 //   stage 1: D = D + 2*F;       K = H + (dt/2)*F
 //   stage 2: D = D + 2*F;       K = H + dt*F
-//   stage 3: D = D + 1*F;       H = H + (dt/6)*D   (D is dead afterwards)
+//   stage 3: D = D + 1*F;       H = H + (dt/6)*D   (D is dead afterwards
+//            within whole steps; the drop-in substeps keep it)
 template <int STAGE, bool EXACT>
 __device__ __forceinline__ void stage_update(const DevStage &st, long e, double Fv)
 {
@@ -184,6 +186,8 @@ __device__ __forceinline__ void stage_update(const DevStage &st, long e, double 
     } else {
         const double hv = st.h[e];
         const double dv = axpy<EXACT>(st.d[e], st.dcoef, Fv);
+        if (st.keep_d)
+            st.d[e] = dv;
         st.out[e] = axpy<EXACT>(hv, st.c, dv);
     }
 }
@@ -212,6 +216,8 @@ __device__ __forceinline__ void stage_update_pair(const DevStage &st, long e, do
         const double2 d0 = *reinterpret_cast<const double2 *>(st.d + e);
         const double dv0 = axpy<EXACT>(d0.x, st.dcoef, F0);
         const double dv1 = axpy<EXACT>(d0.y, st.dcoef, F1);
+        if (st.keep_d)
+            *reinterpret_cast<double2 *>(st.d + e) = make_double2(dv0, dv1);
         *out = make_double2(axpy<EXACT>(hv.x, st.c, dv0), axpy<EXACT>(hv.y, st.c, dv1));
     }
 }
@@ -1109,6 +1115,8 @@ __device__ __forceinline__ void stage_update_pre_pair(const DevStage &st, long e
     } else {
         const double d0 = axpy<EXACT>(dv.x, st.dcoef, F.x);
         const double d1 = axpy<EXACT>(dv.y, st.dcoef, F.y);
+        if (st.keep_d)
+            *reinterpret_cast<double2 *>(st.d + e) = make_double2(d0, d1);
         *out = make_double2(axpy<EXACT>(hv.x, st.c, d0), axpy<EXACT>(hv.y, st.c, d1));
     }
 }
