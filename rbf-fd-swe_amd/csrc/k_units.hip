@@ -386,7 +386,7 @@ void *units_kernel64(const SweUnits &u)
     }
 }
 
-int units_pack64(swe_hip_ctx *c, int units, const int *unit_tile)
+int units_pack64(swe_hip_ctx *c, int units)
 {
     SweUnits &u = c->units;
     const size_t wb = sizeof(double2) * 1024 * (size_t)units;
@@ -398,7 +398,7 @@ int units_pack64(swe_hip_ctx *c, int units, const int *unit_tile)
     c->bytes += (long long)(wb + gb + hb);
     u.bytes += (long long)(wb + gb + hb);
     k_pack_units<<<units, 1024, 0, c->stream>>>(mesh_of(c), u.d_tile_start, u.d_unit_start,
-                                                unit_tile, u.d_perm,
+                                                u.d_unit_tile, u.d_perm,
                                                 static_cast<double2 *>(u.d_wrec),
                                                 static_cast<double2 *>(u.d_grec));
     return hipGetLastError() == hipSuccess && hipStreamSynchronize(c->stream) == hipSuccess

@@ -367,7 +367,7 @@ void *units_kernel32(const SweUnits &u)
                              : reinterpret_cast<void *>(&k_steps_units32<1, UM_RESIDENT, 1>);
 }
 
-int units_pack32(swe_hip_ctx *c, int units, const int *unit_tile)
+int units_pack32(swe_hip_ctx *c, int units)
 {
     SweUnits &u = c->units;
     const size_t rb = sizeof(float4) * 64 * kRec32 * (size_t)units;
@@ -377,7 +377,7 @@ int units_pack32(swe_hip_ctx *c, int units, const int *unit_tile)
     c->bytes += (long long)(rb + hb);
     u.bytes += (long long)(rb + hb);
     k_pack_units32<<<units, 64 * kRec32, 0, c->stream>>>(mesh32_of(c), u.d_tile_start,
-                                                         u.d_unit_start, unit_tile, u.d_perm,
+                                                         u.d_unit_start, u.d_unit_tile, u.d_perm,
                                                          static_cast<float4 *>(u.d_wrec));
     return hipGetLastError() == hipSuccess && hipStreamSynchronize(c->stream) == hipSuccess
                ? 0 : SWE_HIP_EDEVICE;

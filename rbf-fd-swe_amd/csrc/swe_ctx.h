@@ -19,6 +19,8 @@ constexpr int kBlock = 256;            // threads per workgroup, stage kernels
 // (at N = 40962 the pair kernel has 1281 waves: 256-thread workgroups put
 // two on 65 CUs and one on the rest).
 constexpr int kSingleBlock = 64;
+constexpr int kRingSlots = 4;          // pinned staging ring of a context
+constexpr size_t kRingBytes = 512 << 10;
 constexpr int kGraphCount = 4;         // captured step graphs per context
 // Resident whole-step kernel (k_resident.hip): one tile of <= 32 x
 // kResMaxWaves nodes per compute unit, whose stencils touch <= kResMaxRows
@@ -72,6 +74,7 @@ struct SweMesh {
     int order = SWE_HIP_ORDER_HOST;
     int sblk = 0;                 // stencil layout: 0 slot-major, 16 node blocks
     std::vector<int> perm;        // device node -> host node (empty: identity)
+    int *d_inv = nullptr;         // host node -> device node, on the device
     std::vector<double> h_xyz;    // node coordinates, device order, [3][n]
     std::vector<int> h_nbr;       // host copy of nbr, device order, [nnbr][n]
 };
@@ -100,9 +103,11 @@ struct SweUnits {
     int pos = 0, geo = 0;         // units whose positions, geometry the LDS holds
     long long bytes = 0;          // counted in the context's bytes too
     void *d_wrec = nullptr, *d_grec = nullptr, *d_hd = nullptr;
-    uint4 *d_prec = nullptr;
-    int *d_tile_start = nullptr, *d_unit_start = nullptr, *d_ustart = nullptr;
-    int *d_ulist = nullptr, *d_own_row = nullptr, *d_perm = nullptr;
+    char *d_tables = nullptr;     // one allocation, the tables below in it
+    const uint4 *d_prec = nullptr;
+    const int *d_tile_start = nullptr, *d_unit_start = nullptr, *d_ustart = nullptr;
+    const int *d_ulist = nullptr, *d_own_row = nullptr, *d_perm = nullptr;
+    const int *d_unit_tile = nullptr;
 };
 
 struct swe_hip_ctx {
@@ -128,7 +133,10 @@ struct swe_hip_ctx {
     bool fp32 = false;
     float *f_H = nullptr, *f_Ka = nullptr, *f_Kb = nullptr, *f_D = nullptr, *f_F = nullptr;
     bool k_in_b = false;         // drop-in substeps: K is in Kb, not Ka
-    double *d_stage = nullptr;   // [n*4] staging for member upload/read-back
+    void *d_stage = nullptr;     // [n*4] one member in the host layout
+    char *ring = nullptr, *d_ring = nullptr;   // pinned staging of host copies, its device address
+    int ring_slots = 0;
+    hipEvent_t ring_ev[swe::kRingSlots] = {};
     int *d_active = nullptr;     // member slots advanced by the ensemble kernel
     SweTiles tiles;              // LDS-staged ensemble kernel (ntiles == 0: unused)
     hipGraphExec_t graphs[swe::kGraphCount] = {};   // 64, 16, 4 and 1 RK steps
@@ -146,7 +154,6 @@ struct swe_hip_ctx {
     bool timing = false;
     swe_hip_timers acc{};
     long long bytes = 0;         // state buffers
-    std::vector<double> host_tmp;
 };
 
 namespace swe {

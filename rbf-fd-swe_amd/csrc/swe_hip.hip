@@ -3,6 +3,7 @@
 // driver (RK_substep semantics, swe_code/main/rk4_rbffd_swe.c:30-186), the
 // fused and graph-captured fast path, state upload/read-back in the
 // reference's host layouts (swe_code/main/include/swe_config.h:21-54).
+#include "host_par.h"
 #include "swe_ctx.h"
 
 #include <hip/hip_runtime.h>
@@ -51,14 +52,44 @@ __global__ __launch_bounds__(256) void k_axpy_to(double *__restrict__ out,
         out[i] = axpy<EXACT>(y[i], a, x[i]);
 }
 
-// Member slot <-> node-major [node][var] staging copy.
-__global__ __launch_bounds__(256) void k_put_member(double *__restrict__ state,
-                                                    const double *__restrict__ flat,
-                                                    int member, int B, long count)
+// Host-layout state (SVM_LIN_ID) of one member in `stage` -> its slot of the
+// device state, or back; thread = host element, so that a stage in host
+// memory is read and written in order.
+struct HostOrder {
+    const int *inv;     // host node -> device node (NULL: the same)
+    int cfdl, S;        // layout
+    int member, B;
+};
+
+__device__ __forceinline__ long device_elem(const HostOrder &h, long e)
+{
+    long pid = e >> 2, v = e & 3;
+    if (!h.cfdl) {
+        const long block = e / (4L * h.S), r = e - block * 4L * h.S;
+        v = r / h.S;
+        pid = block * h.S + (r - v * h.S);
+    }
+    return (4L * (h.inv ? h.inv[pid] : pid) + v) * h.B + h.member;
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void k_put_state(T *__restrict__ state,
+                                                   const T *__restrict__ stage, HostOrder h,
+                                                   long count)
 {
     const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < count)
-        state[i * B + member] = flat[i];
+        state[device_elem(h, i)] = stage[i];
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void k_get_state(T *__restrict__ stage,
+                                                   const T *__restrict__ state, HostOrder h,
+                                                   long count)
+{
+    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < count)
+        stage[i] = state[device_elem(h, i)];
 }
 
 __global__ void k_set_int(int *dst, int value)
@@ -74,15 +105,6 @@ __global__ __launch_bounds__(256) void k_move_member(double *__restrict__ state,
     const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < rows)
         state[i * B + to] = state[i * B + from];
-}
-
-__global__ __launch_bounds__(256) void k_get_member(double *__restrict__ flat,
-                                                    const double *__restrict__ state,
-                                                    int member, int B, long count)
-{
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < count)
-        flat[i] = state[i * B + member];
 }
 
 // Element-wise kernels of the FP32 drop-in stage driver over `count` values.
@@ -283,6 +305,7 @@ void release_mesh(SweMesh *m)
     if (m->d_nbr) (void)hipFree(m->d_nbr);
     if (m->d_wts) (void)hipFree(m->d_wts);
     if (m->d_geo) (void)hipFree(m->d_geo);
+    if (m->d_inv) (void)hipFree(m->d_inv);
     if (m->d_wts32) (void)hipFree(m->d_wts32);
     if (m->d_geo32) (void)hipFree(m->d_geo32);
     delete m;
@@ -304,6 +327,9 @@ void free_ctx(swe_hip_ctx *c)
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     units_free(c);
+    for (hipEvent_t e : c->ring_ev)
+        if (e) (void)hipEventDestroy(e);
+    if (c->ring) (void)hipHostFree(c->ring);
     if (c->h_res_abort) (void)hipHostFree(c->h_res_abort);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     release_mesh(c->mesh);
@@ -452,35 +478,47 @@ int build_mesh(const swe_hip_static *s, int device, int order, int sblk, bool fp
     std::vector<int> dnbr(sblk ? (size_t)W * nround : 0);
     std::vector<double> wts((size_t)W * nround * 4);
     std::vector<double> geo((size_t)GEO_N * n);
-    for (int dnode = 0; dnode < n; ++dnode) {
-        const int i = host_of(dnode);
-        for (int j = 0; j < W; ++j) {
-            const long d = lay.dm(i, j, pW);
-            const int q = s->idx[d];
-            if (q < 0 || q >= n)
-                return fail(SWE_HIP_ERANGE, "idx[" + std::to_string(d) + "] = " + std::to_string(q)
-                                                + " outside [0, " + std::to_string(n) + ")");
-            nbr[(size_t)j * n + dnode] = dev_of(q);
-            if (sblk)
-                dnbr[pos(j, dnode)] = dev_of(q);
-            double *w = &wts[pos(j, dnode) * 4];
-            w[0] = s->Dx[d];
-            w[1] = s->Dy[d];
-            w[2] = s->Dz[d];
-            w[3] = s->L[d];
+    // the first id out of range, as (device node) W + slot
+    std::atomic<long> bad{(long)n * W};
+    parallel_ranges(n, 4096, [&](int first, int last) {
+        for (int dnode = first; dnode < last; ++dnode) {
+            const int i = host_of(dnode);
+            for (int j = 0; j < W; ++j) {
+                const long d = lay.dm(i, j, pW);
+                const int q = s->idx[d];
+                if (q < 0 || q >= n) {
+                    const long at = (long)dnode * W + j;
+                    for (long b = bad; at < b && !bad.compare_exchange_weak(b, at);) {
+                    }
+                    return;
+                }
+                nbr[(size_t)j * n + dnode] = dev_of(q);
+                if (sblk)
+                    dnbr[pos(j, dnode)] = dev_of(q);
+                double *w = &wts[pos(j, dnode) * 4];
+                w[0] = s->Dx[d];
+                w[1] = s->Dy[d];
+                w[2] = s->Dz[d];
+                w[3] = s->L[d];
+            }
+            geo[(size_t)G_X * n + dnode] = s->x[i];
+            geo[(size_t)G_Y * n + dnode] = s->y[i];
+            geo[(size_t)G_Z * n + dnode] = s->z[i];
+            geo[(size_t)G_F * n + dnode] = s->f[i];
+            geo[(size_t)G_GHM * n + dnode] = s->ghm[i];
+            for (int c3 = 0; c3 < 3; ++c3) {
+                const long v = lay.vect(i, c3);
+                geo[(size_t)(G_PU + c3) * n + dnode] = s->p_u[v];
+                geo[(size_t)(G_PV + c3) * n + dnode] = s->p_v[v];
+                geo[(size_t)(G_PW + c3) * n + dnode] = s->p_w[v];
+                geo[(size_t)(G_GG + c3) * n + dnode] = s->gradghm[v];
+            }
         }
-        geo[(size_t)G_X * n + dnode] = s->x[i];
-        geo[(size_t)G_Y * n + dnode] = s->y[i];
-        geo[(size_t)G_Z * n + dnode] = s->z[i];
-        geo[(size_t)G_F * n + dnode] = s->f[i];
-        geo[(size_t)G_GHM * n + dnode] = s->ghm[i];
-        for (int c3 = 0; c3 < 3; ++c3) {
-            const long v = lay.vect(i, c3);
-            geo[(size_t)(G_PU + c3) * n + dnode] = s->p_u[v];
-            geo[(size_t)(G_PV + c3) * n + dnode] = s->p_v[v];
-            geo[(size_t)(G_PW + c3) * n + dnode] = s->p_w[v];
-            geo[(size_t)(G_GG + c3) * n + dnode] = s->gradghm[v];
-        }
+    });
+    if (bad < (long)n * W) {
+        const long d = lay.dm(host_of((int)(bad / W)), (int)(bad % W), pW);
+        return fail(SWE_HIP_ERANGE, "idx[" + std::to_string(d) + "] = " + std::to_string(s->idx[d])
+                                        + " outside [0, " + std::to_string(n) + ")");
     }
     if (sblk) {   // rows of the last block beyond n repeat the last node
         for (int dnode = n; dnode < (int)nround; ++dnode)
@@ -504,8 +542,13 @@ int build_mesh(const swe_hip_static *s, int device, int order, int sblk, bool fp
     m->fp32 = fp32;
     int rc = 0;
     hipError_t e = hipSuccess;
+    if (!rc && !perm.empty()) {
+        rc = dev_alloc(&m->bytes, (void **)&m->d_inv, sizeof(int) * (size_t)n);
+        if (!rc)
+            e = hipMemcpy(m->d_inv, inv.data(), sizeof(int) * (size_t)n, hipMemcpyHostToDevice);
+    }
     if (!rc) rc = dev_alloc(&m->bytes, (void **)&m->d_nbr, sizeof(int) * upload_nbr.size());
-    if (!rc)
+    if (!rc && e == hipSuccess)
         e = hipMemcpy(m->d_nbr, upload_nbr.data(), sizeof(int) * upload_nbr.size(),
                       hipMemcpyHostToDevice);
     if (fp32) {   // values rounded to float (exact for data read as FP32)
@@ -931,7 +974,12 @@ int swe_hip_create_ex(const swe_hip_static *s, const swe_hip_options *o, swe_hip
                    == hipSuccess
             && s->compute_size <= 32 * kResMaxWaves * ncu)
             order = SWE_HIP_ORDER_HILBERT;
-        int rc = build_mesh(s, device, order, o->slot_block, (o->flags & SWE_HIP_FP32) != 0, &m);
+        int rc = 0;
+        try {
+            rc = build_mesh(s, device, order, o->slot_block, (o->flags & SWE_HIP_FP32) != 0, &m);
+        } catch (const std::bad_alloc &) {
+            rc = fail(SWE_HIP_ENOMEM, "static data: out of host memory");
+        }
         if (rc)
             return rc;
     }
@@ -1017,8 +1065,8 @@ int swe_hip_create_ex(const swe_hip_static *s, const swe_hip_options *o, swe_hip
     void **bufs32[] = {(void **)&c->f_H, (void **)&c->f_Ka, (void **)&c->f_Kb, (void **)&c->f_D};
     for (int k = 0; k < 4; ++k)
         if (!rc) rc = dev_alloc(&c->bytes, fp32 ? bufs32[k] : bufs[k], sbytes);
-    if (!rc && !fp32)
-        rc = dev_alloc(&c->bytes, (void **)&c->d_stage, sizeof(double) * 4 * (size_t)c->n);
+    if (!rc)
+        rc = dev_alloc(&c->bytes, &c->d_stage, sbytes / (size_t)c->B);
     if (!rc) rc = dev_alloc(&c->bytes, (void **)&c->d_active, sizeof(int));
     for (int k = 0; k < 4; ++k)
         if (!rc)
@@ -1348,96 +1396,154 @@ int swe_hip_move_member(swe_hip_ctx *c, int from, int to)
     return check_launch("k_move_member");
 }
 
-static int to_device_member(swe_hip_ctx *c, int member, const double *Hhost, double *dst)
+}  // extern "C"
+
+// Host <-> device copies through a pinned ring of the context, 1 MB a slot:
+// the host copy of one slot runs beside the DMA of the others.  A pageable
+// copy of 64 KB to 1 MB costs the runtime 40 to 137 us, memcpy and DMA 8 to 21
+// (1.3 MB: 53 and 61 us in, 79 and 71 out; 5.2 MB: 159 and 183, 312 and 275).
+static int stage_ring(swe_hip_ctx *c, size_t bytes)
 {
-    const int n = c->n;
-    c->host_tmp.resize(4 * (size_t)n);
-    double *t = c->host_tmp.data();
-    const std::vector<int> &perm = c->mesh->perm;
-    for (int d = 0; d < n; ++d) {
-        const int i = perm.empty() ? d : perm[d];
-        for (int v = 0; v < 4; ++v)
-            t[4 * (size_t)d + v] = Hhost[c->lay.svm(i, v)];
+    if (c->ring_slots)
+        return 0;
+    const int slots = (int)std::min<size_t>(kRingSlots, (bytes + kRingBytes - 1) / kRingBytes);
+    for (int k = 0; k < slots; ++k)
+        if (!c->ring_ev[k])
+            HIPCHK(hipEventCreateWithFlags(&c->ring_ev[k], hipEventDisableTiming));
+    if (hipHostMalloc((void **)&c->ring, std::min(bytes, slots * kRingBytes)) != hipSuccess) {
+        c->ring = nullptr;
+        return fail(SWE_HIP_ENOMEM, "hipHostMalloc of the staging ring");
     }
-    HIPCHK(hipSetDevice(c->dev));
-    if (c->B == 1) {
-        HIPCHK(hipMemcpyAsync(dst, t, sizeof(double) * 4 * n, hipMemcpyHostToDevice, c->stream));
-    } else {
-        HIPCHK(hipMemcpyAsync(c->d_stage, t, sizeof(double) * 4 * n, hipMemcpyHostToDevice,
+    HIPCHK(hipHostGetDevicePointer((void **)&c->d_ring, c->ring, 0));
+    c->ring_slots = slots;
+    return 0;
+}
+
+static int ring_upload(swe_hip_ctx *c, void *dst, const void *host, size_t bytes)
+{
+    if (int rc = stage_ring(c, bytes))
+        return rc;
+    for (size_t off = 0, k = 0; off < bytes; off += kRingBytes, ++k) {
+        const int slot = (int)(k % c->ring_slots);
+        const size_t len = std::min(kRingBytes, bytes - off);
+        if ((int)k >= c->ring_slots)
+            HIPCHK(hipEventSynchronize(c->ring_ev[slot]));
+        std::memcpy(c->ring + slot * kRingBytes, (const char *)host + off, len);
+        HIPCHK(hipMemcpyAsync((char *)dst + off, c->ring + slot * kRingBytes, len,
+                              hipMemcpyHostToDevice, c->stream));
+        if (off + c->ring_slots * kRingBytes < bytes)
+            HIPCHK(hipEventRecord(c->ring_ev[slot], c->stream));
+    }
+    return 0;
+}
+
+static int ring_download(swe_hip_ctx *c, void *host, const void *src, size_t bytes)
+{
+    if (int rc = stage_ring(c, bytes))
+        return rc;
+    const size_t chunks = (bytes + kRingBytes - 1) / kRingBytes;
+    auto issue = [&](size_t k) -> int {
+        const size_t off = k * kRingBytes;
+        const int slot = (int)(k % c->ring_slots);
+        HIPCHK(hipMemcpyAsync(c->ring + slot * kRingBytes, (const char *)src + off,
+                              std::min(kRingBytes, bytes - off), hipMemcpyDeviceToHost,
                               c->stream));
-        k_put_member<<<elementwise_blocks(4L * n), kBlock, 0, c->stream>>>(dst, c->d_stage, member,
-                                                                         c->B, 4L * n);
-        int rc = check_launch("k_put_member");
-        if (rc)
+        if (chunks > 1)
+            HIPCHK(hipEventRecord(c->ring_ev[slot], c->stream));
+        return 0;
+    };
+    for (size_t k = 0; k < chunks && k < (size_t)c->ring_slots; ++k)
+        if (int rc = issue(k))
+            return rc;
+    for (size_t k = 0; k < chunks; ++k) {
+        const int slot = (int)(k % c->ring_slots);
+        const size_t off = k * kRingBytes;
+        if (chunks > 1)
+            HIPCHK(hipEventSynchronize(c->ring_ev[slot]));
+        else
+            HIPCHK(hipStreamSynchronize(c->stream));
+        std::memcpy((char *)host + off, c->ring + slot * kRingBytes,
+                    std::min(kRingBytes, bytes - off));
+        if (k + c->ring_slots < chunks)
+            if (int rc = issue(k + c->ring_slots))
+                return rc;
+    }
+    return 0;
+}
+
+// True when a member's device state is its host-layout state byte for byte.
+static bool same_order(const swe_hip_ctx *c)
+{
+    return c->B == 1 && c->lay.cfdl && !c->mesh->d_inv;
+}
+
+static HostOrder host_order(const swe_hip_ctx *c, int member)
+{
+    return HostOrder{c->mesh->d_inv, c->lay.cfdl, c->lay.S, member, c->B};
+}
+
+// A state that needs reordering and fits the ring is reordered by a kernel
+// that reads or writes the pinned ring itself: 13 us for 20 KB, 19 for 328 KB,
+// 42 for 1.3 MB, where a DMA takes 8, 13 and 47 and the kernel that has to
+// wait for it (or that it waits for) about 8 more.
+template <typename T>
+static int to_device(swe_hip_ctx *c, int member, const T *host, T *dst)
+{
+    const long cnt = 4L * c->n;
+    const size_t bytes = sizeof(T) * cnt;
+    HIPCHK(hipSetDevice(c->dev));
+    if (same_order(c)) {
+        if (int rc = ring_upload(c, dst, host, bytes))
+            return rc;
+    } else {
+        const T *from = static_cast<const T *>(c->d_stage);
+        if (bytes <= kRingSlots * kRingBytes) {
+            if (int rc = stage_ring(c, bytes))
+                return rc;
+            std::memcpy(c->ring, host, bytes);
+            from = reinterpret_cast<const T *>(c->d_ring);
+        } else if (int rc = ring_upload(c, c->d_stage, host, bytes)) {
+            return rc;
+        }
+        k_put_state<T><<<elementwise_blocks(cnt), kBlock, 0, c->stream>>>(
+            dst, from, host_order(c, member), cnt);
+        if (int rc = check_launch("k_put_state"))
             return rc;
     }
     HIPCHK(hipStreamSynchronize(c->stream));
     return 0;
 }
 
-static int from_device_member(swe_hip_ctx *c, int member, const double *src, double *Hhost)
+template <typename T>
+static int from_device(swe_hip_ctx *c, int member, const T *src, T *host)
 {
-    const int n = c->n;
-    c->host_tmp.resize(4 * (size_t)n);
-    double *t = c->host_tmp.data();
+    const long cnt = 4L * c->n;
+    const size_t bytes = sizeof(T) * cnt;
     HIPCHK(hipSetDevice(c->dev));
-    if (c->B == 1) {
-        HIPCHK(hipMemcpyAsync(t, src, sizeof(double) * 4 * n, hipMemcpyDeviceToHost, c->stream));
-    } else {
-        k_get_member<<<elementwise_blocks(4L * n), kBlock, 0, c->stream>>>(c->d_stage, src, member,
-                                                                         c->B, 4L * n);
-        int rc = check_launch("k_get_member");
-        if (rc)
+    if (same_order(c)) {
+        if (int rc = ring_download(c, host, src, bytes))
             return rc;
-        HIPCHK(hipMemcpyAsync(t, c->d_stage, sizeof(double) * 4 * n, hipMemcpyDeviceToHost,
-                              c->stream));
+    } else {
+        const bool direct = bytes <= kRingSlots * kRingBytes;
+        if (direct)
+            if (int rc = stage_ring(c, bytes))
+                return rc;
+        k_get_state<T><<<elementwise_blocks(cnt), kBlock, 0, c->stream>>>(
+            direct ? reinterpret_cast<T *>(c->d_ring) : static_cast<T *>(c->d_stage), src,
+            host_order(c, member), cnt);
+        if (int rc = check_launch("k_get_state"))
+            return rc;
+        if (direct) {
+            HIPCHK(hipStreamSynchronize(c->stream));
+            std::memcpy(host, c->ring, bytes);
+        } else if (int rc = ring_download(c, host, c->d_stage, bytes)) {
+            return rc;
+        }
     }
-    HIPCHK(hipStreamSynchronize(c->stream));
-    if (int rc = check_resident(c))
-        return rc;
-    const std::vector<int> &perm = c->mesh->perm;
-    for (int d = 0; d < n; ++d) {
-        const int i = perm.empty() ? d : perm[d];
-        for (int v = 0; v < 4; ++v)
-            Hhost[c->lay.svm(i, v)] = t[4 * (size_t)d + v];
-    }
-    return 0;
+    return check_resident(c);
 }
 
-// FP32 single state: host layout (SVM_LIN_ID) <-> device [node][4] floats.
-static int to_device32(swe_hip_ctx *c, const float *Hhost, float *dst)
-{
-    const int n = c->n;
-    std::vector<float> t(4 * (size_t)n);
-    const std::vector<int> &perm = c->mesh->perm;
-    for (int d = 0; d < n; ++d) {
-        const int i = perm.empty() ? d : perm[d];
-        for (int v = 0; v < 4; ++v)
-            t[4 * (size_t)d + v] = Hhost[c->lay.svm(i, v)];
-    }
-    HIPCHK(hipSetDevice(c->dev));
-    HIPCHK(hipMemcpyAsync(dst, t.data(), sizeof(float) * 4 * n, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    return 0;
-}
-
-static int from_device32(swe_hip_ctx *c, const float *src, float *Hhost)
-{
-    const int n = c->n;
-    std::vector<float> t(4 * (size_t)n);
-    HIPCHK(hipSetDevice(c->dev));
-    HIPCHK(hipMemcpyAsync(t.data(), src, sizeof(float) * 4 * n, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    if (int rc = check_resident(c))
-        return rc;
-    const std::vector<int> &perm = c->mesh->perm;
-    for (int d = 0; d < n; ++d) {
-        const int i = perm.empty() ? d : perm[d];
-        for (int v = 0; v < 4; ++v)
-            Hhost[c->lay.svm(i, v)] = t[4 * (size_t)d + v];
-    }
-    return 0;
-}
+extern "C" {
 
 int swe_hip_set_state(swe_hip_ctx *c, int member, const double *H)
 {
@@ -1445,7 +1551,7 @@ int swe_hip_set_state(swe_hip_ctx *c, int member, const double *H)
         return fail(SWE_HIP_EINVAL, "set_state: bad ctx, pointer or member");
     if (c->fp32)
         return fail(SWE_HIP_EINVAL, "set_state: FP32 context, use swe_hip_set_state32");
-    return to_device_member(c, member, H, c->d_H);
+    return to_device(c, member, H, c->d_H);
 }
 
 int swe_hip_get_state(swe_hip_ctx *c, int member, double *H)
@@ -1454,7 +1560,7 @@ int swe_hip_get_state(swe_hip_ctx *c, int member, double *H)
         return fail(SWE_HIP_EINVAL, "get_state: bad ctx, pointer or member");
     if (c->fp32)
         return fail(SWE_HIP_EINVAL, "get_state: FP32 context, use swe_hip_get_state32");
-    return from_device_member(c, member, c->d_H, H);
+    return from_device(c, member, c->d_H, H);
 }
 
 int swe_hip_set_state32(swe_hip_ctx *c, int member, const float *H)
@@ -1462,7 +1568,7 @@ int swe_hip_set_state32(swe_hip_ctx *c, int member, const float *H)
     if (!c || !H || member != 0 || !c->fp32)
         return fail(SWE_HIP_EINVAL, "set_state32: bad ctx, pointer or member (FP32 contexts "
                                     "only, member 0)");
-    return to_device32(c, H, c->f_H);
+    return to_device(c, 0, H, c->f_H);
 }
 
 int swe_hip_get_state32(swe_hip_ctx *c, int member, float *H)
@@ -1470,7 +1576,7 @@ int swe_hip_get_state32(swe_hip_ctx *c, int member, float *H)
     if (!c || !H || member != 0 || !c->fp32)
         return fail(SWE_HIP_EINVAL, "get_state32: bad ctx, pointer or member (FP32 contexts "
                                     "only, member 0)");
-    return from_device32(c, c->f_H, H);
+    return from_device(c, 0, c->f_H, H);
 }
 
 // The RHS buffer F of the drop-in path, allocated (and zeroed) on its first
@@ -1505,14 +1611,14 @@ int swe_hip_eval_rhs32(swe_hip_ctx *c, int member, const float *K, float *F)
                                     "only, member 0)");
     int rc = ensure_F(c);
     if (!rc)
-        rc = to_device32(c, K, c->k_in_b ? c->f_Ka : c->f_Kb);   // not the substeps' K
+        rc = to_device(c, 0, K, c->k_in_b ? c->f_Ka : c->f_Kb);   // not the substeps' K
     if (rc)
         return rc;
     launch_rhs32(c, c->k_in_b ? c->f_Ka : c->f_Kb, c->f_F);
     rc = check_launch("eval_RHS kernel (FP32)");
     if (rc)
         return rc;
-    return from_device32(c, c->f_F, F);
+    return from_device(c, 0, c->f_F, F);
 }
 
 // The drop-in substep of an FP32 context: RK_substep with the reference's
@@ -1567,14 +1673,14 @@ int swe_hip_eval_rhs(swe_hip_ctx *c, int member, const double *K, double *F)
     if (rc)
         return rc;
     double *in = c->k_in_b ? c->d_Ka : c->d_Kb;   // not the substeps' K
-    rc = to_device_member(c, member, K, in);
+    rc = to_device(c, member, K, in);
     if (rc)
         return rc;
     launch_rhs(c, in, c->d_F);
     rc = check_launch("eval_RHS kernel");
     if (rc)
         return rc;
-    return from_device_member(c, member, c->d_F, F);
+    return from_device(c, member, c->d_F, F);
 }
 
 int swe_hip_rk_substep(swe_hip_ctx *c, int s)

@@ -1,35 +1,30 @@
 // Host side of the matrix-core resident kernels: the kernel order, the tiles
 // and their row lists, the launch.
+#include "host_par.h"
 #include "units.h"
 
 #include <algorithm>
-#include <atomic>
 #include <cmath>
+#include <cstring>
 #include <new>
 #include <numeric>
-#include <system_error>
-#include <thread>
 
 namespace swe {
 
 namespace {
 
-template <typename T>
-int upload(swe_hip_ctx *c, T **dst, const std::vector<T> &v, std::string *err)
-{
-    const size_t bytes = sizeof(T) * v.size();
-    if (hipMalloc((void **)dst, bytes ? bytes : 8) != hipSuccess) {
-        *err = "unit tables: hipMalloc";
-        return SWE_HIP_ENOMEM;
+// The tables, gathered for one allocation and one copy.
+struct Tables {
+    std::vector<char> bytes;
+    template <typename T>
+    size_t add(const std::vector<T> &v)
+    {
+        const size_t at = (bytes.size() + 255) / 256 * 256;
+        bytes.resize(at + sizeof(T) * v.size());
+        std::memcpy(bytes.data() + at, v.data(), sizeof(T) * v.size());
+        return at;
     }
-    c->bytes += (long long)bytes;
-    c->units.bytes += (long long)bytes;
-    if (hipMemcpy(*dst, v.data(), bytes, hipMemcpyHostToDevice) != hipSuccess) {
-        *err = "unit tables: upload";
-        return SWE_HIP_EDEVICE;
-    }
-    return 0;
-}
+};
 
 // Place of (node of the unit, slot) in a unit's 512 row numbers: FP64 [group of
 // 4 nodes][slot & 3][node][slot / 4], FP32 [slot / 8][node][slot & 7].
@@ -39,50 +34,12 @@ int prec_at(bool fp32, int m, int slot)
                 : (m >> 2) * 128 + ((slot & 3) * 4 + (m & 3)) * 8 + (slot >> 2);
 }
 
-// Runs the tasks on host threads of their own (in line where no thread can be
-// had); an exception in any (out of memory) is thrown again once all are done.
-template <typename F>
-void in_parallel(int tasks, F f)
-{
-    std::atomic<bool> failed{false};
-    auto guarded = [&](int k) {
-        try {
-            f(k);
-        } catch (...) {
-            failed = true;
-        }
-    };
-    std::vector<std::thread> th(tasks > 1 ? tasks - 1 : 0);
-    for (int k = 1; k < tasks; ++k) {
-        try {
-            th[k - 1] = std::thread(guarded, k);
-        } catch (const std::system_error &) {
-            guarded(k);
-        }
-    }
-    guarded(0);
-    for (std::thread &t : th)
-        if (t.joinable())
-            t.join();
-    if (failed)
-        throw std::bad_alloc();
-}
-
-// f(first, last) over [0, n) in up to 8 ranges.
-template <typename F>
-void parallel_ranges(int n, F f)
-{
-    const int nt = std::max(1, std::min({n, 8, (int)std::thread::hardware_concurrency()}));
-    in_parallel(nt, [&](int k) { f((int)((long)n * k / nt), (int)((long)n * (k + 1) / nt)); });
-}
-
 }  // namespace
 
 void units_free(swe_hip_ctx *c)
 {
     SweUnits &u = c->units;
-    void *ptrs[] = {u.d_wrec, u.d_prec, u.d_grec, u.d_tile_start, u.d_unit_start, u.d_ustart,
-                    u.d_ulist, u.d_own_row, u.d_perm, u.d_hd};
+    void *ptrs[] = {u.d_wrec, u.d_grec, u.d_hd, u.d_tables};
     for (void *p : ptrs)
         if (p)
             (void)hipFree(p);
@@ -164,7 +121,7 @@ static int build(swe_hip_ctx *c, std::vector<std::vector<int>> *nbr_tiles, std::
     std::vector<int> perm(n), inv(n);
     std::iota(perm.begin(), perm.end(), 0);
     bisect(xyz, n, perm, 0, n, tmax);
-    parallel_ranges(nt, [&](int a, int b) {
+    parallel_ranges(nt, 4096 / tmax, [&](int a, int b) {
         for (int t = a; t < b; ++t)
             bisect(xyz, n, perm, t * tmax, std::min(n, (t + 1) * tmax), 16);
     });
@@ -181,7 +138,7 @@ static int build(swe_hip_ctx *c, std::vector<std::vector<int>> *nbr_tiles, std::
     std::vector<uint4> precq((size_t)units * 64);
     unsigned short *prec = reinterpret_cast<unsigned short *>(precq.data());
     nbr_tiles->assign(nt, {});
-    parallel_ranges(nt, [&](int a, int b) {
+    parallel_ranges(nt, 4096 / tmax, [&](int a, int b) {
         std::vector<int> mark(n, -1), where(n);
         for (int t = a; t < b; ++t) {
             std::vector<int> &l = list[t];
@@ -241,24 +198,35 @@ static int build(swe_hip_ctx *c, std::vector<std::vector<int>> *nbr_tiles, std::
     std::vector<int> unit_tile(units);
     for (int t = 0; t < nt; ++t)
         std::fill(unit_tile.begin() + unit_start[t], unit_tile.begin() + unit_start[t + 1], t);
-    int *d_unit_tile = nullptr;
-    int rc = upload(c, &u.d_tile_start, tstart, err);
-    if (!rc) rc = upload(c, &u.d_unit_start, unit_start, err);
-    if (!rc) rc = upload(c, &u.d_ustart, ustart, err);
-    if (!rc) rc = upload(c, &u.d_ulist, ulist, err);
-    if (!rc) rc = upload(c, &u.d_own_row, own_row, err);
-    if (!rc) rc = upload(c, &u.d_perm, perm, err);
-    if (!rc) rc = upload(c, &u.d_prec, precq, err);
-    if (!rc) rc = upload(c, &d_unit_tile, unit_tile, err);
+    Tables tb;
+    const size_t at[] = {tb.add(precq),  tb.add(tstart), tb.add(unit_start), tb.add(ustart),
+                         tb.add(ulist),  tb.add(own_row), tb.add(perm),      tb.add(unit_tile)};
+    int rc = 0;
+    if (hipMalloc((void **)&u.d_tables, tb.bytes.size()) != hipSuccess) {
+        u.d_tables = nullptr;
+        *err = "unit tables: hipMalloc";
+        return SWE_HIP_ENOMEM;
+    }
+    c->bytes += (long long)tb.bytes.size();
+    u.bytes += (long long)tb.bytes.size();
+    if (hipMemcpy(u.d_tables, tb.bytes.data(), tb.bytes.size(), hipMemcpyHostToDevice)
+        != hipSuccess) {
+        *err = "unit tables: upload";
+        return SWE_HIP_EDEVICE;
+    }
+    auto ints = [&](int k) { return reinterpret_cast<const int *>(u.d_tables + at[k]); };
+    u.d_prec = reinterpret_cast<const uint4 *>(u.d_tables + at[0]);
+    u.d_tile_start = ints(1);
+    u.d_unit_start = ints(2);
+    u.d_ustart = ints(3);
+    u.d_ulist = ints(4);
+    u.d_own_row = ints(5);
+    u.d_perm = ints(6);
+    u.d_unit_tile = ints(7);
     if (!rc) {
-        rc = c->fp32 ? units_pack32(c, units, d_unit_tile) : units_pack64(c, units, d_unit_tile);
+        rc = c->fp32 ? units_pack32(c, units) : units_pack64(c, units);
         if (rc)
             *err = "unit records: allocation or pack kernel";
-    }
-    if (d_unit_tile) {
-        (void)hipFree(d_unit_tile);
-        c->bytes -= (long long)(sizeof(int) * unit_tile.size());
-        u.bytes -= (long long)(sizeof(int) * unit_tile.size());
     }
     return rc;
 }

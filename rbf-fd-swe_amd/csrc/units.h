@@ -41,8 +41,8 @@ bool units_plan32(SweUnits &u);
 // Kernel of a plan, its record packing and its launch.
 void *units_kernel64(const SweUnits &u);
 void *units_kernel32(const SweUnits &u);
-int units_pack64(swe_hip_ctx *c, int units, const int *unit_tile);
-int units_pack32(swe_hip_ctx *c, int units, const int *unit_tile);
+int units_pack64(swe_hip_ctx *c, int units);
+int units_pack32(swe_hip_ctx *c, int units);
 hipError_t units_launch64(swe_hip_ctx *c, int nsteps, const DevResSync &y);
 hipError_t units_launch32(swe_hip_ctx *c, int nsteps, const DevResSync &y);
 // The table part of a launch's arguments.
