@@ -115,8 +115,10 @@ int swe_hip_eval_rhs32(swe_hip_ctx *ctx, int member, const float *K, float *F);
 
 /* Extended creation.  members/flags/device as swe_hip_create; member_block
  * is the number of members one lane group of the ensemble kernel serves
- * (a power of two 2..64 dividing members; 0 = the largest such value; 64
- * with a 31-point stencil = the member-pair kernel, two members per lane);
+ * (a power of two 2..64 dividing members; 0 = the library's choice: in fast
+ * mode with a 31-point stencil the matrix-core ensemble kernel, which keeps
+ * weight and geometry records of 1.3 KB per node, else the largest such value;
+ * 64 with a 31-point stencil = the member-pair kernel, two members per lane);
  * share, when not NULL, is a context of the same mesh whose device copy of
  * the static data is reused (s may then be NULL): the static data stay
  * resident until the last context using them is destroyed.  Out-of-range
@@ -203,7 +205,11 @@ typedef struct swe_hip_options {
                                    with share: the mesh's order is used)    */
     int tiled;                  /* 1: LDS-staged ensemble kernel (members
                                    >= 32, member_block 32, 31-point
-                                   stencil): persistent member-lane tiles,
+                                   stencil): in fast mode the matrix-core
+                                   kernel (same bits; tile_nodes, tile_rows
+                                   and prefetch then have no effect) unless
+                                   its tiles do not fit; else persistent
+                                   member-lane tiles,
                                    loader and compute waves over two LDS
                                    images, 160 KB per workgroup             */
     int slot_block;             /* stencil arrays: 0 slot-major [nnbr][n];

@@ -314,42 +314,54 @@ __global__ __launch_bounds__(512) void k_steps_units(DevUnits64 p)
     }
 }
 
-// Packs the unit records (units_build): thread = (unit, group and slot pair,
-// lane) of wrec, and the first 192 of a unit's threads its geometry.
-__global__ void k_pack_units(DevMesh m, const int *tile_start, const int *unit_start,
-                             const int *unit_tile, const int *perm, double2 *wrec, double2 *grec)
+// Packs the weight records: one workgroup per unit, thread = (group and slot
+// pair, lane).
+__global__ void k_pack_weights(DevMesh m, const int *tile_start, const int *unit_start,
+                               const int *unit_tile, const int *perm, double2 *wrec)
 {
     const int unit = (int)blockIdx.x;
     const int tile = unit_tile[unit];
     const int lane = (int)threadIdx.x & 63, q = (int)threadIdx.x >> 6;
-    const int n0 = tile_start[tile] + 16 * (unit - unit_start[tile]);
+    const int g = q >> 2, k = lane >> 4, b = (lane >> 2) & 3, x = lane & 3;
+    const int node = tile_start[tile] + 16 * (unit - unit_start[tile]) + 4 * g + b;
+    double v[2] = {0.0, 0.0};
+    for (int c = 0; c < 2; ++c) {
+        const int slot = 4 * (2 * (q & 3) + c) + k;
+        if (node < tile_start[tile + 1] && slot < m.nnbr)
+            v[c] = m.wts[4L * (slot_base<0>(m, perm[node]) + (long)slot * slot_stride(m)) + x];
+    }
+    wrec[(long)unit * 1024 + 64 * q + lane] = make_double2(v[0], v[1]);
+}
+
+// Packs the geometry records: one workgroup per unit, thread = (piece, lane).
+__global__ void k_pack_geo(DevMesh m, const int *tile_start, const int *unit_start,
+                           const int *unit_tile, const int *perm, double2 *grec)
+{
+    const int unit = (int)blockIdx.x;
+    const int tile = unit_tile[unit];
+    const int lane = (int)threadIdx.x & 63, q = (int)threadIdx.x >> 6;
+    const int j = lane & 3;
+    const int node = tile_start[tile] + 16 * (unit - unit_start[tile])
+                     + (q < 2 ? lane >> 2 : lane & 15);
     const int n1 = tile_start[tile + 1];
-    {
-        const int g = q >> 2, k = lane >> 4, b = (lane >> 2) & 3, x = lane & 3;
-        const int node = n0 + 4 * g + b;
-        double v[2] = {0.0, 0.0};
-        for (int c = 0; c < 2; ++c) {
-            const int slot = 4 * (2 * (q & 3) + c) + k;
-            if (node < n1 && slot < m.nnbr)
-                v[c] = m.wts[4L * (slot_base<0>(m, perm[node]) + (long)slot * slot_stride(m)) + x];
-        }
-        wrec[(long)unit * 1024 + 64 * q + lane] = make_double2(v[0], v[1]);
-    }
+    const int field[4][4] = {{G_X, G_PU, G_PU + 1, G_PU + 2},
+                             {G_Y, G_PV, G_PV + 1, G_PV + 2},
+                             {G_Z, G_PW, G_PW + 1, G_PW + 2},
+                             {G_F, G_GG, G_GG + 1, G_GG + 2}};
+    auto fetch = [&](int f) { return node < n1 ? m.geo[(long)f * m.ld + perm[node]] : 0.0; };
     double2 *gu = grec + (long)kUnitGeo * unit;
-    if (q < 3) {
-        const int node = n0 + (q < 2 ? lane >> 2 : lane & 15), j = lane & 3;
-        const int field[4][4] = {{G_X, G_PU, G_PU + 1, G_PU + 2},
-                                 {G_Y, G_PV, G_PV + 1, G_PV + 2},
-                                 {G_Z, G_PW, G_PW + 1, G_PW + 2},
-                                 {G_F, G_GG, G_GG + 1, G_GG + 2}};
-        auto fetch = [&](int f) {
-            return node < n1 ? m.geo[(long)f * m.ld + perm[node]] : 0.0;
-        };
-        if (q < 2)
-            gu[64 * q + lane] = make_double2(fetch(field[j][2 * q]), fetch(field[j][2 * q + 1]));
-        else if (lane < 16)
-            reinterpret_cast<double *>(gu + 128)[lane] = fetch(G_GHM);
-    }
+    if (q < 2)
+        gu[64 * q + lane] = make_double2(fetch(field[j][2 * q]), fetch(field[j][2 * q + 1]));
+    else if (lane < 16)
+        reinterpret_cast<double *>(gu + 128)[lane] = fetch(G_GHM);
+}
+
+void pack_weights64(swe_hip_ctx *c, int units)
+{
+    const SweUnits &u = c->units;
+    k_pack_weights<<<units, 1024, 0, c->stream>>>(mesh_of(c), u.d_tile_start, u.d_unit_start,
+                                                  u.d_unit_tile, u.d_perm,
+                                                  static_cast<double2 *>(u.d_wrec));
 }
 
 bool units_plan64(SweUnits &u)
@@ -397,10 +409,10 @@ int units_pack64(swe_hip_ctx *c, int units)
         return SWE_HIP_ENOMEM;
     c->bytes += (long long)(wb + gb + hb);
     u.bytes += (long long)(wb + gb + hb);
-    k_pack_units<<<units, 1024, 0, c->stream>>>(mesh_of(c), u.d_tile_start, u.d_unit_start,
-                                                u.d_unit_tile, u.d_perm,
-                                                static_cast<double2 *>(u.d_wrec),
-                                                static_cast<double2 *>(u.d_grec));
+    pack_weights64(c, units);
+    k_pack_geo<<<units, 192, 0, c->stream>>>(mesh_of(c), u.d_tile_start, u.d_unit_start,
+                                             u.d_unit_tile, u.d_perm,
+                                             static_cast<double2 *>(u.d_grec));
     return hipGetLastError() == hipSuccess && hipStreamSynchronize(c->stream) == hipSuccess
                ? 0 : SWE_HIP_EDEVICE;
 }

@@ -99,6 +99,7 @@ struct SweUnits {
     int units = 0, rows = 0;      // most units and rows of one tile
     int waves = 0, lds = 0;       // waves per workgroup, dynamic LDS bytes
     int mode = 0;                 // UnitMode (units.h)
+    int halves = 0;               // ensembles: 8-member halves of an item
     int chains = 1;               // FP32: partial sums per stencil sum, as split32's lanes
     int pos = 0, geo = 0;         // units whose positions, geometry the LDS holds
     long long bytes = 0;          // counted in the context's bytes too
@@ -238,11 +239,14 @@ void launch_fp32_stage(const swe_hip_ctx *c, int stage, const DevStage32 &st);
 void launch_single_stage(const swe_hip_ctx *c, int stage, const DevStage &st);
 void launch_members_stage(const swe_hip_ctx *c, int stage, const DevStage &st);
 void launch_tiled_stage(const swe_hip_ctx *c, int stage, const DevStage &st);
+void launch_ensemble_stage(const swe_hip_ctx *c, int stage, const DevStage &st);
 
 inline void launch_stage(const swe_hip_ctx *c, int stage, const DevStage &st)
 {
     if (c->B == 1)
         launch_single_stage(c, stage, st);
+    else if (c->units.ntiles > 0)
+        launch_ensemble_stage(c, stage, st);
     else if (c->tiles.ntiles > 0)
         launch_tiled_stage(c, stage, st);
     else

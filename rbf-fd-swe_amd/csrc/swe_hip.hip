@@ -480,7 +480,7 @@ int build_mesh(const swe_hip_static *s, int device, int order, int sblk, bool fp
     std::vector<double> geo((size_t)GEO_N * n);
     // the first id out of range, as (device node) W + slot
     std::atomic<long> bad{(long)n * W};
-    parallel_ranges(n, 4096, [&](int first, int last) {
+    parallel_ranges(n, 2048, [&](int first, int last) {
         for (int dnode = first; dnode < last; ++dnode) {
             const int i = host_of(dnode);
             for (int j = 0; j < W; ++j) {
@@ -1180,7 +1180,22 @@ int swe_hip_create_ex(const swe_hip_static *s, const swe_hip_options *o, swe_hip
             rc = 0;
         }
     }
-    if (!rc && o->tiled) {
+    // fast-mode ensembles on 31-point stencils run on the matrix cores when the
+    // caller leaves the kernel open (no member block named) or asks for LDS
+    // tiles, unless a tile's rows do not fit the LDS or the records the
+    // device's memory; a named member block keeps its kernel and its bytes
+    if (!rc && c->B > 1 && c->nnbr == 31 && !exact(c) && (o->member_block == 0 || o->tiled)) {
+        std::string why;
+        std::vector<std::vector<int>> reads;
+        int e = units_build(c, &reads, &why);
+        if (!e)
+            e = units_prepare(c, &why);
+        if (e) {
+            (void)hipGetLastError();
+            units_free(c);
+        }
+    }
+    if (!rc && o->tiled && c->units.ntiles == 0) {
         int lds_max = 0;
         {
             if (c->nnbr != 31)

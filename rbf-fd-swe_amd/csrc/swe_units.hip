@@ -99,7 +99,7 @@ void bisect(const double *xyz, int n, std::vector<int> &ids, int first, int last
     auto half = [&](int k) {
         bisect(xyz, n, ids, k ? first + left : first, k ? last : first + left, chunk);
     };
-    if (count > 16384) {
+    if (count > 4096) {
         in_parallel(2, half);
     } else {
         half(0);
@@ -113,7 +113,10 @@ static int build(swe_hip_ctx *c, std::vector<std::vector<int>> *nbr_tiles, std::
 {
     const int n = c->n, W = c->nnbr;
     SweUnits &u = c->units;
-    const int tmax = std::max(16, (n + c->ncu - 1) / c->ncu);
+    const bool ensemble = c->B > 1;
+    // ensembles: items of 16 members on tiles of 32 nodes, or 8 on 64
+    u.halves = c->B > 8 ? 2 : 1;
+    const int tmax = ensemble ? kEnsNodes / u.halves : std::max(16, (n + c->ncu - 1) / c->ncu);
     const int nt = (n + tmax - 1) / tmax;
     const std::vector<int> &nbr = c->mesh->h_nbr;
     // kernel order: compact tiles of compact units
@@ -121,7 +124,7 @@ static int build(swe_hip_ctx *c, std::vector<std::vector<int>> *nbr_tiles, std::
     std::vector<int> perm(n), inv(n);
     std::iota(perm.begin(), perm.end(), 0);
     bisect(xyz, n, perm, 0, n, tmax);
-    parallel_ranges(nt, 4096 / tmax, [&](int a, int b) {
+    parallel_ranges(nt, 1024 / tmax, [&](int a, int b) {
         for (int t = a; t < b; ++t)
             bisect(xyz, n, perm, t * tmax, std::min(n, (t + 1) * tmax), 16);
     });
@@ -138,7 +141,7 @@ static int build(swe_hip_ctx *c, std::vector<std::vector<int>> *nbr_tiles, std::
     std::vector<uint4> precq((size_t)units * 64);
     unsigned short *prec = reinterpret_cast<unsigned short *>(precq.data());
     nbr_tiles->assign(nt, {});
-    parallel_ranges(nt, 4096 / tmax, [&](int a, int b) {
+    parallel_ranges(nt, 1024 / tmax, [&](int a, int b) {
         std::vector<int> mark(n, -1), where(n);
         for (int t = a; t < b; ++t) {
             std::vector<int> &l = list[t];
@@ -158,7 +161,7 @@ static int build(swe_hip_ctx *c, std::vector<std::vector<int>> *nbr_tiles, std::
             for (int k = 0; k < (int)l.size(); ++k) {
                 where[l[k]] = k;
                 const int o = l[k] / tmax;
-                if (o != t && ((*nbr_tiles)[t].empty() || (*nbr_tiles)[t].back() != o))
+                if (!ensemble && o != t && ((*nbr_tiles)[t].empty() || (*nbr_tiles)[t].back() != o))
                     (*nbr_tiles)[t].push_back(o);
             }
             own_row[t] = where[tstart[t]];
@@ -191,7 +194,11 @@ static int build(swe_hip_ctx *c, std::vector<std::vector<int>> *nbr_tiles, std::
     u.units = (tmax + 15) / 16;
     u.rows = rows;
     u.waves = std::min(8, std::max(4, u.units));
-    if (!(c->fp32 ? units_plan32(u) : units_plan64(u)) || rows > 65534) {
+    if (ensemble)
+        for (int &q : ulist)
+            q = perm[q];   // rows by device node: stages exchange the state itself
+    if (!(ensemble ? ensemble_plan(u) : c->fp32 ? units_plan32(u) : units_plan64(u))
+        || rows > 65534) {
         *err = "unit kernel: a tile's rows do not fit the LDS";
         return SWE_HIP_EINVAL;
     }
@@ -224,7 +231,8 @@ static int build(swe_hip_ctx *c, std::vector<std::vector<int>> *nbr_tiles, std::
     u.d_perm = ints(6);
     u.d_unit_tile = ints(7);
     if (!rc) {
-        rc = c->fp32 ? units_pack32(c, units) : units_pack64(c, units);
+        rc = ensemble ? ensemble_pack(c, units)
+                      : c->fp32 ? units_pack32(c, units) : units_pack64(c, units);
         if (rc)
             *err = "unit records: allocation or pack kernel";
     }
@@ -261,6 +269,8 @@ void units_tables(const swe_hip_ctx *c, int nsteps, const DevResSync &y, DevUnit
 
 int units_prepare(swe_hip_ctx *c, std::string *err)
 {
+    if (c->B > 1)
+        return ensemble_prepare(c, err);
     void *fn = c->fp32 ? units_kernel32(c->units) : units_kernel64(c->units);
     int per_cu = 0;
     if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, kUnitsMaxLds)

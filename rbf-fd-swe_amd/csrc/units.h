@@ -41,7 +41,13 @@ bool units_plan32(SweUnits &u);
 // Kernel of a plan, its record packing and its launch.
 void *units_kernel64(const SweUnits &u);
 void *units_kernel32(const SweUnits &u);
+void pack_weights64(swe_hip_ctx *c, int units);
 int units_pack64(swe_hip_ctx *c, int units);
+// The same for the ensemble stage kernel (k_ensemble.hip).
+bool ensemble_plan(SweUnits &u);
+int ensemble_pack(swe_hip_ctx *c, int units);
+int ensemble_prepare(swe_hip_ctx *c, std::string *err);
+constexpr int kEnsNodes = 64;   // nodes per tile of the ensemble kernel with items of 8 members
 int units_pack32(swe_hip_ctx *c, int units);
 hipError_t units_launch64(swe_hip_ctx *c, int nsteps, const DevResSync &y);
 hipError_t units_launch32(swe_hip_ctx *c, int nsteps, const DevResSync &y);
