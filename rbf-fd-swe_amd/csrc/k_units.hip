@@ -28,8 +28,9 @@
 //   N = 10242    2.69 against 3.39   exchange latency
 //   N = 40962    3.7  against 4.35   exchange latency; 0.6 us of LDS conflicts
 //   N = 163842   19.4 against 32.6   111 MB re-read (16 of 41 units per tile stay)
-//   N = 302762   74   against 96
-//   N = 655362   180  against 197    1.4 KB per node re-read, 4.9 TB/s
+//   N = 302762   70   against 96
+//   N = 655362   170  against 197    1.37 KB per node and stage, 5.3 TB/s (180
+//                                    with H kept beside D instead of in X0)
 #include "units.h"
 
 #include <algorithm>
@@ -41,7 +42,7 @@ struct DevUnits64 : DevUnits {
     const double2 *grec;        // [units][kUnitGeo] UnitGeo of its 64 lanes
     double *H;                  // the context's state
     double *X0, *Xa, *Xb;       // exchanged states, kernel order
-    double2 *hd;                // [units][64] H, D of streamed units (UM_GLOBAL)
+    double *d;                  // [units][64] D of streamed units (UM_GLOBAL; H is X0's)
     double gh0;
     double c[4];                // K = H + c F (dt/2, dt/2, dt); stage 3: H += c D (dt/6)
     double dcoef[4];            // D += dcoef F (0: D = F, 2, 2, 1)
@@ -127,7 +128,7 @@ __global__ __launch_bounds__(512) void k_steps_units(DevUnits64 p)
     });
     double2 ring[STREAM ? RING : 1];
     uint4 pnext[MODE == UM_GLOBAL ? 4 : 1];
-    double2 *const hd_mem = p.hd + 64L * ug + lane;
+    double *const d_mem = p.d + 64L * ug + lane;
     if constexpr (STREAM) {
         for (int u = wv + R * nw; u < nu; u += nw) {
             double h = 0.0;
@@ -135,8 +136,10 @@ __global__ __launch_bounds__(512) void k_steps_units(DevUnits64 p)
                 h = p.H[4L * p.perm[first + 16 * u] + j];
             if constexpr (MODE == UM_STREAM)
                 hd[64 * (u - R * nw) + lane] = make_double2(h, 0.0);
-            else
-                hd_mem[64L * u] = make_double2(h, 0.0);
+            else if (16 * u + (lane >> 2) < tcount)
+                __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, h),
+                                                      state_rsrc(p.X0, p.bytes),
+                                                      8 * (4 * t0 + 64 * u + lane), 0, kSc1);
         }
         const int u = wv + R * nw;
         if (u < nu) {
@@ -283,7 +286,17 @@ __global__ __launch_bounds__(512) void k_steps_units(DevUnits64 p)
                             pv[q] = pos[64 * u + 16 * q + (lane >> 2)];
                     } else {
                         g = geo_of(p.grec + (long)kUnitGeo * (ug + u));
-                        hv = hd_mem[64L * u];
+                        // stage 0 gathers H: it is in the own row
+                        if constexpr (s == 0) {
+                            hv.x = *reinterpret_cast<const double *>(
+                                rows + 32 * (own0 + 16 * u + (lane >> 2)) + 8 * j);
+                        } else {
+                            hv.x = __builtin_bit_cast(
+                                double, __builtin_amdgcn_raw_buffer_load_b64(
+                                            state_rsrc(p.X0, p.bytes),
+                                            8 * (4 * t0 + 64 * u + lane), 0, kSc1));
+                            hv.y = d_mem[64L * u];
+                        }
 #pragma unroll
                         for (int q = 0; q < 4; ++q) {
                             pv[q] = pnext[q];
@@ -305,8 +318,8 @@ __global__ __launch_bounds__(512) void k_steps_units(DevUnits64 p)
                     update(u, rhs(u, acc, g), hv.x, hv.y);
                     if constexpr (MODE == UM_STREAM)
                         hd[64 * (u - R * nw) + lane] = hv;
-                    else
-                        hd_mem[64L * u] = hv;
+                    else if constexpr (s < 3)
+                        d_mem[64L * u] = hv.y;
                 }
             }
             res_publish(p.y, tile, ++stage);
@@ -403,7 +416,7 @@ int units_pack64(swe_hip_ctx *c, int units)
     SweUnits &u = c->units;
     const size_t wb = sizeof(double2) * 1024 * (size_t)units;
     const size_t gb = sizeof(double2) * kUnitGeo * (size_t)units;
-    const size_t hb = u.mode == UM_GLOBAL ? sizeof(double2) * 64 * (size_t)units : 0;
+    const size_t hb = u.mode == UM_GLOBAL ? sizeof(double) * 64 * (size_t)units : 0;
     if (hipMalloc(&u.d_wrec, wb) != hipSuccess || hipMalloc(&u.d_grec, gb) != hipSuccess
         || (hb && hipMalloc(&u.d_hd, hb) != hipSuccess))
         return SWE_HIP_ENOMEM;
@@ -424,7 +437,7 @@ hipError_t units_launch64(swe_hip_ctx *c, int nsteps, const DevResSync &y)
     units_tables(c, nsteps, y, &p);
     p.wrec = static_cast<const double2 *>(u.d_wrec);
     p.grec = static_cast<const double2 *>(u.d_grec);
-    p.hd = static_cast<double2 *>(u.d_hd);
+    p.d = static_cast<double *>(u.d_hd);
     p.H = c->d_H;
     p.X0 = c->d_D;   // D lives in the kernel
     p.Xa = c->d_Ka;

@@ -26,7 +26,7 @@ struct DevUnits32 : DevUnits {
     const float4 *rec;          // [units][kRec32][64]: 31 slots and ghm, geometry
     float *H;                   // the context's state
     float *X0, *Xa, *Xb;        // exchanged states, kernel order
-    float2 *hd;                 // [units][64] H, D of streamed units (UM_GLOBAL)
+    float *d;                   // [units][64] D of streamed units (UM_GLOBAL; H is X0's)
     float gh0;
     float c[3];                 // K = H + c F: (float)(dt/2.0), (float)(dt/2.0), dt
     double c6;                  // stage 3: H += (dt/6.0) D in double
@@ -111,7 +111,7 @@ __global__ __launch_bounds__(512) void k_steps_units32(DevUnits32 p)
     });
     float4 ring[STREAM ? kRec32 : 1];   // the next streamed record
     uint4 pnext[MODE == UM_GLOBAL ? 4 : 1];
-    float2 *const hd_mem = p.hd + 64L * ug + lane;
+    float *const d_mem = p.d + 64L * ug + lane;
     if constexpr (STREAM) {
         for (int u = wv + R * nw; u < nu; u += nw) {
             float h = 0.0f;
@@ -119,8 +119,10 @@ __global__ __launch_bounds__(512) void k_steps_units32(DevUnits32 p)
                 h = p.H[4L * p.perm[first + 16 * u] + j];
             if constexpr (MODE == UM_STREAM)
                 hd[64 * (u - R * nw) + lane] = make_float2(h, 0.0f);
-            else
-                hd_mem[64L * u] = make_float2(h, 0.0f);
+            else if (16 * u + (lane >> 2) < tcount)
+                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, h),
+                                                      state_rsrc(p.X0, p.bytes),
+                                                      4 * (4 * t0 + 64 * u + lane), 0, kSc1);
         }
         const int u = wv + R * nw;
         if (u < nu) {
@@ -265,8 +267,19 @@ __global__ __launch_bounds__(512) void k_steps_units32(DevUnits32 p)
                             pnext[q] = p.prec[64L * (ug + un) + 16 * q + (lane >> 2)];
                         }
                     }
-                    if constexpr (MODE == UM_GLOBAL)
-                        hv = hd_mem[64L * u];
+                    if constexpr (MODE == UM_GLOBAL) {
+                        // stage 0 gathers H: it is in the own row
+                        if constexpr (s == 0) {
+                            hv.x = *reinterpret_cast<const float *>(
+                                rows + 16 * (own0 + 16 * u + (lane >> 2)) + 4 * j);
+                        } else {
+                            hv.x = __builtin_bit_cast(
+                                float, __builtin_amdgcn_raw_buffer_load_b32(
+                                           state_rsrc(p.X0, p.bytes),
+                                           4 * (4 * t0 + 64 * u + lane), 0, kSc1));
+                            hv.y = d_mem[64L * u];
+                        }
+                    }
                     Acc acc = {};
                     const float4 g = ring[8];
                     const float ghm = ring[7].w;
@@ -283,8 +296,8 @@ __global__ __launch_bounds__(512) void k_steps_units32(DevUnits32 p)
                     update(u, rhs(u, acc, g, ghm), hv.x, hv.y);
                     if constexpr (MODE == UM_STREAM)
                         hd[64 * (u - R * nw) + lane] = hv;
-                    else
-                        hd_mem[64L * u] = hv;
+                    else if constexpr (s < 3)
+                        d_mem[64L * u] = hv.y;
                 }
             }
             res_publish(p.y, tile, ++stage);
@@ -371,7 +384,7 @@ int units_pack32(swe_hip_ctx *c, int units)
 {
     SweUnits &u = c->units;
     const size_t rb = sizeof(float4) * 64 * kRec32 * (size_t)units;
-    const size_t hb = u.mode == UM_GLOBAL ? sizeof(float2) * 64 * (size_t)units : 0;
+    const size_t hb = u.mode == UM_GLOBAL ? sizeof(float) * 64 * (size_t)units : 0;
     if (hipMalloc(&u.d_wrec, rb) != hipSuccess || (hb && hipMalloc(&u.d_hd, hb) != hipSuccess))
         return SWE_HIP_ENOMEM;
     c->bytes += (long long)(rb + hb);
@@ -389,7 +402,7 @@ hipError_t units_launch32(swe_hip_ctx *c, int nsteps, const DevResSync &y)
     DevUnits32 p{};
     units_tables(c, nsteps, y, &p);
     p.rec = static_cast<const float4 *>(u.d_wrec);
-    p.hd = static_cast<float2 *>(u.d_hd);
+    p.d = static_cast<float *>(u.d_hd);
     p.H = c->f_H;
     p.X0 = c->f_D;   // D lives in the kernel
     p.Xa = c->f_Ka;

@@ -45,17 +45,24 @@ __device__ __forceinline__ void st_agent(unsigned *p, unsigned v)
 }
 
 // Wave 0 polls the neighbour tiles' stage counts (one per lane) until every
-// one has reached `need`; false once any wait in the grid was aborted.
+// one has reached `need`; false once any wait in the grid was aborted.  The
+// lanes without a neighbour read the abort word in the same load (a second
+// load per poll cost 0.05 us a stage).
 __device__ __forceinline__ bool res_wait(const DevResSync &r, int tile, unsigned need)
 {
     __shared__ int ok;
     if (threadIdx.x < 64) {
         const int u = r.nbrs[tile * kResMaxNbrs + (int)threadIdx.x];
-        const unsigned *f = r.sync + (long)(1 + (u >= 0 ? u : tile)) * kResLine;
+        const unsigned *f = u >= 0 ? r.sync + (long)(1 + u) * kResLine : r.sync;
+        const bool watched = __any(u < 0);
         int good = 1;
         unsigned polls = 0;
-        while (!__all(u < 0 || ld_agent(f) >= need)) {
-            if (++polls > r.spin_limit || ld_agent(r.sync)) {
+        for (;;) {
+            const unsigned v = ld_agent(f);
+            if (!__any(u >= 0 && v < need))
+                break;
+            if (++polls > r.spin_limit || __any(u < 0 && v != 0)
+                || (!watched && ld_agent(r.sync))) {
                 if (threadIdx.x == 0) {
                     st_agent(r.sync, 1u);
                     __hip_atomic_store(r.host_abort, 1u, __ATOMIC_RELAXED,

@@ -33,7 +33,7 @@ constexpr int kUnitsMaxLds = 160 * 1024 - 64;   // dynamic LDS of k_steps_units
 // Nodes per compute unit up to which AUTO tries the streaming form of the unit
 // kernels (their own LDS check decides: ~4600 FP64 rows of 32 bytes).  Beyond
 // 256 nodes per unit it beats the stage kernels at every size measured (us per
-// stage, FP64: N = 163842 19.4 against 32.6, 655362 180 against 197; FP32: 7.5
+// stage, FP64: N = 163842 19.4 against 32.6, 655362 170 against 197; FP32: 7.5
 // against 19.7, 78 against 110).
 constexpr int kUnitsMaxPerCu = 4096;
 constexpr int kResMaxNbrs = 64;           // tiles one tile exchanges rows with (one wave)
