@@ -1,6 +1,7 @@
 // Whole RK4 steps of one single-state mesh in one cooperative launch, exact
-// mode (fast mode: k_units.hip, k_units32.hip, whose matrix instructions fuse
-// every multiply-add): each workgroup owns one tile of consecutive nodes for
+// mode (FP64 up to 64 nodes per compute unit: k_exact.hip; fast mode:
+// k_units.hip, k_units32.hip, whose matrix instructions fuse every
+// multiply-add): each workgroup owns one tile of consecutive nodes for
 // the whole launch and keeps everything static about them -- 31 x 4 weights,
 // stencil positions, geometry -- and its running H and D in registers; per
 // stage it waits for the tiles it exchanges rows with, copies its tile's

@@ -36,6 +36,10 @@ constexpr int kUnitsMaxLds = 160 * 1024 - 64;   // dynamic LDS of k_steps_units
 // stage, FP64: N = 163842 19.4 against 32.6, 655362 170 against 197; FP32: 7.5
 // against 19.7, 78 against 110).
 constexpr int kUnitsMaxPerCu = 4096;
+// Nodes per compute unit up to which exact FP64 contexts run k_steps_exact (a
+// 4-node group on each of 16 waves; 126 registers, more waves do not fit):
+// 3.58 against 4.16 us per stage at N = 16002; k_steps_resident above.
+constexpr int kExactMaxPerCu = 64;
 constexpr int kResMaxNbrs = 64;           // tiles one tile exchanges rows with (one wave)
 constexpr int kResAutoMinSteps = 4;       // AUTO contexts: shorter calls replay stage graphs
 

@@ -1082,7 +1082,7 @@ int swe_hip_create_ex(const swe_hip_static *s, const swe_hip_options *o, swe_hip
         rc = build_tiles(c, c->tile_nodes, 4 * c->tile_nodes);
     }
     if (!rc && c->kernel == SWE_HIP_KERNEL_RESIDENT) {
-        if (!exact(c)) {
+        if (!exact(c) || (!fp32 && c->n <= kExactMaxPerCu * c->ncu)) {
             std::string why;
             std::vector<std::vector<int>> reads;
             if (c->nnbr != 31 || (!c->res_auto && c->n > 32 * kResMaxWaves * c->ncu))

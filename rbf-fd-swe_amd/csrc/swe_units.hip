@@ -26,11 +26,12 @@ struct Tables {
     }
 };
 
-// Place of (node of the unit, slot) in a unit's 512 row numbers: FP64 [group of
-// 4 nodes][slot & 3][node][slot / 4], FP32 [slot / 8][node][slot & 7].
-int prec_at(bool fp32, int m, int slot)
+// Place of (node of the unit, slot) in a unit's 512 row numbers: for the FP64
+// matrix instructions [group of 4 nodes][slot & 3][node][slot / 4], by node
+// (FP32, exact) [slot / 8][node][slot & 7].
+int prec_at(bool by_node, int m, int slot)
 {
-    return fp32 ? (slot >> 3) * 128 + m * 8 + (slot & 7)
+    return by_node ? (slot >> 3) * 128 + m * 8 + (slot & 7)
                 : (m >> 2) * 128 + ((slot & 3) * 4 + (m & 3)) * 8 + (slot >> 2);
 }
 
@@ -113,7 +114,7 @@ static int build(swe_hip_ctx *c, std::vector<std::vector<int>> *nbr_tiles, std::
 {
     const int n = c->n, W = c->nnbr;
     SweUnits &u = c->units;
-    const bool ensemble = c->B > 1;
+    const bool ensemble = c->B > 1, by_node = c->fp32 || exact(c);
     // ensembles: items of 16 members on tiles of 32 nodes, or 8 on 64
     u.halves = c->B > 8 ? 2 : 1;
     const int tmax = ensemble ? kEnsNodes / u.halves : std::max(16, (n + c->ncu - 1) / c->ncu);
@@ -169,7 +170,7 @@ static int build(swe_hip_ctx *c, std::vector<std::vector<int>> *nbr_tiles, std::
                 const int m = i - tstart[t];
                 unsigned short *p = &prec[(size_t)(unit_start[t] + m / 16) * 512];
                 for (int slot = 0; slot < W; ++slot)
-                    p[prec_at(c->fp32, m & 15, slot)] =
+                    p[prec_at(by_node, m & 15, slot)] =
                         (unsigned short)where[inv[nbr[(size_t)slot * n + perm[i]]]];
             }
         }
@@ -184,7 +185,7 @@ static int build(swe_hip_ctx *c, std::vector<std::vector<int>> *nbr_tiles, std::
     for (int t = 0; t < nt; ++t)
         ulist.insert(ulist.end(), list[t].begin(), list[t].end());
     // FP64 slots past the stencil read the zero row after the last
-    if (!c->fp32)
+    if (!by_node)
         for (int k = 0; k < units; ++k)
             for (int slot = W; slot < 32; ++slot)
                 for (int m = 0; m < 16; ++m)
@@ -193,11 +194,13 @@ static int build(swe_hip_ctx *c, std::vector<std::vector<int>> *nbr_tiles, std::
     u.ntiles = nt;
     u.units = (tmax + 15) / 16;
     u.rows = rows;
-    u.waves = std::min(8, std::max(4, u.units));
+    // a wave takes whole units, in exact mode one group of 4 nodes
+    u.waves = exact(c) ? std::max(4, (tmax + 3) / 4) : std::min(8, std::max(4, u.units));
     if (ensemble)
         for (int &q : ulist)
             q = perm[q];   // rows by device node: stages exchange the state itself
-    if (!(ensemble ? ensemble_plan(u) : c->fp32 ? units_plan32(u) : units_plan64(u))
+    if (!(ensemble ? ensemble_plan(u)
+          : exact(c) ? units_plan_exact(u) : c->fp32 ? units_plan32(u) : units_plan64(u))
         || rows > 65534) {
         *err = "unit kernel: a tile's rows do not fit the LDS";
         return SWE_HIP_EINVAL;
@@ -230,7 +233,7 @@ static int build(swe_hip_ctx *c, std::vector<std::vector<int>> *nbr_tiles, std::
     u.d_own_row = ints(5);
     u.d_perm = ints(6);
     u.d_unit_tile = ints(7);
-    if (!rc) {
+    if (!rc && !exact(c)) {   // the exact kernel reads the mesh itself
         rc = ensemble ? ensemble_pack(c, units)
                       : c->fp32 ? units_pack32(c, units) : units_pack64(c, units);
         if (rc)
@@ -271,7 +274,8 @@ int units_prepare(swe_hip_ctx *c, std::string *err)
 {
     if (c->B > 1)
         return ensemble_prepare(c, err);
-    void *fn = c->fp32 ? units_kernel32(c->units) : units_kernel64(c->units);
+    void *fn = exact(c) ? units_kernel_exact()
+               : c->fp32 ? units_kernel32(c->units) : units_kernel64(c->units);
     int per_cu = 0;
     if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, kUnitsMaxLds)
             != hipSuccess
@@ -286,7 +290,8 @@ int units_prepare(swe_hip_ctx *c, std::string *err)
 
 hipError_t units_launch(swe_hip_ctx *c, int nsteps, const DevResSync &y)
 {
-    return c->fp32 ? units_launch32(c, nsteps, y) : units_launch64(c, nsteps, y);
+    return exact(c) ? units_launch_exact(c, nsteps, y)
+           : c->fp32 ? units_launch32(c, nsteps, y) : units_launch64(c, nsteps, y);
 }
 
 }  // namespace swe

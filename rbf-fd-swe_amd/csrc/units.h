@@ -41,6 +41,9 @@ bool units_plan32(SweUnits &u);
 // Kernel of a plan, its record packing and its launch.
 void *units_kernel64(const SweUnits &u);
 void *units_kernel32(const SweUnits &u);
+bool units_plan_exact(SweUnits &u);
+void *units_kernel_exact();
+hipError_t units_launch_exact(swe_hip_ctx *c, int nsteps, const DevResSync &y);
 void pack_weights64(swe_hip_ctx *c, int units);
 int units_pack64(swe_hip_ctx *c, int units);
 // The same for the ensemble stage kernel (k_ensemble.hip).

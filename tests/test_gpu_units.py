@@ -69,6 +69,19 @@ def test_fp32_auto_bitwise_vs_stage_kernel(pkg, tmp_path, n, kernel):
     assert np.array_equal(got, want)
 
 
+@pytest.mark.parametrize("n,order", [(1000, "host"), (4097, "morton"), (16384, "host"),
+                                     (16385, "host")])
+def test_exact_auto_bitwise_vs_pair(pkg, tmp_path, n, order):
+    """k_steps_exact up to 64 nodes per compute unit, k_steps_resident above."""
+    prob = _sphere(pkg, tmp_path, n)
+    print(f"case: exact N={n} order={order}, calls of 5, 1 and 4 steps", flush=True)
+    want = _run(pkg, prob, [10], kernel="pair", exact=True)
+    got = _run(pkg, prob, [5, 1, 4], exact=True, order=order,
+               slot_block=16 if order == "morton" else 0)
+    assert np.isfinite(want).all() and not np.array_equal(want, prob.H_init)
+    assert np.array_equal(got, want)
+
+
 def test_auto_calls_of_one_step_above_the_register_size(pkg, tmp_path):
     """Above 256 nodes per compute unit every call length runs the same sums."""
     prob = _sphere(pkg, tmp_path, 70001, fp32=True)
