@@ -15,9 +15,9 @@
 // vector issue per slot and 32 nodes) the matrix cores need 16 per 4 slots
 // and 4 nodes and leave the vector unit to addresses and the RHS.
 //
-// The data.  One workgroup per compute unit and tile, at most 8 waves (two per
-// SIMD, 256 registers): every wave keeps R units' weights (64 registers each)
-// for the whole launch; what the registers do not hold is read again every
+// The data.  One workgroup per compute unit and tile, 4 to 12 waves (streaming:
+// 8, two per SIMD with 256 registers): every wave keeps R units' weights (64
+// registers each) for the whole launch; what the registers do not hold is read again every
 // stage, RING 16-byte loads per lane in flight (nothing beyond the L2 moves
 // faster than 7.0 TB/s here, last-level cache or HBM, so a stage costs what it
 // re-reads).  Rows, positions, H, D and geometry sit in LDS as far as it goes.
@@ -25,8 +25,9 @@
 //
 // us per RK stage over 100 to 30 steps, against the pair-mapped resident
 // kernel up to 65536 nodes and k_stage_pair above:
-//   N = 10242    2.69 against 3.39   exchange latency
-//   N = 40962    3.7  against 4.35   exchange latency; 0.6 us of LDS conflicts
+//   N = 2562     2.15 against 3.3    exchange latency
+//   N = 10242    2.64 against 3.39   exchange latency
+//   N = 40962    3.66 against 4.35   exchange latency; 0.6 us of LDS conflicts
 //   N = 163842   19.4 against 32.6   111 MB re-read (16 of 41 units per tile stay)
 //   N = 302762   70   against 96
 //   N = 655362   170  against 197    1.37 KB per node and stage, 5.3 TB/s (180
@@ -58,17 +59,22 @@ struct UnitGeo {
     double ghm;
 };
 
-template <int R, int MODE>
-__global__ __launch_bounds__(512) void k_steps_units(DevUnits64 p)
+// G groups of 4 nodes per wave and pass (4 a whole unit; fewer on small tiles,
+// RESIDENT only): lane rows 0 .. G - 1 hold nodes after the transpose.
+template <int R, int MODE, int G>
+__global__ __launch_bounds__(MODE == UM_RESIDENT && R == 1 ? 64 * units_waves(G) : 512)
+void k_steps_units(DevUnits64 p)
 {
     constexpr bool STREAM = MODE != UM_RESIDENT;
+    static_assert(G == 4 || !STREAM, "whole units stream");
+    constexpr int N = 4 * G;   // nodes per pass
     constexpr int RING = MODE == UM_GLOBAL ? 16 : 8;   // streamed loads in flight per lane
     extern __shared__ double2 lds[];
     const int tile = (int)blockIdx.x;
     const int t0 = p.tile_start[tile];
     const int tcount = p.tile_start[tile + 1] - t0;
     const int ug = p.unit_start[tile];
-    const int nu = p.unit_start[tile + 1] - ug;
+    const int nu = (tcount + N - 1) / N;
     const int u0 = p.ustart[tile];
     const int ucount = p.ustart[tile + 1] - u0;
     const int tid = (int)threadIdx.x;
@@ -89,22 +95,25 @@ __global__ __launch_bounds__(512) void k_steps_units(DevUnits64 p)
     if constexpr (MODE != UM_GLOBAL)
         for (int i = tid; i < ucount; i += (int)blockDim.x)
             ids[i] = ulist[i];
-    for (int i = tid; i < 64 * (nu < p.lds_pos ? nu : p.lds_pos); i += (int)blockDim.x)
+    const int n16 = p.unit_start[tile + 1] - ug;
+    for (int i = tid; i < 64 * (n16 < p.lds_pos ? n16 : p.lds_pos); i += (int)blockDim.x)
         pos[i] = p.prec[64L * ug + i];
-    for (int i = tid; i < kUnitGeo * (nu < p.lds_geo ? nu : p.lds_geo); i += (int)blockDim.x)
+    for (int i = tid; i < kUnitGeo * (n16 < p.lds_geo ? n16 : p.lds_geo); i += (int)blockDim.x)
         gl[i] = p.grec[(long)kUnitGeo * ug + i];
     if (tid < 2)
         lds[2 * p.lds_rows + tid] = make_double2(0.0, 0.0);
 
-    auto geo_of = [&](const double2 *g) {
+    // geometry of the unit at g; l = this lane's place in it
+    auto geo_of = [&](const double2 *g, int l) {
         UnitGeo r;
-        r.a = g[lane];
-        r.b = g[64 + lane];
-        r.ghm = reinterpret_cast<const double *>(g + 128)[lane >> 2];
+        r.a = g[l];
+        r.b = g[64 + l];
+        r.ghm = reinterpret_cast<const double *>(g + 128)[l >> 2];
         return r;
     };
-    const int first = t0 + (lane >> 2);   // + 16 u: this lane's node of unit u
-    double2 w[R][16];
+    const int first = t0 + (lane >> 2);   // + N u: this lane's node of pass u
+    auto mine = [&](int u) { return lane < 16 * G && N * u + (lane >> 2) < tcount; };
+    double2 w[R][4 * G];
     UnitGeo gr[STREAM ? 1 : R];
     double H[R], D[R];
     static_for<R>([&](auto rc) {
@@ -112,17 +121,21 @@ __global__ __launch_bounds__(512) void k_steps_units(DevUnits64 p)
         const int u = wv + r * nw;
         H[r] = D[r] = 0.0;
         if (u < nu) {
-            const double2 *wp = p.wrec + (long)(ug + u) * 1024 + lane;
+            // the record's next group is 256 on, across units too
+            const double2 *wp = p.wrec + (long)ug * 1024 + 256L * G * u + lane;
 #pragma unroll
-            for (int q = 0; q < 16; ++q)
+            for (int q = 0; q < 4 * G; ++q)
                 w[r][q] = wp[64 * q];
-            if constexpr (!STREAM)
-                gr[r] = geo_of(p.grec + (long)kUnitGeo * (ug + u));
-            if (16 * u + (lane >> 2) < tcount)
-                H[r] = p.H[4L * p.perm[first + 16 * u] + j];
+            if constexpr (!STREAM) {
+                const int l = 16 * G * u + lane;   // past the tile's units: any record
+                gr[r] = geo_of(p.grec + (long)kUnitGeo * (ug + (l >> 6 < n16 ? l >> 6 : 0)),
+                               l & 63);
+            }
+            if (mine(u))
+                H[r] = p.H[4L * p.perm[first + N * u] + j];
         } else {
 #pragma unroll
-            for (int q = 0; q < 16; ++q)
+            for (int q = 0; q < 4 * G; ++q)
                 w[r][q] = make_double2(0.0, 0.0);
         }
     });
@@ -132,14 +145,14 @@ __global__ __launch_bounds__(512) void k_steps_units(DevUnits64 p)
     if constexpr (STREAM) {
         for (int u = wv + R * nw; u < nu; u += nw) {
             double h = 0.0;
-            if (16 * u + (lane >> 2) < tcount)
-                h = p.H[4L * p.perm[first + 16 * u] + j];
+            if (mine(u))
+                h = p.H[4L * p.perm[first + N * u] + j];
             if constexpr (MODE == UM_STREAM)
                 hd[64 * (u - R * nw) + lane] = make_double2(h, 0.0);
-            else if (16 * u + (lane >> 2) < tcount)
+            else if (mine(u))
                 __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, h),
                                                       state_rsrc(p.X0, p.bytes),
-                                                      8 * (4 * t0 + 64 * u + lane), 0, kSc1);
+                                                      8 * (4 * t0 + 4 * N * u + lane), 0, kSc1);
         }
         const int u = wv + R * nw;
         if (u < nu) {
@@ -178,8 +191,8 @@ __global__ __launch_bounds__(512) void k_steps_units(DevUnits64 p)
         swap_rows32(x1, x3);
         swap_rows16(x0, x1);
         swap_rows16(x2, x3);
-        // x0..x3: Dx, Dy, Dz, L sums of variable j of node 16 u + lane / 4
-        const double2 *own = lds + 2 * (own0 + 16 * u + (lane >> 2));
+        // x0..x3: Dx, Dy, Dz, L sums of variable j of node N u + lane / 4
+        const double2 *own = lds + 2 * (own0 + N * u + (lane >> 2));
         const double2 uv = own[0], wh = own[1];
         const bool k3 = j == 3;
         const double s1 = j == 0 ? wh.x : (j == 1 ? uv.x : uv.y);
@@ -240,9 +253,9 @@ __global__ __launch_bounds__(512) void k_steps_units(DevUnits64 p)
                     const double d = axpy<false>(Dv, p.dcoef[3], F);
                     K = Hv = axpy<false>(Hv, p.c[3], d);
                 }
-                if (16 * u + (lane >> 2) < tcount) {
-                    const int e = last ? 4 * p.perm[first + 16 * u] + j
-                                       : 4 * t0 + 64 * u + lane;
+                if (mine(u)) {
+                    const int e = last ? 4 * p.perm[first + N * u] + j
+                                       : 4 * t0 + 4 * N * u + lane;
                     __builtin_amdgcn_raw_buffer_store_b64(
                         __builtin_bit_cast(u32x2, K), state_rsrc(last ? p.H : out, p.bytes),
                         8 * e, 0, kSc1);
@@ -256,13 +269,13 @@ __global__ __launch_bounds__(512) void k_steps_units(DevUnits64 p)
                     if constexpr (!STREAM)
                         g = gr[r];
                     else if (MODE == UM_STREAM && u < p.lds_geo)
-                        g = geo_of(gl + kUnitGeo * u);
+                        g = geo_of(gl + kUnitGeo * u, lane);
                     else
-                        g = geo_of(p.grec + (long)kUnitGeo * (ug + u));
-                    double acc[4];
-                    const uint4 *pu = pos + 64 * u + (lane >> 2);
+                        g = geo_of(p.grec + (long)kUnitGeo * (ug + u), lane);
+                    double acc[4] = {0.0, 0.0, 0.0, 0.0};
+                    const uint4 *pu = pos + 16 * G * u + (lane >> 2);
 #pragma unroll
-                    for (int q = 0; q < 4; ++q)
+                    for (int q = 0; q < G; ++q)
                         acc[q] = group(w[r] + 4 * q, pu[16 * q]);
                     update(u, rhs(u, acc, g), H[r], D[r]);
                 }
@@ -278,14 +291,14 @@ __global__ __launch_bounds__(512) void k_steps_units(DevUnits64 p)
                     double2 hv;
                     if constexpr (MODE == UM_STREAM) {
                         if (u < p.lds_geo)
-                            g = geo_of(gl + kUnitGeo * u);
+                            g = geo_of(gl + kUnitGeo * u, lane);
                         else
-                            g = geo_of(p.grec + (long)kUnitGeo * (ug + u));
+                            g = geo_of(p.grec + (long)kUnitGeo * (ug + u), lane);
 #pragma unroll
                         for (int q = 0; q < 4; ++q)
                             pv[q] = pos[64 * u + 16 * q + (lane >> 2)];
                     } else {
-                        g = geo_of(p.grec + (long)kUnitGeo * (ug + u));
+                        g = geo_of(p.grec + (long)kUnitGeo * (ug + u), lane);
                         // stage 0 gathers H: it is in the own row
                         if constexpr (s == 0) {
                             hv.x = *reinterpret_cast<const double *>(
@@ -294,7 +307,7 @@ __global__ __launch_bounds__(512) void k_steps_units(DevUnits64 p)
                             hv.x = __builtin_bit_cast(
                                 double, __builtin_amdgcn_raw_buffer_load_b64(
                                             state_rsrc(p.X0, p.bytes),
-                                            8 * (4 * t0 + 64 * u + lane), 0, kSc1));
+                                            8 * (4 * t0 + 4 * N * u + lane), 0, kSc1));
                             hv.y = d_mem[64L * u];
                         }
 #pragma unroll
@@ -306,12 +319,12 @@ __global__ __launch_bounds__(512) void k_steps_units(DevUnits64 p)
                     double acc[4];
 #pragma unroll
                     for (int q = 0; q < 4; ++q) {
-                        constexpr int G = RING / 4;   // groups in flight
-                        acc[q] = group(ring + 4 * (q % G), pv[q]);
+                        constexpr int AHEAD = RING / 4;   // groups in flight
+                        acc[q] = group(ring + 4 * (q % AHEAD), pv[q]);
 #pragma unroll
                         for (int i = 0; i < 4; ++i)
-                            ring[4 * (q % G) + i] = q + G < 4 ? wc[64 * (4 * (q + G) + i)]
-                                                              : wn[64 * (4 * (q + G - 4) + i)];
+                            ring[4 * (q % AHEAD) + i] = q + AHEAD < 4 ? wc[64 * (4 * (q + AHEAD) + i)]
+                                                              : wn[64 * (4 * (q + AHEAD - 4) + i)];
                     }
                     if constexpr (MODE == UM_STREAM)
                         hv = hd[64 * (u - R * nw) + lane];
@@ -377,11 +390,23 @@ void pack_weights64(swe_hip_ctx *c, int units)
                                                   static_cast<double2 *>(u.d_wrec));
 }
 
+// All weights resident: one pass of 1, 2 or 4 groups per wave, the fewest that
+// leave one wave per SIMD (what a wave does in a stage is a chain of latencies,
+// 1820 cycles for 4 groups alone: N = 2562 2.15 against 2.51 us per stage, 7292
+// 2.33 against 2.57; with more waves of fewer groups the RHS, which costs a
+// wave the same for 4 nodes as for 16, is what is issued: N = 16002 2.90 on 16
+// waves against 2.71 on 4), on at most 12 waves (40962 3.66 against 3.78 with
+// two passes on 8), else two passes of a unit on 8.
 bool units_plan64(SweUnits &u)
 {
-    const int kept = 2 * u.waves;   // units whose weights two waves per SIMD can hold
+    const int groups = (u.nodes + 3) / 4;
+    u.groups = groups <= 4 ? 1 : groups <= 8 ? 2 : 4;
+    u.waves = std::max(4, (groups + u.groups - 1) / u.groups);
+    if (u.waves > units_waves(u.groups))
+        u.waves = 8;
+    const int kept = u.waves > 8 ? u.waves : 2 * u.waves;
     long lds = 32L * (u.rows + 1);
-    if (u.units <= kept) {
+    if (u.groups < 4 || u.units <= kept) {
         u.mode = UM_RESIDENT;
         u.pos = u.units;
         lds += 1024L * u.pos + 4L * u.rows;
@@ -403,12 +428,16 @@ bool units_plan64(SweUnits &u)
 void *units_kernel64(const SweUnits &u)
 {
     switch (u.mode) {
-    case UM_STREAM: return reinterpret_cast<void *>(&k_steps_units<2, UM_STREAM>);
-    case UM_GLOBAL: return reinterpret_cast<void *>(&k_steps_units<1, UM_GLOBAL>);
-    default:
-        return u.units > u.waves ? reinterpret_cast<void *>(&k_steps_units<2, UM_RESIDENT>)
-                                 : reinterpret_cast<void *>(&k_steps_units<1, UM_RESIDENT>);
+    case UM_STREAM: return reinterpret_cast<void *>(&k_steps_units<2, UM_STREAM, 4>);
+    case UM_GLOBAL: return reinterpret_cast<void *>(&k_steps_units<1, UM_GLOBAL, 4>);
+    default: break;
     }
+    if (u.groups == 1)
+        return reinterpret_cast<void *>(&k_steps_units<1, UM_RESIDENT, 1>);
+    if (u.groups == 2)
+        return reinterpret_cast<void *>(&k_steps_units<1, UM_RESIDENT, 2>);
+    return u.units > u.waves ? reinterpret_cast<void *>(&k_steps_units<2, UM_RESIDENT, 4>)
+                             : reinterpret_cast<void *>(&k_steps_units<1, UM_RESIDENT, 4>);
 }
 
 int units_pack64(swe_hip_ctx *c, int units)

@@ -12,8 +12,9 @@
 //
 // us per RK stage over 100 to 30 steps, against one lane per node resident up
 // to 65536 nodes and the stage kernels above:
-//   N = 2562     2.45 against 3.04   exchange latency
-//   N = 40962    3.25 against 3.25   exchange latency
+//   N = 2562     2.35 against 3.04   exchange latency
+//   N = 40962    3.13 against 3.25   exchange latency (a unit per wave on 11
+//                                    waves; 3.25 with two passes on 8)
 //   N = 163842   7.5  against 19.7   9 of 41 units per tile re-read, from L2
 //   N = 655362   78   against 110    128 of 160 re-read
 #include "units.h"
@@ -51,7 +52,7 @@ __device__ __forceinline__ float quad_bcast32(float v)
 }
 
 template <int R, int MODE, int CHAINS>
-__global__ __launch_bounds__(512) void k_steps_units32(DevUnits32 p)
+__global__ __launch_bounds__(MODE == UM_RESIDENT ? 1024 : 512) void k_steps_units32(DevUnits32 p)
 {
     constexpr bool STREAM = MODE != UM_RESIDENT;
     extern __shared__ float4 lds32[];
@@ -340,9 +341,11 @@ constexpr int kUnits32Kept = 4;   // resident units per wave of the streaming mo
 
 bool units_plan32(SweUnits &u)
 {
-    const int kept = kUnits32Kept * u.waves;
+    // up to 16 units one per wave (74 registers), else kUnits32Kept on 8 waves
+    const int kept = kUnits32Kept * 8;
     long lds = 16L * u.rows;
-    if (u.units <= 2 * u.waves) {
+    u.waves = u.units <= 16 ? std::max(4, u.units) : 8;
+    if (u.units <= u.waves) {
         u.mode = UM_RESIDENT;
         u.pos = u.units;
         lds += 1024L * u.pos + 4L * u.rows;
@@ -376,8 +379,7 @@ void *units_kernel32(const SweUnits &u)
 {
     if (u.mode != UM_RESIDENT)
         return u.chains == 2 ? streaming32<2>(u) : streaming32<1>(u);
-    return u.units > u.waves ? reinterpret_cast<void *>(&k_steps_units32<2, UM_RESIDENT, 1>)
-                             : reinterpret_cast<void *>(&k_steps_units32<1, UM_RESIDENT, 1>);
+    return reinterpret_cast<void *>(&k_steps_units32<1, UM_RESIDENT, 1>);
 }
 
 int units_pack32(swe_hip_ctx *c, int units)

@@ -100,9 +100,10 @@ struct SweTiles {
 // consecutive nodes along a space-filling curve, cut into units of 16.
 struct SweUnits {
     int ntiles = 0;               // 0: not built
-    int units = 0, rows = 0;      // most units and rows of one tile
+    int nodes = 0, units = 0, rows = 0;   // most nodes, units and rows of one tile
     int waves = 0, lds = 0;       // waves per workgroup, dynamic LDS bytes
     int mode = 0;                 // UnitMode (units.h)
+    int groups = 4;               // FP64: 4-node groups per wave and pass
     int halves = 0;               // ensembles: 8-member halves of an item
     int chains = 1;               // FP32: partial sums per stencil sum, as split32's lanes
     int pos = 0, geo = 0;         // units whose positions, geometry the LDS holds

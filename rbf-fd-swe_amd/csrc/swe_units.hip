@@ -192,10 +192,11 @@ static int build(swe_hip_ctx *c, std::vector<std::vector<int>> *nbr_tiles, std::
                     prec[(size_t)k * 512 + prec_at(false, m, slot)] = (unsigned short)rows;
     u.chains = c->fp32 && c->split32 == 2 ? 2 : 1;
     u.ntiles = nt;
-    u.units = (tmax + 15) / 16;
+    u.nodes = std::min(n, tmax);
+    u.units = (u.nodes + 15) / 16;
     u.rows = rows;
-    // a wave takes whole units, in exact mode one group of 4 nodes
-    u.waves = exact(c) ? std::max(4, (tmax + 3) / 4) : std::min(8, std::max(4, u.units));
+    // exact mode: a group of 4 nodes per wave; else the plan's
+    u.waves = exact(c) ? std::max(4, (tmax + 3) / 4) : 0;
     if (ensemble)
         for (int &q : ulist)
             q = perm[q];   // rows by device node: stages exchange the state itself

@@ -18,6 +18,10 @@ enum UnitMode {
     UM_GLOBAL      // the same with those units' positions, H and D in memory
 };
 
+// Most waves per workgroup with G groups of 4 nodes resident on each (FP64: 136
+// registers for 4).
+constexpr int units_waves(int G) { return G < 4 ? 4 : 12; }
+
 struct DevUnits {
     DevResSync y;
     const int *tile_start;      // [ntiles + 1] first node (kernel order)

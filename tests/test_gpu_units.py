@@ -2,8 +2,8 @@
 contexts run in fast mode, against the stage kernels: bitwise equal, because
 the FP64 and FP32 matrix instructions round every product-sum like the
 fused multiply-add they replace and the sums keep their order.  Sizes on both
-sides of every change of plan: one 16-node unit per tile, one and two
-resident units per wave, the first mesh whose units stream their weights
+sides of every change of plan: one, two and four 4-node groups per wave, one
+and two resident units per wave, the first mesh whose units stream their weights
 (LDS tables, then tables in memory), a last tile with a ragged unit, padded
 nodes outside every stencil."""
 import numpy as np
@@ -43,8 +43,9 @@ def _run(pkg, prob, calls, **kw):
         return ctx.get_state()
 
 
-@pytest.mark.parametrize("n,order", [(1000, "host"), (4100, "morton"), (32768, "host"),
-                                     (32769, "host"), (65536, "hilbert"), (65537, "host"),
+@pytest.mark.parametrize("n,order", [(1000, "host"), (4100, "morton"), (8192, "host"),
+                                     (8193, "host"), (32769, "host"), (49152, "hilbert"),
+                                     (49153, "host"), (65536, "hilbert"), (65537, "host"),
                                      (120001, "morton"), (300001, "host")])
 def test_fp64_auto_bitwise_vs_pair(pkg, tmp_path, n, order):
     prob = _sphere(pkg, tmp_path, n)
