@@ -20,7 +20,9 @@
 // registers each) for the whole launch; what the registers do not hold is read again every
 // stage, RING 16-byte loads per lane in flight (nothing beyond the L2 moves
 // faster than 7.0 TB/s here, last-level cache or HBM, so a stage costs what it
-// re-reads).  Rows, positions, H, D and geometry sit in LDS as far as it goes.
+// re-reads).  UM_GLOBAL loads the weights non-temporally: the rest, 330 bytes a
+// node, then stays in the last-level cache (N = 655362 170 -> 133 us per stage;
+// geometry non-temporal too: 144; UM_STREAM: no change).  Rows, positions, H, D and geometry sit in LDS as far as it goes.
 // Every wave's rows of a tile are copied once per stage (res_sync.h).
 //
 // us per RK stage over 100 to 30 steps, against the pair-mapped resident
@@ -29,9 +31,8 @@
 //   N = 10242    2.64 against 3.39   exchange latency
 //   N = 40962    3.66 against 4.35   exchange latency; 0.6 us of LDS conflicts
 //   N = 163842   19.4 against 32.6   111 MB re-read (16 of 41 units per tile stay)
-//   N = 302762   70   against 96
-//   N = 655362   170  against 197    1.37 KB per node and stage, 5.3 TB/s (180
-//                                    with H kept beside D instead of in X0)
+//   N = 302762   59   against 96
+//   N = 655362   133  against 197    1.30 KB per node and stage at 6.4 TB/s
 #include "units.h"
 
 #include <algorithm>
@@ -323,8 +324,13 @@ void k_steps_units(DevUnits64 p)
                         acc[q] = group(ring + 4 * (q % AHEAD), pv[q]);
 #pragma unroll
                         for (int i = 0; i < 4; ++i)
-                            ring[4 * (q % AHEAD) + i] = q + AHEAD < 4 ? wc[64 * (4 * (q + AHEAD) + i)]
-                                                              : wn[64 * (4 * (q + AHEAD - 4) + i)];
+{
+                            const double2 *from = q + AHEAD < 4
+                                                      ? wc + 64 * (4 * (q + AHEAD) + i)
+                                                      : wn + 64 * (4 * (q + AHEAD - 4) + i);
+                            ring[4 * (q % AHEAD) + i] =
+                                MODE == UM_GLOBAL ? load_nt(from) : *from;
+                        }
                     }
                     if constexpr (MODE == UM_STREAM)
                         hv = hd[64 * (u - R * nw) + lane];

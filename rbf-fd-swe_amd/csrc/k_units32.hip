@@ -16,7 +16,7 @@
 //   N = 40962    3.13 against 3.25   exchange latency (a unit per wave on 11
 //                                    waves; 3.25 with two passes on 8)
 //   N = 163842   7.5  against 19.7   9 of 41 units per tile re-read, from L2
-//   N = 655362   78   against 110    128 of 160 re-read
+//   N = 655362   69   against 110    128 of 160 re-read
 #include "units.h"
 
 #include <algorithm>
@@ -51,7 +51,7 @@ __device__ __forceinline__ float quad_bcast32(float v)
     return dpp32<K * 0x55>(v);
 }
 
-template <int R, int MODE, int CHAINS>
+template <int R, int MODE, int CHAINS, bool NT = false>
 __global__ __launch_bounds__(MODE == UM_RESIDENT ? 1024 : 512) void k_steps_units32(DevUnits32 p)
 {
     constexpr bool STREAM = MODE != UM_RESIDENT;
@@ -284,13 +284,13 @@ __global__ __launch_bounds__(MODE == UM_RESIDENT ? 1024 : 512) void k_steps_unit
                     Acc acc = {};
                     const float4 g = ring[8];
                     const float ghm = ring[7].w;
-                    ring[8] = wn[64 * 8];
+                    ring[8] = NT ? load_nt(wn + 64 * 8) : wn[64 * 8];
 #pragma unroll
                     for (int q = 0; q < 8; ++q) {
                         const uint4 v = pv[q >> 1];
                         acc = (q & 1) ? quarter(acc, q, ring[q], v.z, v.w)
                                       : quarter(acc, q, ring[q], v.x, v.y);
-                        ring[q] = wn[64 * q];
+                        ring[q] = NT ? load_nt(wn + 64 * q) : wn[64 * q];
                     }
                     if constexpr (MODE == UM_STREAM)
                         hv = hd[64 * (u - R * nw) + lane];
@@ -359,6 +359,11 @@ bool units_plan32(SweUnits &u)
             lds += whole;
         } else {
             u.mode = UM_GLOBAL;
+            // past the 256 MB last-level cache the records are better not kept
+            // there at all (N = 605162: 62.2 against 65.7 us per stage, 655362
+            // 69 against 77); while they fit they are (576002: 55.5 against
+            // 58.9, 349692 27.8 against 34.2)
+            u.stream_nt = 1024L * kRec32 * (u.units - kept) * u.ntiles > (256L << 20);
             u.pos = u.geo = kept;
             lds += 2048L * kept;
         }
@@ -370,6 +375,8 @@ bool units_plan32(SweUnits &u)
 template <int CHAINS>
 static void *streaming32(const SweUnits &u)
 {
+    if (u.mode == UM_GLOBAL && u.stream_nt)
+        return reinterpret_cast<void *>(&k_steps_units32<kUnits32Kept, UM_GLOBAL, CHAINS, true>);
     return u.mode == UM_STREAM
                ? reinterpret_cast<void *>(&k_steps_units32<kUnits32Kept, UM_STREAM, CHAINS>)
                : reinterpret_cast<void *>(&k_steps_units32<kUnits32Kept, UM_GLOBAL, CHAINS>);

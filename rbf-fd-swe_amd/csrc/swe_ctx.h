@@ -33,8 +33,8 @@ constexpr int kUnitsMaxLds = 160 * 1024 - 64;   // dynamic LDS of k_steps_units
 // Nodes per compute unit up to which AUTO tries the streaming form of the unit
 // kernels (their own LDS check decides: ~4600 FP64 rows of 32 bytes).  Beyond
 // 256 nodes per unit it beats the stage kernels at every size measured (us per
-// stage, FP64: N = 163842 19.4 against 32.6, 655362 170 against 197; FP32: 7.5
-// against 19.7, 78 against 110).
+// stage, FP64: N = 163842 19.4 against 32.6, 655362 133 against 197; FP32: 7.5
+// against 19.7, 69 against 110).
 constexpr int kUnitsMaxPerCu = 4096;
 // Nodes per compute unit up to which exact FP64 contexts run k_steps_exact (a
 // 4-node group on each of 16 waves; 126 registers, more waves do not fit):
@@ -105,6 +105,7 @@ struct SweUnits {
     int mode = 0;                 // UnitMode (units.h)
     int groups = 4;               // FP64: 4-node groups per wave and pass
     int halves = 0;               // ensembles: 8-member halves of an item
+    bool stream_nt = false;       // FP32: streamed records bypass the last-level cache
     int chains = 1;               // FP32: partial sums per stencil sum, as split32's lanes
     int pos = 0, geo = 0;         // units whose positions, geometry the LDS holds
     long long bytes = 0;          // counted in the context's bytes too

@@ -61,4 +61,12 @@ hipError_t units_launch32(swe_hip_ctx *c, int nsteps, const DevResSync &y);
 // The table part of a launch's arguments.
 void units_tables(const swe_hip_ctx *c, int nsteps, const DevResSync &y, DevUnits *p);
 
+// A 16-byte load of data no cache needs to keep.
+template <typename T>
+__device__ __forceinline__ T load_nt(const T *p)
+{
+    static_assert(sizeof(T) == 16, "16 bytes");
+    return __builtin_bit_cast(T, __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(p)));
+}
+
 }  // namespace swe

@@ -4,7 +4,7 @@ the FP64 and FP32 matrix instructions round every product-sum like the
 fused multiply-add they replace and the sums keep their order.  Sizes on both
 sides of every change of plan: one, two and four 4-node groups per wave, one
 and two resident units per wave, the first mesh whose units stream their weights
-(LDS tables, then tables in memory), a last tile with a ragged unit, padded
+(LDS tables, then tables in memory, then records past the last-level cache), a last tile with a ragged unit, padded
 nodes outside every stencil."""
 import numpy as np
 import pytest
@@ -58,7 +58,7 @@ def test_fp64_auto_bitwise_vs_pair(pkg, tmp_path, n, order):
 
 @pytest.mark.parametrize("n,kernel", [(1000, "lane"), (32769, "lane"), (65536, "lane"),
                                       (65537, "pair"), (120001, "pair"), (262144, "pair"),
-                                      (300001, "lane")])
+                                      (300001, "lane"), (400001, "lane"), (620001, "lane")])
 def test_fp32_auto_bitwise_vs_stage_kernel(pkg, tmp_path, n, kernel):
     """AUTO keeps the partial sums of the stage kernel it ran at that size:
     two per stencil sum (PAIR) from 65536 to 262144 nodes, else one (LANE)."""
