@@ -169,10 +169,30 @@ def dominant_kernel(args):
         else "k_stage_members"
 
 
-RESIDENT_NOTE = ("k_steps_resident runs every stage of a call in one launch: 'launch' here is "
+# Fast mode with 31-point stencils: the matrix-core kernels that run what the
+# options above select, as far as they reach.
+UNIT_KERNELS = {"k_steps_resident": "k_steps_units", "k_steps_resident32": "k_steps_units32",
+                "k_stage_tspec": "k_stage_ensemble"}
+UNITS_MAX_NODES = 4096 * 256   # 4096 nodes per compute unit
+
+
+def measured_kernel(args):
+    """Name of the kernel a run of these options spends its time in."""
+    name = dominant_kernel(args)
+    if args.exact:
+        return "k_steps_exact" if name == "k_steps_resident" and args.nodes <= 64 * 256 else name
+    if args.members == 1 and args.kernel == "auto" and args.nodes <= UNITS_MAX_NODES:
+        return "k_steps_units32" if args.fp32 else "k_steps_units"
+    if args.members > 1 and not args.fp32 and (args.tiled or args.member_block == 0):
+        return "k_stage_ensemble"
+    return UNIT_KERNELS.get(name, name)
+
+
+RESIDENT_NOTE = ("the kernel runs every stage of a call in one launch: 'launch' here is "
                  "one RK stage (launch time / 4 steps), 'achieved' the stage kernels' "
-                 "algorithmic bytes per stage over that time; the kernel reads the static "
-                 "stencil data (1252 of the 1388 B per node) once per launch, not per stage, "
+                 "algorithmic bytes per stage over that time; up to 256 nodes per compute unit "
+                 "it reads the static stencil data (1252 of the 1388 B per node) once per "
+                 "launch, beyond that the part its registers and caches do not hold, "
                  "so frac can exceed 1; its HBM traffic is 'traffic' (rocprofv3 counts)")
 
 FP64_PEAK_TFLOPS = 78.6
@@ -219,17 +239,26 @@ def leg_kernel(opts):
     return "k_stage_mpair" if opts["member_block"] == 64 else "k_stage_members"
 
 
+def tuned_kernel(opts):
+    """Short name of the kernel a tuned fast-mode option set spends its time in."""
+    if opts.get("members", 1) == 1 and opts["kernel"] == "auto":
+        return "k_steps_units"
+    if opts.get("members", 1) > 1 and opts["member_block"] == 0:
+        return "k_stage_ensemble"
+    name = leg_kernel(opts)
+    return UNIT_KERNELS.get(name, name)
+
+
 def describe(opts):
     if opts.get("members", 1) == 1:
+        if opts["kernel"] in ("auto", "resident"):
+            return "k_steps_units (matrix cores, whole steps in one cooperative launch)"
         if opts["kernel"] == "tile":
             return (f"k_stage_ptile (pair mapping over LDS tiles of {opts['tile_nodes']} nodes, "
                     f"row staging {opts['prefetch']})")
-        if opts["kernel"] == "resident":
-            return "k_steps_resident (whole steps in one cooperative launch)"
         return "k_stage_pair"
-    if opts["tiled"]:
-        return (f"k_stage_tspec (member-lane LDS tiles, {opts['tile_nodes'] or 8} nodes x "
-                f"{opts['tile_rows'] or 70} rows, loader and compute waves, direct-to-LDS loads)")
+    if opts["tiled"] or opts["member_block"] == 0:
+        return "k_stage_ensemble (matrix cores, LDS tiles of 32 nodes x 16 members)"
     if opts["member_block"] == 64:
         return "k_stage_mpair (member pairs, 16-byte gathers)"
     return f"k_stage_members (member block {opts['member_block']})"
@@ -250,7 +279,7 @@ def c3_leg(pkg, torch, steps=200):
     n = prob.n_nodes
     launch_us = ms * 1e3 / 4
     achieved = stage_bytes(prob.padded, 1) / (launch_us * 1e-6) / 1e9
-    traffic, traffic_source = stored_traffic(leg_kernel(opts), n, 1)
+    traffic, traffic_source = stored_traffic(tuned_kernel(opts), n, 1)
     return {"workload": f"N={n}, 1 member, {steps} RK4 steps, FP64, fused stages + HIP graphs",
             "kernel": describe(opts), "options": opts, "ms_per_step": ms,
             "gnode_rhs_per_s": n * 4 / (ms * 1e-3) / 1e9,
@@ -285,7 +314,7 @@ def ensemble_leg(pkg, torch, steps=500):
     flops_launch = float(N) * 64 * FLOP_PER_NODE_RHS
     achieved = bytes_launch / (launch_us * 1e-6) / 1e9
     tflops = flops_launch / (launch_us * 1e-6) / 1e12
-    traffic, traffic_source = stored_traffic(leg_kernel(opts), n, 64)
+    traffic, traffic_source = stored_traffic(tuned_kernel(opts), n, 64)
     return {"workload": f"N={n}, 64 members (seeded 1e-3 perturbations), {steps} RK4 steps, "
                         "Hilbert-ordered device copy, fused stages + HIP graphs",
             "kernel": describe(opts), "options": opts,
@@ -374,8 +403,9 @@ FP32_KERNELS = {"lane": "k_stage_lane32 (one lane per node)",
                 "quad": "k_stage_split32 (4 lanes per node split the stencil slots)",
                 "oct": "k_stage_split32 (8 lanes per node split the stencil slots)",
                 "tile": "k_stage_tile32 (one lane per node over LDS tiles of {tn} nodes)",
-                "resident": "k_steps_resident32 (whole steps in one cooperative launch, one lane "
-                            "per node)"}
+                "auto": "k_steps_units32 (matrix cores, whole steps in one cooperative launch)",
+                "resident": "k_steps_units32 (matrix cores, whole steps in one cooperative "
+                            "launch)"}
 
 
 def fp32_leg(pkg, torch, nodes, steps, warmup):
@@ -402,7 +432,7 @@ def fp32_leg(pkg, torch, nodes, steps, warmup):
                          "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS,
                          "bytes_per_launch": stage_bytes(prob.padded, 1, fp32=True),
                          "avg_launch_us": launch_us,
-                         "note": RESIDENT_NOTE if opts["kernel"] == "resident"
+                         "note": RESIDENT_NOTE if opts["kernel"] in ("auto", "resident")
                          else "one launch = one fused RK stage"},
             "state_finite": finite}
 
@@ -471,7 +501,7 @@ def main():
     # outside this process; the stored count is reported with its source and
     # only when it was taken for the kernel this run selects
     traffic, traffic_source = (None, None) if args.fp32 else \
-        stored_traffic(dominant_kernel(args), args.nodes, args.members)
+        stored_traffic(measured_kernel(args), args.nodes, args.members)
     node_rhs = float(prob.n_nodes) * 4 * args.steps * args.members
     value = node_rhs / (gpu_ms * 1e-3) / 1e9
     ctx.close()
@@ -520,7 +550,7 @@ def main():
         "dtype": "f32" if args.fp32 else "f64",
         "data": "synthetic (seeded icosahedral mesh + Gaussian RBF-FD weights, TC5-like state)",
         "config": {"workload": f"RBF-FD SWE RK4, N={prob.n_nodes} nodes, stencil 31, "
-                               f"{args.members} member(s), {dominant_kernel(args)}"
+                               f"{args.members} member(s), {measured_kernel(args)}"
                                + (" (the 40962-node, 1000-step single-member case timed "
                                   "against the reference CPU path)"
                                   if prob.n_nodes == 40962 and args.members == 1 else ""),
@@ -532,10 +562,10 @@ def main():
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
                      "traffic_source": traffic_source,
-                     "kernel": dominant_kernel(args),
+                     "kernel": measured_kernel(args),
                      "bytes_per_launch": stage_bytes(N, args.members, args.fp32),
                      "avg_launch_us": launch_s * 1e6,
-                     "note": RESIDENT_NOTE if dominant_kernel(args) == "k_steps_resident"
+                     "note": RESIDENT_NOTE if measured_kernel(args).startswith("k_steps_")
                      else "one launch = one fused RK stage"},
         "cpu_baseline": cpu,
         "cpu_baseline_sfdl": cpu_sfdl,

@@ -1304,6 +1304,12 @@ int swe_hip_tune_ex(swe_hip_ctx *base, int members, unsigned flags, int steps,
         cand.push_back(swe_hip_options{members, flags, base->dev, mb, base, kernel, prefetch, 0,
                                        tiled, 0, tn, tr});
     };
+    const bool fast31 = base->nnbr == 31 && !(flags & SWE_HIP_EXACT);
+    // above RESIDENT's sizes only AUTO reaches the streaming unit kernels
+    // (N = 655362: 133 us per stage against TILE's 168, 163842: 19 against 33)
+    if (members == 1 && fast31 && base->n > 32 * kResMaxWaves * base->ncu
+        && base->n <= (long)kUnitsMaxPerCu * base->ncu)
+        add(0, SWE_HIP_KERNEL_AUTO, 0, 0, 0, 0);
     if (base->fp32) {   // lanes per node (exact mode: one, in order) and LDS tiles
         add(0, SWE_HIP_KERNEL_LANE, 0, 0, 0, 0);
         if (!(flags & SWE_HIP_EXACT))
@@ -1327,11 +1333,15 @@ int swe_hip_tune_ex(swe_hip_ctx *base, int members, unsigned flags, int steps,
             if (members % mb)
                 continue;
             add(mb, 0, 0, 0, 0, 0);
-            if (mb == 32 && base->nnbr == 31)   // member-lane tiles: nodes x rows per tile
+            if (mb == 32 && fast31)   // the matrix-core kernel cuts tiles of its own
+                add(mb, 0, 0, 1, 8, kTmemRows);
+            else if (mb == 32 && base->nnbr == 31)   // member-lane tiles: nodes x rows per tile
                 for (int tn : {8, 6})
                     for (int tr : {kTmemRows, 56})
                         add(mb, 0, 0, 1, tn, tr);
         }
+        if (members % 32 && fast31)   // that kernel again where 32 does not divide
+            add(0, 0, 0, 0, 0, 0);    // (16 members at N = 10242: 23 against 42 us per stage)
     }
     double best_t = 1e300;
     int found = -1;

@@ -88,3 +88,21 @@ def test_auto_calls_of_one_step_above_the_register_size(pkg, tmp_path):
     prob = _sphere(pkg, tmp_path, 70001, fp32=True)
     print("case: FP32 units N=70001, calls of 1, 2 and 3 steps", flush=True)
     assert np.array_equal(_run(pkg, prob, [1, 2, 3], fp32=True), _run(pkg, prob, [6], fp32=True))
+
+
+@pytest.mark.parametrize("members", [1, 16])
+def test_tuner_choice_runs_the_same_bits(pkg, tmp_path, members):
+    """Above RESIDENT's sizes the tuner times the streaming form too, and for
+    ensembles the matrix-core kernel whatever divides the member count."""
+    prob = _sphere(pkg, tmp_path, 70001 if members == 1 else 3000)
+    print(f"case: tuner, {members} member(s), {prob.n_nodes} nodes", flush=True)
+    with pkg.runtime.HipContext(prob, kernel="pair", order="hilbert") as base:
+        opts, ms = base.tune(members, steps=3)
+        assert ms > 0 and (opts["kernel"] in ("auto", "pair", "tile"))
+        with pkg.runtime.HipContext(prob, share=base, **opts) as ctx:
+            ctx.set_state(prob.H_init, members - 1)
+            ctx.rk_steps(4)
+            got = ctx.get_state(members - 1)
+        base.set_state(prob.H_init)
+        base.rk_steps(4)
+        assert np.array_equal(got, base.get_state())
