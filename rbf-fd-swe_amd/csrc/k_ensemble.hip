@@ -139,7 +139,7 @@ __global__ __launch_bounds__(256, 2) void k_stage_ensemble(DevEnsemble p, DevSta
                 __syncthreads();   // the previous tile's LDS is free
                 if (tid < ucount)   // at most 254 rows
                     ids[tid] = p.ulist[u0 + tid];
-                // a last tile's missing units read the zero row
+                // the missing units of a last or cut tile read the zero row
                 const unsigned z = (unsigned)p.lds_rows << 16 | (unsigned)p.lds_rows;
                 if (tid < 64 * UNITS) {
                     const uint4 pr =
@@ -277,14 +277,24 @@ __global__ void k_pack_ensemble(DevMesh m, const int *tile_start, const int *uni
         node < tile_start[tile + 1] && f < GEO_N ? m.geo[(long)f * m.ld + perm[node]] : 0.0;
 }
 
+static int ensemble_lds(int halves, int rows)
+{
+    const int nodes = kEnsNodes / halves;
+    return 256 * halves * (rows + 1) + 64 * nodes + 16 * nodes * kEnsGeo + 4 * rows;
+}
+
+int ensemble_rows(int halves)
+{
+    // two workgroups per compute unit, 16-bit row offsets
+    return std::min(254, (kUnitsMaxLds / 2 - ensemble_lds(halves, 0)) / (256 * halves + 4));
+}
+
 bool ensemble_plan(SweUnits &u)
 {
     u.mode = UM_RESIDENT;
     u.waves = 4;
-    const int nodes = kEnsNodes / u.halves;
-    u.lds = 256 * u.halves * (u.rows + 1) + 64 * nodes + 16 * nodes * kEnsGeo + 4 * u.rows;
-    // two workgroups per compute unit, 16-bit row offsets
-    return 2 * u.lds <= kUnitsMaxLds && u.rows < 255;
+    u.lds = ensemble_lds(u.halves, u.rows);
+    return u.rows <= ensemble_rows(u.halves);
 }
 
 int ensemble_pack(swe_hip_ctx *c, int units)

@@ -118,7 +118,7 @@ static int build(swe_hip_ctx *c, std::vector<std::vector<int>> *nbr_tiles, std::
     // ensembles: items of 16 members on tiles of 32 nodes, or 8 on 64
     u.halves = c->B > 8 ? 2 : 1;
     const int tmax = ensemble ? kEnsNodes / u.halves : std::max(16, (n + c->ncu - 1) / c->ncu);
-    const int nt = (n + tmax - 1) / tmax;
+    int nt = (n + tmax - 1) / tmax;
     const std::vector<int> &nbr = c->mesh->h_nbr;
     // kernel order: compact tiles of compact units
     const double *xyz = c->mesh->h_xyz.data();
@@ -131,18 +131,14 @@ static int build(swe_hip_ctx *c, std::vector<std::vector<int>> *nbr_tiles, std::
     });
     for (int i = 0; i < n; ++i)
         inv[perm[i]] = i;
-    std::vector<int> tstart(nt + 1), ustart(nt + 1, 0), unit_start(nt + 1, 0), own_row(nt);
+    std::vector<int> tstart(nt + 1), ustart, unit_start, own_row;
     for (int t = 0; t <= nt; ++t)
         tstart[t] = std::min(n, t * tmax);
-    for (int t = 0; t < nt; ++t)
-        unit_start[t + 1] = unit_start[t] + (tstart[t + 1] - tstart[t] + 15) / 16;
-    const int units = unit_start[nt];
     // distinct rows of each tile (its own nodes among them), ascending
-    std::vector<std::vector<int>> list(nt);
-    std::vector<uint4> precq((size_t)units * 64);
-    unsigned short *prec = reinterpret_cast<unsigned short *>(precq.data());
-    nbr_tiles->assign(nt, {});
-    parallel_ranges(nt, 1024 / tmax, [&](int a, int b) {
+    std::vector<std::vector<int>> list;
+    std::vector<uint4> precq;
+    unsigned short *prec = nullptr;
+    auto list_rows = [&](int a, int b) {
         std::vector<int> mark(n, -1), where(n);
         for (int t = a; t < b; ++t) {
             std::vector<int> &l = list[t];
@@ -174,7 +170,35 @@ static int build(swe_hip_ctx *c, std::vector<std::vector<int>> *nbr_tiles, std::
                         (unsigned short)where[inv[nbr[(size_t)slot * n + perm[i]]]];
             }
         }
-    });
+    };
+    for (;;) {
+        nt = (int)tstart.size() - 1;
+        ustart.assign(nt + 1, 0);
+        unit_start.assign(nt + 1, 0);
+        own_row.assign(nt, 0);
+        list.assign(nt, {});
+        nbr_tiles->assign(nt, {});
+        for (int t = 0; t < nt; ++t)
+            unit_start[t + 1] = unit_start[t] + (tstart[t + 1] - tstart[t] + 15) / 16;
+        precq.assign((size_t)unit_start[nt] * 64, uint4{});
+        prec = reinterpret_cast<unsigned short *>(precq.data());
+        parallel_ranges(nt, 1024 / tmax, list_rows);
+        if (!ensemble)
+            break;
+        // a few tiles (icosahedral nodes, N = 163842: one of 5121, 146 rows) may
+        // read more rows than an item has room for: each becomes two, of whole units
+        std::vector<int> cut;
+        for (int t = 0; t < nt; ++t) {
+            cut.push_back(tstart[t]);
+            if ((int)list[t].size() > ensemble_rows(u.halves) && tstart[t + 1] - tstart[t] > 16)
+                cut.push_back(tstart[t] + 16 * ((unit_start[t + 1] - unit_start[t]) / 2));
+        }
+        if ((int)cut.size() == nt)
+            break;
+        cut.push_back(n);
+        tstart = cut;
+    }
+    const int units = unit_start[nt];
     int rows = 0;
     for (int t = 0; t < nt; ++t) {
         ustart[t + 1] = ustart[t] + (int)list[t].size();

@@ -52,6 +52,7 @@ void pack_weights64(swe_hip_ctx *c, int units);
 int units_pack64(swe_hip_ctx *c, int units);
 // The same for the ensemble stage kernel (k_ensemble.hip).
 bool ensemble_plan(SweUnits &u);
+int ensemble_rows(int halves);   // most rows of a tile
 int ensemble_pack(swe_hip_ctx *c, int units);
 int ensemble_prepare(swe_hip_ctx *c, std::string *err);
 constexpr int kEnsNodes = 64;   // nodes per tile of the ensemble kernel with items of 8 members

@@ -68,3 +68,31 @@ def test_scattered_stencils_fall_back(pkg, tmp_path):
         one.set_state(H[3])
         one.rk_steps(2)
         assert np.array_equal(ens.get_state(3), one.get_state())
+
+
+@pytest.mark.parametrize("members", [4, 16])
+def test_tiles_with_too_many_rows_are_cut(pkg, tmp_path, members):
+    """Three random neighbours per node in a part of the mesh: its tiles exceed
+    an item's rows, their halves do not, and the kernel still runs (its records
+    are in the context's bytes)."""
+    m = pkg.mesh
+    case = m.read_bin(m.case_path(2562, seed=1))
+    rng = np.random.default_rng(3)
+    some = np.flatnonzero(case.X[:, 2] > 0.8)
+    case.idx[some, 28:] = rng.integers(0, 2562, (len(some), 3))
+    path = str(tmp_path / "cut.bin")
+    m.write_bin(path, case)
+    prob = pkg.host.Problem(path, use_rcm=False, layout="cfdl")
+    print(f"case: ensemble with cut tiles, N=2562 members={members}", flush=True)
+    H = _states(prob, members, 1)
+    with pkg.runtime.HipContext(prob, kernel="pair") as one, \
+            pkg.runtime.HipContext(prob, members=members) as ens:
+        n = prob.compute_size
+        assert ens.device_bytes() > 4 * 32 * n * members + 1024 * n
+        for k in range(members):
+            ens.set_state(H[k], k)
+        ens.rk_steps(2)
+        for k in (0, members - 1):
+            one.set_state(H[k])
+            one.rk_steps(2)
+            assert np.array_equal(ens.get_state(k), one.get_state()), k
