@@ -171,8 +171,7 @@ def dominant_kernel(args):
 
 # Fast mode with 31-point stencils: the matrix-core kernels that run what the
 # options above select, as far as they reach.
-UNIT_KERNELS = {"k_steps_resident": "k_steps_units", "k_steps_resident32": "k_steps_units32",
-                "k_stage_tspec": "k_stage_ensemble"}
+UNIT_KERNELS = {"k_steps_resident": "k_steps_units", "k_steps_resident32": "k_steps_units32"}
 UNITS_MAX_NODES = 4096 * 256   # 4096 nodes per compute unit
 
 
@@ -183,9 +182,19 @@ def measured_kernel(args):
         return "k_steps_exact" if name == "k_steps_resident" and args.nodes <= 64 * 256 else name
     if args.members == 1 and args.kernel == "auto" and args.nodes <= UNITS_MAX_NODES:
         return "k_steps_units32" if args.fp32 else "k_steps_units"
-    if args.members > 1 and not args.fp32 and (args.tiled or args.member_block == 0):
-        return "k_stage_ensemble"
+    if args.members > 1:
+        return "k_stage_ensemble" if args.member_block == 0 and not args.tiled or \
+            args.tiled and ensemble_fills(args.nodes, args.members) else name
     return UNIT_KERNELS.get(name, name)
+
+
+def ensemble_fills(nodes, members):
+    """The library's rule for tiled fast-mode ensembles, on 256 compute units."""
+    halves = 2 if members > 8 else 1
+    tiles = -(-(-(-nodes // (64 // halves))) // 8)
+    nmb = -(-members // (8 * halves))
+    turns = tiles // 64 * nmb + -(-(tiles % 64 * nmb) // 64)
+    return 20 * tiles * nmb >= 19 * turns * 64
 
 
 RESIDENT_NOTE = ("the kernel runs every stage of a call in one launch: 'launch' here is "
@@ -239,17 +248,17 @@ def leg_kernel(opts):
     return "k_stage_mpair" if opts["member_block"] == 64 else "k_stage_members"
 
 
-def tuned_kernel(opts):
+def tuned_kernel(opts, nodes):
     """Short name of the kernel a tuned fast-mode option set spends its time in."""
-    if opts.get("members", 1) == 1 and opts["kernel"] == "auto":
-        return "k_steps_units"
-    if opts.get("members", 1) > 1 and opts["member_block"] == 0:
-        return "k_stage_ensemble"
     name = leg_kernel(opts)
-    return UNIT_KERNELS.get(name, name)
+    if opts.get("members", 1) == 1:
+        return "k_steps_units" if opts["kernel"] == "auto" else UNIT_KERNELS.get(name, name)
+    if opts["member_block"] == 0 or opts["tiled"] and ensemble_fills(nodes, opts["members"]):
+        return "k_stage_ensemble"
+    return name
 
 
-def describe(opts):
+def describe(opts, nodes):
     if opts.get("members", 1) == 1:
         if opts["kernel"] in ("auto", "resident"):
             return "k_steps_units (matrix cores, whole steps in one cooperative launch)"
@@ -257,8 +266,11 @@ def describe(opts):
             return (f"k_stage_ptile (pair mapping over LDS tiles of {opts['tile_nodes']} nodes, "
                     f"row staging {opts['prefetch']})")
         return "k_stage_pair"
-    if opts["tiled"] or opts["member_block"] == 0:
+    if tuned_kernel(opts, nodes) == "k_stage_ensemble":
         return "k_stage_ensemble (matrix cores, LDS tiles of 32 nodes x 16 members)"
+    if opts["tiled"]:
+        return (f"k_stage_tspec (member-lane LDS tiles, {opts['tile_nodes'] or 8} nodes x "
+                f"{opts['tile_rows'] or 70} rows, loader and compute waves, direct-to-LDS loads)")
     if opts["member_block"] == 64:
         return "k_stage_mpair (member pairs, 16-byte gathers)"
     return f"k_stage_members (member block {opts['member_block']})"
@@ -279,9 +291,9 @@ def c3_leg(pkg, torch, steps=200):
     n = prob.n_nodes
     launch_us = ms * 1e3 / 4
     achieved = stage_bytes(prob.padded, 1) / (launch_us * 1e-6) / 1e9
-    traffic, traffic_source = stored_traffic(tuned_kernel(opts), n, 1)
-    return {"workload": f"N={n}, 1 member, {steps} RK4 steps, FP64, fused stages + HIP graphs",
-            "kernel": describe(opts), "options": opts, "ms_per_step": ms,
+    traffic, traffic_source = stored_traffic(tuned_kernel(opts, n), n, 1)
+    return {"workload": f"N={n}, 1 member, {steps} RK4 steps, FP64",
+            "kernel": describe(opts, n), "options": opts, "ms_per_step": ms,
             "gnode_rhs_per_s": n * 4 / (ms * 1e-3) / 1e9,
             "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS,
                          "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS,
@@ -314,10 +326,10 @@ def ensemble_leg(pkg, torch, steps=500):
     flops_launch = float(N) * 64 * FLOP_PER_NODE_RHS
     achieved = bytes_launch / (launch_us * 1e-6) / 1e9
     tflops = flops_launch / (launch_us * 1e-6) / 1e12
-    traffic, traffic_source = stored_traffic(tuned_kernel(opts), n, 64)
+    traffic, traffic_source = stored_traffic(tuned_kernel(opts, n), n, 64)
     return {"workload": f"N={n}, 64 members (seeded 1e-3 perturbations), {steps} RK4 steps, "
                         "Hilbert-ordered device copy, fused stages + HIP graphs",
-            "kernel": describe(opts), "options": opts,
+            "kernel": describe(opts, n), "options": opts,
             "member_steps_per_s": 64 / (ms * 1e-3), "ms_per_step": ms,
             "gnode_rhs_per_s": n * 4 * 64 / (ms * 1e-3) / 1e9,
             "single_member_steps_per_s": 1 / (ms1 * 1e-3),
@@ -384,7 +396,7 @@ def serve_leg(pkg, n_requests, rate, kernel="tiles", seed=2026, sample_every=250
     lat = np.array(lat)
     return {"workload": f"{n_requests} requests, Poisson {rate}/s, N in {{2562,10242,40962,163842}}, "
                         "1-32 members, 50-500 steps, HBM cap 200 GB, batches of 64 slots on "
-                        + ("member-lane LDS tiles" if tiles else "member pairs"),
+                        + ("LDS tiles" if tiles else "member pairs"),
             "p50_latency_s": float(np.percentile(lat, 50)),
             "p99_latency_s": float(np.percentile(lat, 99)),
             "p50_queue_s": float(np.percentile(np.array(que), 50)),

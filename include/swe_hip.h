@@ -249,10 +249,9 @@ int swe_hip_tune_ensemble(swe_hip_ctx *base, int members, unsigned flags, int st
  *     through registers, 4: direct-to-LDS, 8: direct-to-LDS with the first
  *     weights loaded before the tile barrier), and in fast mode AUTO above
  *     256 nodes per compute unit (the streaming form);
- *   members > 1: every member block untiled, and member block 32 tiled: in
- *     exact mode on member-lane tiles of tile_nodes 8 or 6 x tile_rows 70 or
- *     56, in fast mode the matrix-core ensemble kernel, which takes
- *     member_block 0 where 32 does not divide members;
+ *   members > 1: every member block untiled, member block 32 on
+ *     member-lane tiles of tile_nodes 8 or 6 x tile_rows 70 or 56, and in
+ *     fast mode the matrix-core ensemble kernel (member_block 0);
  *   SWE_HIP_FP32 contexts (flags must carry SWE_HIP_FP32, members == 1):
  *     LANE, TILE with 64, 128 and 256 nodes, and in fast mode PAIR, QUAD
  *     and OCT (lanes per node), and RESIDENT and AUTO as above.

@@ -289,6 +289,21 @@ int ensemble_rows(int halves)
     return std::min(254, (kUnitsMaxLds / 2 - ensemble_lds(halves, 0)) / (256 * halves + 4));
 }
 
+// Whether the items of a stage keep the workgroups busy: at least 95 % of the
+// turns the longest of them takes.  Members in blocks of 16 on 32 nodes make
+// coarse items: against k_stage_tspec (whole calls, all members active) N =
+// 4412 x 64 is 0.73 as fast at 54 %, 12252 x 32 0.88 at 75 %, 10242 x 64 0.91 at
+// 84 %, 60842 x 32 0.95 at 93 %, but 90252 x 64 1.06 at 96 %, 16002 x 64 1.04 at
+// 98 %, 116642 x 96 1.11 at 99 %.
+bool ensemble_fills(int n, int members, int ncu)
+{
+    const int halves = members > 8 ? 2 : 1, nodes = kEnsNodes / halves;
+    const long nmb = (members + 8 * halves - 1) / (8 * halves);
+    const long tiles = ((n + nodes - 1) / nodes + 7) / 8, W = (2L * ncu + 7) / 8;   // of one XCD
+    const long turns = tiles / W * nmb + (tiles % W * nmb + W - 1) / W;
+    return 20 * tiles * nmb >= 19 * turns * W;
+}
+
 bool ensemble_plan(SweUnits &u)
 {
     u.mode = UM_RESIDENT;

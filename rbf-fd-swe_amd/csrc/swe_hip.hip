@@ -1182,9 +1182,10 @@ int swe_hip_create_ex(const swe_hip_static *s, const swe_hip_options *o, swe_hip
     }
     // fast-mode ensembles on 31-point stencils run on the matrix cores when the
     // caller leaves the kernel open (no member block named) or asks for LDS
-    // tiles, unless a tile's rows do not fit the LDS or the records the
+    // tiles and the items are many enough, unless a tile's rows do not fit the LDS or the records the
     // device's memory; a named member block keeps its kernel and its bytes
-    if (!rc && c->B > 1 && c->nnbr == 31 && !exact(c) && (o->member_block == 0 || o->tiled)) {
+    if (!rc && c->B > 1 && c->nnbr == 31 && !exact(c) 
+        && (o->member_block == 0 || (o->tiled && ensemble_fills(c->n, c->B, c->ncu)))) {
         std::string why;
         std::vector<std::vector<int>> reads;
         int e = units_build(c, &reads, &why);
@@ -1333,15 +1334,13 @@ int swe_hip_tune_ex(swe_hip_ctx *base, int members, unsigned flags, int steps,
             if (members % mb)
                 continue;
             add(mb, 0, 0, 0, 0, 0);
-            if (mb == 32 && fast31)   // the matrix-core kernel cuts tiles of its own
-                add(mb, 0, 0, 1, 8, kTmemRows);
-            else if (mb == 32 && base->nnbr == 31)   // member-lane tiles: nodes x rows per tile
+            if (mb == 32 && base->nnbr == 31)   // member-lane tiles: nodes x rows per tile
                 for (int tn : {8, 6})
                     for (int tr : {kTmemRows, 56})
                         add(mb, 0, 0, 1, tn, tr);
         }
-        if (members % 32 && fast31)   // that kernel again where 32 does not divide
-            add(0, 0, 0, 0, 0, 0);    // (16 members at N = 10242: 23 against 42 us per stage)
+        if (fast31)   // the matrix-core kernel (16 members at N = 10242: 14.5
+            add(0, 0, 0, 0, 0, 0);   // against 42 us per stage)
     }
     double best_t = 1e300;
     int found = -1;

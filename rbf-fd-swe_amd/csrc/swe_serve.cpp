@@ -223,7 +223,22 @@ int new_batch(swe_srv *s, int mesh_id, int *batch_id)
                       owner, 0, 0, m.tiled ? SWE_HIP_ORDER_HILBERT : SWE_HIP_ORDER_HOST,
                       m.tiled ? 1 : 0, 0, 0, 0};
     swe_hip_ctx *ctx = nullptr;
-    int rc = swe_hip_create_ex(owner ? nullptr : &m.desc, &o, &ctx);
+    int rc = 0;
+    if (m.tiled && !(s->cfg.flags & SWE_HIP_EXACT)) {
+        // a batch is seldom full, so the kernel with blocks of 16 members serves
+        // it better than the one with 32 (20 mixed requests 98 against 118 ms);
+        // a context without its records has fallen back to another kernel
+        swe_hip_options e = o;
+        e.member_block = e.tiled = 0;
+        rc = swe_hip_create_ex(owner ? nullptr : &m.desc, &e, &ctx);
+        if (!rc && swe_hip_device_bytes(ctx) < m.slot_state_est * s->cfg.slots_per_batch
+                                                   + 1024LL * m.desc.compute_size) {
+            swe_hip_destroy(ctx);
+            ctx = nullptr;
+        }
+    }
+    if (!ctx)
+        rc = swe_hip_create_ex(owner ? nullptr : &m.desc, &o, &ctx);
     if (rc == SWE_HIP_ENOMEM)   // the device itself is full: wait while work
         return will_free() ? 1 : SWE_HIP_ENOMEM;   // is in flight, else fail
     if (rc)
@@ -349,6 +364,11 @@ int swe_srv_create(const swe_srv_config *cfg, swe_srv **out)
         return SWE_HIP_EINVAL;
     swe_srv *s = new swe_srv();
     s->cfg = *cfg;
+    // a batch stays within the bytes that admission counts: not the kernel with
+    // records of its own that the library would choose
+    if (s->cfg.member_block == 0)
+        for (s->cfg.member_block = 64; s->cfg.slots_per_batch % s->cfg.member_block != 0;)
+            s->cfg.member_block /= 2;
     *out = s;
     return 0;
 }

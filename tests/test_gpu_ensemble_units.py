@@ -17,7 +17,8 @@ def _states(prob, members, seed):
 @pytest.mark.parametrize("n,members,kw", [
     (642, 2, {}), (642, 6, {}), (642, 8, {}), (2562, 10, {}), (642, 16, {}), (2562, 24, {}),
     (10242, 4, dict(order="hilbert")), (10242, 40, dict(order="morton", slot_block=16)),
-    (2562, 96, dict(member_block=32, tiled=1, order="hilbert"))])
+    (2562, 96, dict(member_block=32, tiled=1, order="hilbert")),
+    (10242, 96, dict(member_block=32, tiled=1, order="hilbert"))])
 def test_members_equal_single_runs(pkg, n, members, kw):
     prob = pkg.host.Problem(pkg.mesh.case_path(n, seed=1), use_rcm=True, layout="cfdl")
     print(f"case: ensemble units N={n} members={members} {kw}", flush=True)
@@ -96,3 +97,17 @@ def test_tiles_with_too_many_rows_are_cut(pkg, tmp_path, members):
             one.set_state(H[k])
             one.rk_steps(2)
             assert np.array_equal(ens.get_state(k), one.get_state()), k
+
+
+def test_untiled_server_batches_hold_what_admission_counts(pkg):
+    """member_block 0 in a server: no records beside the static data and the
+    slots' states, which is all that admission counts for an untiled batch."""
+    prob = pkg.host.Problem(pkg.mesh.case_path(642, seed=1), use_rcm=True, layout="cfdl")
+    print("case: server with member_block 0, N=642", flush=True)
+    peak = {}
+    for mb in (0, 4):
+        req = pkg.serve.Request(mesh=0, inits=_states(prob, 3, 1), nsteps=2, tag=0, arrival_s=0.0)
+        with pkg.serve.Server(slots=4, member_block=mb) as srv:
+            srv.add_mesh(prob)
+            peak[mb] = srv.run([req])["hbm_peak"]
+    assert peak[0] == peak[4]
