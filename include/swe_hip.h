@@ -207,8 +207,9 @@ typedef struct swe_hip_options {
                                    >= 32, member_block 32, 31-point
                                    stencil): in fast mode the matrix-core
                                    kernel (same bits; tile_nodes, tile_rows
-                                   and prefetch then have no effect) unless
-                                   its tiles do not fit; else persistent
+                                   and prefetch then have no effect) where
+                                   its items of 32 nodes x 16 members fill
+                                   the chip and its tiles fit; else persistent
                                    member-lane tiles,
                                    loader and compute waves over two LDS
                                    images, 160 KB per workgroup             */
