@@ -104,7 +104,9 @@ __global__ __launch_bounds__(1024) void k_steps_exact(DevUnitsExact p)
             __builtin_amdgcn_s_waitcnt(0);
             __syncthreads();
             double x0 = 0.0;
-            {
+            // a short last tile has no units, and pos no entries, for the waves
+            // past its nodes
+            if (4 * wv < tcount) {
                 const uint4 *pu = pos + 64 * (wv >> 2) + 4 * (wv & 3) + b;
                 unsigned pw[16];
 #pragma unroll
