@@ -1486,6 +1486,13 @@ static int ring_download(swe_hip_ctx *c, void *host, const void *src, size_t byt
             HIPCHK(hipEventSynchronize(c->ring_ev[slot]));
         else
             HIPCHK(hipStreamSynchronize(c->stream));
+        // the work before the copy is done: a state it left invalid never
+        // reaches the caller's buffer
+        if (k == 0)
+            if (int rc = check_resident(c)) {
+                HIPCHK(hipStreamSynchronize(c->stream));   // the other slots' copies
+                return rc;
+            }
         std::memcpy((char *)host + off, c->ring + slot * kRingBytes,
                     std::min(kRingBytes, bytes - off));
         if (k + c->ring_slots < chunks)
@@ -1559,12 +1566,14 @@ static int from_device(swe_hip_ctx *c, int member, const T *src, T *host)
             return rc;
         if (direct) {
             HIPCHK(hipStreamSynchronize(c->stream));
+            if (int rc = check_resident(c))
+                return rc;
             std::memcpy(host, c->ring, bytes);
         } else if (int rc = ring_download(c, host, c->d_stage, bytes)) {
             return rc;
         }
     }
-    return check_resident(c);
+    return 0;
 }
 
 extern "C" {
