@@ -289,6 +289,18 @@ int ensemble_rows(int halves)
     return std::min(254, (kUnitsMaxLds / 2 - ensemble_lds(halves, 0)) / (256 * halves + 4));
 }
 
+// Items of 32 nodes x 16 members (64 x 8) of one XCD, and the turns its
+// workgroups need for them.
+static void ensemble_items(int n, int members, int ncu, long *items, long *turns, long *width)
+{
+    const int halves = members > 8 ? 2 : 1, nodes = kEnsNodes / halves;
+    const long nmb = (members + 8 * halves - 1) / (8 * halves);
+    const long tiles = ((n + nodes - 1) / nodes + 7) / 8, W = (2L * ncu + 7) / 8;
+    *items = tiles * nmb;
+    *turns = tiles / W * nmb + (tiles % W * nmb + W - 1) / W;
+    *width = W;
+}
+
 // Whether the items of a stage keep the workgroups busy: at least 95 % of the
 // turns the longest of them takes.  Members in blocks of 16 on 32 nodes make
 // coarse items: against k_stage_tspec (whole calls, all members active) N =
@@ -297,11 +309,27 @@ int ensemble_rows(int halves)
 // 98 %, 116642 x 96 1.11 at 99 %.
 bool ensemble_fills(int n, int members, int ncu)
 {
-    const int halves = members > 8 ? 2 : 1, nodes = kEnsNodes / halves;
-    const long nmb = (members + 8 * halves - 1) / (8 * halves);
-    const long tiles = ((n + nodes - 1) / nodes + 7) / 8, W = (2L * ncu + 7) / 8;   // of one XCD
-    const long turns = tiles / W * nmb + (tiles % W * nmb + W - 1) / W;
-    return 20 * tiles * nmb >= 19 * turns * W;
+    long items, turns, W;
+    ensemble_items(n, members, ncu, &items, &turns, &W);
+    return 20 * items >= 19 * turns * W;
+}
+
+// Whether an ensemble that names no member block runs this kernel.  Against
+// k_stage_members, the choice where 64 does not divide the members, it always
+// does (1.2 to 4.4 times as fast); k_stage_mpair's items are finer, and it is the
+// better one until 80 % of the turns are busy (in the first turn: half of
+// them, so that both workgroups of a compute unit are).  Against it, per
+// stage: N = 642 x 64 0.94 at 19 %, 1962 x 64 0.95 at 50 %, 5762 x 64 0.87 at 72 %,
+// 2562 x 192 0.87 at 69 %, 3242 x 192 1.01 at 81 %, 10242 x 64 1.05 at 85 %, 7842
+// x 64 1.09 at 97 %, first turn 2252 x 64 1.06 at 56 %.  Fewer than two tiles per
+// XCD are too uneven to tell (362 x 320 0.80).
+bool ensemble_default(int n, int members, int ncu)
+{
+    if (members % 64)
+        return true;
+    long items, turns, W;
+    ensemble_items(n, members, ncu, &items, &turns, &W);
+    return n >= 16 * kEnsNodes / 2 && (turns == 1 ? 2 * items > W : 5 * items >= 4 * turns * W);
 }
 
 bool ensemble_plan(SweUnits &u)

@@ -218,7 +218,9 @@ int resident_check(swe_hip_ctx *c, std::string *err);
 // with each tile's list of tiles it reads rows from, the co-residency check,
 // one launch of n steps.
 int units_build(swe_hip_ctx *c, std::vector<std::vector<int>> *nbr_tiles, std::string *err);
-bool ensemble_fills(int n, int members, int ncu);   // whether tiled ensembles run its ensemble form
+// whether tiled ensembles, and those that name no member block, run its ensemble form
+bool ensemble_fills(int n, int members, int ncu);
+bool ensemble_default(int n, int members, int ncu);
 int units_prepare(swe_hip_ctx *c, std::string *err);
 hipError_t units_launch(swe_hip_ctx *c, int nsteps, const DevResSync &y);
 void units_free(swe_hip_ctx *c);

@@ -1182,10 +1182,12 @@ int swe_hip_create_ex(const swe_hip_static *s, const swe_hip_options *o, swe_hip
     }
     // fast-mode ensembles on 31-point stencils run on the matrix cores when the
     // caller leaves the kernel open (no member block named) or asks for LDS
-    // tiles and the items are many enough, unless a tile's rows do not fit the LDS or the records the
-    // device's memory; a named member block keeps its kernel and its bytes
-    if (!rc && c->B > 1 && c->nnbr == 31 && !exact(c) 
-        && (o->member_block == 0 || (o->tiled && ensemble_fills(c->n, c->B, c->ncu)))) {
+    // tiles and the items are many enough, unless a tile's rows do not fit the
+    // LDS or the records the device's memory; a named member block keeps its
+    // kernel and its bytes
+    if (!rc && c->B > 1 && c->nnbr == 31 && !exact(c)
+        && (o->tiled ? ensemble_fills(c->n, c->B, c->ncu)
+                     : o->member_block == 0 && ensemble_default(c->n, c->B, c->ncu))) {
         std::string why;
         std::vector<std::vector<int>> reads;
         int e = units_build(c, &reads, &why);
