@@ -326,8 +326,10 @@ int swe_hip_info(const swe_hip_ctx *ctx, int *n_nodes, int *members,
                  int *nnbr, unsigned *flags);
 void *swe_hip_state_device_ptr(swe_hip_ctx *ctx);
 void *swe_hip_stream(swe_hip_ctx *ctx);
-/* Device bytes held by the context's state buffers, and by the static
- * data it uses (shared between contexts created with `share`). */
+/* Device bytes held by the context's state buffers and the unit records of
+ * its matrix-core or exact kernel, and by the static data it uses.  Contexts
+ * created with `share` use one copy of the static data and one of each form
+ * of records; the records count in every context that runs them. */
 long long swe_hip_device_bytes(const swe_hip_ctx *ctx);
 long long swe_hip_static_bytes(const swe_hip_ctx *ctx);
 

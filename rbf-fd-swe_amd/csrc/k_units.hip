@@ -451,12 +451,10 @@ int units_pack64(swe_hip_ctx *c, int units)
     SweUnits &u = c->units;
     const size_t wb = sizeof(double2) * 1024 * (size_t)units;
     const size_t gb = sizeof(double2) * kUnitGeo * (size_t)units;
-    const size_t hb = u.mode == UM_GLOBAL ? sizeof(double) * 64 * (size_t)units : 0;
-    if (hipMalloc(&u.d_wrec, wb) != hipSuccess || hipMalloc(&u.d_grec, gb) != hipSuccess
-        || (hb && hipMalloc(&u.d_hd, hb) != hipSuccess))
+    if (hipMalloc(&u.d_wrec, wb) != hipSuccess || hipMalloc(&u.d_grec, gb) != hipSuccess)
         return SWE_HIP_ENOMEM;
-    c->bytes += (long long)(wb + gb + hb);
-    u.bytes += (long long)(wb + gb + hb);
+    c->bytes += (long long)(wb + gb);
+    u.bytes += (long long)(wb + gb);
     pack_weights64(c, units);
     k_pack_geo<<<units, 192, 0, c->stream>>>(mesh_of(c), u.d_tile_start, u.d_unit_start,
                                              u.d_unit_tile, u.d_perm,

@@ -393,11 +393,10 @@ int units_pack32(swe_hip_ctx *c, int units)
 {
     SweUnits &u = c->units;
     const size_t rb = sizeof(float4) * 64 * kRec32 * (size_t)units;
-    const size_t hb = u.mode == UM_GLOBAL ? sizeof(float) * 64 * (size_t)units : 0;
-    if (hipMalloc(&u.d_wrec, rb) != hipSuccess || (hb && hipMalloc(&u.d_hd, hb) != hipSuccess))
+    if (hipMalloc(&u.d_wrec, rb) != hipSuccess)
         return SWE_HIP_ENOMEM;
-    c->bytes += (long long)(rb + hb);
-    u.bytes += (long long)(rb + hb);
+    c->bytes += (long long)rb;
+    u.bytes += (long long)rb;
     k_pack_units32<<<units, 64 * kRec32, 0, c->stream>>>(mesh32_of(c), u.d_tile_start,
                                                          u.d_unit_start, u.d_unit_tile, u.d_perm,
                                                          static_cast<float4 *>(u.d_wrec));

@@ -82,6 +82,7 @@ struct SweMesh {
     int sblk = 0;                 // stencil layout: 0 slot-major, 16 node blocks
     std::vector<int> perm;        // device node -> host node (empty: identity)
     int *d_inv = nullptr;         // host node -> device node, on the device
+    std::vector<struct SweUnitRecords *> unit_records;   // those contexts use (swe_units.hip)
     std::vector<double> h_xyz;    // node coordinates, device order, [3][n]
     std::vector<int> h_nbr;       // host copy of nbr, device order, [nnbr][n]
 };
@@ -99,9 +100,11 @@ struct SweTiles {
     double *d_geo_node = nullptr;            // [n][32] (member-lane kernel)
 };
 
-// Unit records of the matrix-core resident kernel (k_units.hip): tiles of
-// consecutive nodes along a space-filling curve, cut into units of 16.
+// Unit records of the matrix-core and exact unit kernels (k_units.hip,
+// k_units32.hip, k_exact.hip, k_ensemble.hip): compact tiles of a kernel order of
+// their own (recursive bisection), cut into units of 16 nodes.
 struct SweUnits {
+    struct SweUnitRecords *shared = nullptr;   // owner of all but d_hd
     int ntiles = 0;               // 0: not built
     int nodes = 0, units = 0, rows = 0;   // most nodes, units and rows of one tile
     int waves = 0, lds = 0;       // waves per workgroup, dynamic LDS bytes
@@ -111,6 +114,7 @@ struct SweUnits {
     bool stream_nt = false;       // FP32: streamed records bypass the last-level cache
     int chains = 1;               // FP32: partial sums per stencil sum, as split32's lanes
     int pos = 0, geo = 0;         // units whose positions, geometry the LDS holds
+    int all_units = 0;            // of all tiles
     long long bytes = 0;          // counted in the context's bytes too
     void *d_wrec = nullptr, *d_grec = nullptr, *d_hd = nullptr;
     char *d_tables = nullptr;     // one allocation, the tables below in it
@@ -118,6 +122,15 @@ struct SweUnits {
     const int *d_tile_start = nullptr, *d_unit_start = nullptr, *d_ustart = nullptr;
     const int *d_ulist = nullptr, *d_own_row = nullptr, *d_perm = nullptr;
     const int *d_unit_tile = nullptr;
+};
+
+// One form of the records of a mesh, read-only on the device and shared by the
+// contexts that run it; freed with the last of them.
+struct SweUnitRecords {
+    SweUnits u;
+    std::vector<std::vector<int>> reads;   // tiles each tile reads rows from
+    int form = 0;
+    int refs = 0;
 };
 
 struct swe_hip_ctx {
@@ -151,7 +164,8 @@ struct swe_hip_ctx {
     SweTiles tiles;              // LDS-staged ensemble kernel (ntiles == 0: unused)
     hipGraphExec_t graphs[swe::kGraphCount] = {};   // 64, 16, 4 and 1 RK steps
     // resident whole-step kernel (kernel == SWE_HIP_KERNEL_RESIDENT)
-    SweUnits units;                   // its matrix-core form (FP64, fast mode)
+    SweUnits units;                   // its unit form (all fast contexts, small exact FP64
+                                      // ones) or an ensemble's
     int res_block = 0, res_lds = 0;   // threads per workgroup, dynamic LDS bytes
     void *d_res_sync = nullptr;       // abort word + per-tile stage counts
     unsigned *h_res_abort = nullptr;  // pinned: wait time-out flag of the resident launches

@@ -6,6 +6,8 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <memory>
+#include <mutex>
 #include <new>
 #include <numeric>
 
@@ -37,13 +39,34 @@ int prec_at(bool by_node, int m, int slot)
 
 }  // namespace
 
-void units_free(swe_hip_ctx *c)
+// Guards the meshes' lists of records: contexts of one mesh may be destroyed by
+// different threads.
+static std::mutex g_records;
+
+static void free_records(SweUnits &u)
 {
-    SweUnits &u = c->units;
-    void *ptrs[] = {u.d_wrec, u.d_grec, u.d_hd, u.d_tables};
+    void *ptrs[] = {u.d_wrec, u.d_grec, u.d_tables};
     for (void *p : ptrs)
         if (p)
             (void)hipFree(p);
+}
+
+void units_free(swe_hip_ctx *c)
+{
+    SweUnits &u = c->units;
+    if (u.d_hd)
+        (void)hipFree(u.d_hd);
+    if (u.shared) {
+        std::lock_guard<std::mutex> lock(g_records);
+        if (--u.shared->refs == 0) {
+            std::vector<SweUnitRecords *> &all = c->mesh->unit_records;
+            all.erase(std::find(all.begin(), all.end(), u.shared));
+            free_records(u.shared->u);
+            delete u.shared;
+        }
+    } else {
+        free_records(u);   // of a build that failed
+    }
     c->bytes -= u.bytes;
     u = SweUnits{};
 }
@@ -214,8 +237,8 @@ static int build(swe_hip_ctx *c, std::vector<std::vector<int>> *nbr_tiles, std::
             for (int slot = W; slot < 32; ++slot)
                 for (int m = 0; m < 16; ++m)
                     prec[(size_t)k * 512 + prec_at(false, m, slot)] = (unsigned short)rows;
-    u.chains = c->fp32 && c->split32 == 2 ? 2 : 1;
     u.ntiles = nt;
+    u.all_units = units;
     u.nodes = std::min(n, tmax);
     u.units = (u.nodes + 15) / 16;
     u.rows = rows;
@@ -267,14 +290,58 @@ static int build(swe_hip_ctx *c, std::vector<std::vector<int>> *nbr_tiles, std::
     return rc;
 }
 
+// Contexts of one mesh share the records of the form they run: N = 655362 in
+// FP64 holds 0.75 GB of them.
+static int share_or_build(swe_hip_ctx *c, std::vector<std::vector<int>> *nbr_tiles,
+                          std::string *err)
+{
+    const int form = c->B > 8 ? 2 : c->B > 1 ? 1 : exact(c) ? 3 : 0;
+    std::vector<SweUnitRecords *> &all = c->mesh->unit_records;
+    std::lock_guard<std::mutex> lock(g_records);
+    auto at = std::find_if(all.begin(), all.end(),
+                           [&](const SweUnitRecords *r) { return r->form == form; });
+    if (at == all.end()) {
+        if (int rc = build(c, nbr_tiles, err))
+            return rc;
+        auto r = std::make_unique<SweUnitRecords>();
+        r->u = c->units;
+        r->reads = *nbr_tiles;
+        r->form = form;
+        r->refs = 1;
+        all.push_back(r.get());
+        c->units.shared = r.release();
+    } else {
+        c->units = (*at)->u;
+        c->units.shared = *at;
+        ++(*at)->refs;
+        c->bytes += c->units.bytes;
+        *nbr_tiles = (*at)->reads;
+    }
+    c->units.chains = c->fp32 && c->split32 == 2 ? 2 : 1;
+    return 0;
+}
+
 int units_build(swe_hip_ctx *c, std::vector<std::vector<int>> *nbr_tiles, std::string *err)
 {
     try {
-        return build(c, nbr_tiles, err);
+        if (int rc = share_or_build(c, nbr_tiles, err))
+            return rc;
     } catch (const std::bad_alloc &) {
         *err = "unit tables: out of host memory";
         return SWE_HIP_ENOMEM;
     }
+    SweUnits &u = c->units;
+    if (c->B == 1 && u.mode == UM_GLOBAL) {   // D of the streamed units is the context's own
+        const size_t hb = (c->fp32 ? sizeof(float) : sizeof(double)) * 64 * (size_t)u.all_units;
+        if (hipMalloc(&u.d_hd, hb) != hipSuccess) {
+            u.d_hd = nullptr;
+            *err = "unit records: allocation of D";
+            return SWE_HIP_ENOMEM;
+        }
+        c->bytes += (long long)hb;
+        u.bytes += (long long)hb;
+    }
+    return 0;
 }
 
 void units_tables(const swe_hip_ctx *c, int nsteps, const DevResSync &y, DevUnits *p)
