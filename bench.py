@@ -183,18 +183,31 @@ def measured_kernel(args):
     if args.members == 1 and args.kernel == "auto" and args.nodes <= UNITS_MAX_NODES:
         return "k_steps_units32" if args.fp32 else "k_steps_units"
     if args.members > 1:
-        return "k_stage_ensemble" if args.member_block == 0 and not args.tiled or \
-            args.tiled and ensemble_fills(args.nodes, args.members) else name
+        return "k_stage_ensemble" if args.tiled and ensemble_fills(args.nodes, args.members) or \
+            not args.tiled and args.member_block == 0 and \
+            ensemble_default(args.nodes, args.members) else name
     return UNIT_KERNELS.get(name, name)
 
 
-def ensemble_fills(nodes, members):
-    """The library's rule for tiled fast-mode ensembles, on 256 compute units."""
+def ensemble_items(nodes, members):
+    """Items of one XCD and the turns they take, on 256 compute units."""
     halves = 2 if members > 8 else 1
     tiles = -(-(-(-nodes // (64 // halves))) // 8)
     nmb = -(-members // (8 * halves))
-    turns = tiles // 64 * nmb + -(-(tiles % 64 * nmb) // 64)
-    return 20 * tiles * nmb >= 19 * turns * 64
+    return tiles * nmb, tiles // 64 * nmb + -(-(tiles % 64 * nmb) // 64)
+
+
+def ensemble_default(nodes, members):
+    """The library's rule for fast-mode ensembles that name no member block."""
+    items, turns = ensemble_items(nodes, members)
+    return members % 64 != 0 or nodes >= 512 and (
+        2 * items > 64 if turns == 1 else 5 * items >= 4 * turns * 64)
+
+
+def ensemble_fills(nodes, members):
+    """The library's rule for tiled fast-mode ensembles."""
+    items, turns = ensemble_items(nodes, members)
+    return turns >= 4 and 20 * items >= 19 * turns * 64
 
 
 RESIDENT_NOTE = ("the kernel runs every stage of a call in one launch: 'launch' here is "
@@ -253,8 +266,10 @@ def tuned_kernel(opts, nodes):
     name = leg_kernel(opts)
     if opts.get("members", 1) == 1:
         return "k_steps_units" if opts["kernel"] == "auto" else UNIT_KERNELS.get(name, name)
-    if opts["member_block"] == 0 or opts["tiled"] and ensemble_fills(nodes, opts["members"]):
-        return "k_stage_ensemble"
+    if opts["tiled"]:
+        return "k_stage_ensemble" if ensemble_fills(nodes, opts["members"]) else name
+    if opts["member_block"] == 0:
+        return "k_stage_ensemble" if ensemble_default(nodes, opts["members"]) else "k_stage_mpair"
     return name
 
 

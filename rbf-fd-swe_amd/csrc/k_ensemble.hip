@@ -306,12 +306,14 @@ static void ensemble_items(int n, int members, int ncu, long *items, long *turns
 // coarse items: against k_stage_tspec (whole calls, all members active) N =
 // 4412 x 64 is 0.73 as fast at 54 %, 12252 x 32 0.88 at 75 %, 10242 x 64 0.91 at
 // 84 %, 60842 x 32 0.95 at 93 %, but 90252 x 64 1.06 at 96 %, 16002 x 64 1.04 at
-// 98 %, 116642 x 96 1.11 at 99 %.
+// 98 %, 116642 x 96 1.11 at 99 %.  Not before the fourth turn, up to which 12 to 14
+// us a turn instead of 11 keep it behind (12252 x 64 0.97 in three full ones,
+// 16002 x 32 0.96 in two).
 bool ensemble_fills(int n, int members, int ncu)
 {
     long items, turns, W;
     ensemble_items(n, members, ncu, &items, &turns, &W);
-    return 20 * items >= 19 * turns * W;
+    return turns >= 4 && 20 * items >= 19 * turns * W;
 }
 
 // Whether an ensemble that names no member block runs this kernel.  Against

@@ -33,3 +33,26 @@ def test_default_kernel_rule(pkg, tmp_path, n, members, records):
             one.set_state(H[m])
             one.rk_steps(3)
             assert np.array_equal(ens.get_state(m), one.get_state()), m
+
+
+@pytest.mark.parametrize("n,members,records", [
+    (12252, 64, False), (16000, 32, False),      # full, but in three and two turns
+    (16000, 64, True), (10244, 96, True),        # 98 % and 96 % of four
+    (2560, 96, False), (10240, 64, False)])      # 52 % and 84 %
+def test_tiled_kernel_rule(pkg, tmp_path, n, members, records):
+    """Tiled contexts: the matrix-core kernel shows as item records without the
+    member-lane tiles' node-major copies (1280 bytes per node)."""
+    prob = _sphere(pkg, tmp_path, n)
+    print(f"case: tiled ensemble N={n} members={members}", flush=True)
+    size = prob.compute_size
+    with pkg.runtime.HipContext(prob, kernel="pair", order="hilbert") as one, \
+            pkg.runtime.HipContext(prob, members=members, member_block=32, tiled=1,
+                                   share=one) as ens:
+        extra = ens.device_bytes() - 4 * 32 * size * members - 32 * size
+        assert (1024 * size < extra < 1350 * size) == records, extra / size
+        for m in range(members):
+            ens.set_state(prob.H_init, m)
+        ens.rk_steps(3)
+        one.set_state(prob.H_init)
+        one.rk_steps(3)
+        assert np.array_equal(ens.get_state(members - 1), one.get_state())
