@@ -334,6 +334,32 @@ bool ensemble_default(int n, int members, int ncu)
     return n >= 16 * kEnsNodes / 2 && (turns == 1 ? 2 * items > W : 5 * items >= 4 * turns * W);
 }
 
+// Whether a launch of a batch context (tiles and records) runs this kernel.  It
+// works on blocks of 16 active members, k_stage_tspec on whole slots: measured
+// over 642 to 163842 nodes x 32 to 128 slots, the one takes 9 to 14 us in the first
+// turn and 11 to 13 per turn beyond, the other 3.5 us and 4.5e-5 per node and slot,
+// a tenth less when one block of 32 is active.  N = 10242 x 64: 16, 32, 48 and 64
+// active members 14.2, 25.3, 26.8, 37.1 against 32.1, 32.1, 32.7, 32.7; 2562 x 64: 9.1,
+// 9.6, 11.3, 13.5 against 11.4, 11.0, 11.7, 11.7; 642 x 64: 9 against 6.  Beside
+// other batches the compute units that turns leave idle are not lost, so only the
+// floor of a turn counts: two full batches of 64 slots at once take 0.88 of
+// k_stage_tspec's time at N = 2562, 10242 and 40962, but 1.36 at 642.
+bool ensemble_batch(int n, int slots, int active, bool alone, int ncu)
+{
+    long items, turns, W;
+    ensemble_items(n, std::max(active, 9), ncu, &items, &turns, &W);
+    const double mine = !alone ? 9.3 : turns > 1 ? 13.0 * turns : 2 * items > W ? 14.0 : 9.3;
+    const double blocks = (double)((active + 31) / 32) / (slots / 32.0);
+    return mine <= 3.5 + 4.5e-5 * n * slots * (0.9 + 0.1 * blocks);
+}
+
+long long ensemble_bytes(int n)
+{
+    // tiles of two units: weights, geometry, positions, rows, their owners
+    const long long tile = 2 * (16 * 1024 + 16 * 16 * kEnsGeo + 1024) + 4 * 2 * 254 + 64;
+    return (n / (kEnsNodes / 2) + 1) * tile + 4LL * n + 8 * 256;
+}
+
 bool ensemble_plan(SweUnits &u)
 {
     u.mode = UM_RESIDENT;

@@ -43,6 +43,9 @@ constexpr int kUnitsMaxPerCu = 4096;
 // 4-node group on each of 16 waves; 126 registers, more waves do not fit):
 // 3.58 against 4.16 us per stage at N = 16002; k_steps_resident above.
 constexpr int kExactMaxPerCu = 64;
+// Bytes per node of the member-lane kernel's tiles, at most (1485 to 1510 for
+// 642 to 163842 nodes).
+constexpr long long kMemberTileBytes = 2048;
 constexpr int kResMaxNbrs = 64;           // tiles one tile exchanges rows with (one wave)
 constexpr int kResAutoMinSteps = 4;       // AUTO contexts: shorter calls replay stage graphs
 
@@ -162,7 +165,11 @@ struct swe_hip_ctx {
     hipEvent_t ring_ev[swe::kRingSlots] = {};
     int *d_active = nullptr;     // member slots advanced by the ensemble kernel
     SweTiles tiles;              // LDS-staged ensemble kernel (ntiles == 0: unused)
-    hipGraphExec_t graphs[swe::kGraphCount] = {};   // 64, 16, 4 and 1 RK steps
+    int active = 0;              // its last value set by the host
+    bool alone = true;           // batch contexts: no other batch has work (swe_batch.h)
+    bool late_tiles = false;     // and the tiles are built for the first launch that runs them
+    // 64, 16, 4 and 1 RK steps; [1] on the ensemble form of a batch context
+    hipGraphExec_t graphs[2][swe::kGraphCount] = {};
     // resident whole-step kernel (kernel == SWE_HIP_KERNEL_RESIDENT)
     SweUnits units;                   // its unit form (all fast contexts, small exact FP64
                                       // ones) or an ensemble's
@@ -235,9 +242,11 @@ int units_build(swe_hip_ctx *c, std::vector<std::vector<int>> *nbr_tiles, std::s
 // whether tiled ensembles, and those that name no member block, run its ensemble form
 bool ensemble_fills(int n, int members, int ncu);
 bool ensemble_default(int n, int members, int ncu);
+bool ensemble_batch(int n, int slots, int active, bool alone, int ncu);   // and launches of batch contexts
 int units_prepare(swe_hip_ctx *c, std::string *err);
 hipError_t units_launch(swe_hip_ctx *c, int nsteps, const DevResSync &y);
 void units_free(swe_hip_ctx *c);
+long long ensemble_bytes(int n);   // at most, of an ensemble of more than 8 members
 
 // Looks up this device's no-allocation scratch address (swe_noalloc.hip);
 // the device must be current.  On failure *err says why.
@@ -267,11 +276,18 @@ void launch_members_stage(const swe_hip_ctx *c, int stage, const DevStage &st);
 void launch_tiled_stage(const swe_hip_ctx *c, int stage, const DevStage &st);
 void launch_ensemble_stage(const swe_hip_ctx *c, int stage, const DevStage &st);
 
+// Whether a stage of this ensemble runs k_stage_ensemble.
+inline bool ensemble_form(const swe_hip_ctx *c)
+{
+    return c->B > 1 && c->units.ntiles > 0
+           && (c->tiles.ntiles == 0 || ensemble_batch(c->n, c->B, c->active, c->alone, c->ncu));
+}
+
 inline void launch_stage(const swe_hip_ctx *c, int stage, const DevStage &st)
 {
     if (c->B == 1)
         launch_single_stage(c, stage, st);
-    else if (c->units.ntiles > 0)
+    else if (ensemble_form(c))
         launch_ensemble_stage(c, stage, st);
     else if (c->tiles.ntiles > 0)
         launch_tiled_stage(c, stage, st);

@@ -4,6 +4,7 @@
 // fused and graph-captured fast path, state upload/read-back in the
 // reference's host layouts (swe_code/main/include/swe_config.h:21-54).
 #include "host_par.h"
+#include "swe_batch.h"
 #include "swe_ctx.h"
 
 #include <hip/hip_runtime.h>
@@ -317,7 +318,9 @@ void free_ctx(swe_hip_ctx *c)
         return;
     (void)hipSetDevice(c->dev);
     if (c->stream) (void)hipStreamSynchronize(c->stream);
-    for (hipGraphExec_t g : c->graphs)
+    for (hipGraphExec_t g : c->graphs[0])
+        if (g) (void)hipGraphExecDestroy(g);
+    for (hipGraphExec_t g : c->graphs[1])
         if (g) (void)hipGraphExecDestroy(g);
     void *ptrs[] = {c->d_H, c->d_Ka, c->d_Kb, c->d_D, c->d_F, c->d_stage, c->d_active,
                     c->f_H, c->f_Ka, c->f_Kb, c->f_D, c->f_F,
@@ -740,6 +743,35 @@ int build_tiles(swe_hip_ctx *c, int tmax, int umax, std::vector<int> *h_tstart =
     return rc;
 }
 
+// The member-lane kernel's tiles.
+int build_member_tiles(swe_hip_ctx *c)
+{
+    int lds_max = 0;
+    if (c->nnbr != 31)
+        return fail(SWE_HIP_EINVAL, "the member-lane tiled kernel (member block 32) needs a "
+                                    "31-point stencil");
+    if (hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, c->dev)
+            != hipSuccess
+        || (size_t)lds_max < sizeof(double) * (size_t)kTmemLdsDoubles)
+        return fail(SWE_HIP_EDEVICE, "the member-lane tiled kernel needs 160 KB of LDS per "
+                                     "workgroup");
+    return build_tiles(c, c->tile_nodes ? c->tile_nodes : kTmemTile,
+                       c->tile_rows ? c->tile_rows : kTmemRows);
+}
+
+// The matrix-core ensemble kernel's records; false (and none) where a tile's
+// rows do not fit the LDS or the records the device's memory.
+bool ensemble_records(swe_hip_ctx *c)
+{
+    std::string why;
+    std::vector<std::vector<int>> reads;
+    if (!units_build(c, &reads, &why) && !units_prepare(c, &why))
+        return true;
+    (void)hipGetLastError();
+    units_free(c);
+    return false;
+}
+
 // Resident kernels: for every tile, the tiles it must wait for before a
 // stage -- owners of the rows it reads (reads[t]) and tiles that read its
 // rows -- at a stride of kResMaxNbrs, -1 padded.
@@ -1074,6 +1106,7 @@ int swe_hip_create_ex(const swe_hip_static *s, const swe_hip_options *o, swe_hip
                   "hipMemsetAsync");
     if (!rc) {
         k_set_int<<<1, 64, 0, c->stream>>>(c->d_active, c->B);
+        c->active = c->B;
         rc = check_launch("k_set_int");
     }
     if (!rc && c->B == 1 && c->kernel == SWE_HIP_KERNEL_TILE && (!fp32 || c->nnbr == 31)) {
@@ -1187,33 +1220,10 @@ int swe_hip_create_ex(const swe_hip_static *s, const swe_hip_options *o, swe_hip
     // kernel and its bytes
     if (!rc && c->B > 1 && c->nnbr == 31 && !exact(c)
         && (o->tiled ? ensemble_fills(c->n, c->B, c->ncu)
-                     : o->member_block == 0 && ensemble_default(c->n, c->B, c->ncu))) {
-        std::string why;
-        std::vector<std::vector<int>> reads;
-        int e = units_build(c, &reads, &why);
-        if (!e)
-            e = units_prepare(c, &why);
-        if (e) {
-            (void)hipGetLastError();
-            units_free(c);
-        }
-    }
-    if (!rc && o->tiled && c->units.ntiles == 0) {
-        int lds_max = 0;
-        {
-            if (c->nnbr != 31)
-                rc = fail(SWE_HIP_EINVAL, "the member-lane tiled kernel (member block 32) needs "
-                                          "a 31-point stencil");
-            else if (hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock,
-                                           device) != hipSuccess ||
-                     (size_t)lds_max < sizeof(double) * (size_t)kTmemLdsDoubles)
-                rc = fail(SWE_HIP_EDEVICE, "the member-lane tiled kernel needs 160 KB of LDS "
-                                           "per workgroup");
-            else
-                rc = build_tiles(c, c->tile_nodes ? c->tile_nodes : kTmemTile,
-                                 c->tile_rows ? c->tile_rows : kTmemRows);
-        }
-    }
+                     : o->member_block == 0 && ensemble_default(c->n, c->B, c->ncu)))
+        (void)ensemble_records(c);
+    if (!rc && o->tiled && c->units.ntiles == 0)
+        rc = build_member_tiles(c);
     if (!rc)
         check(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
     if (rc) {
@@ -1407,7 +1417,39 @@ int swe_hip_set_active(swe_hip_ctx *c, int active)
         return fail(SWE_HIP_EINVAL, "set_active: bad ctx or count");
     HIPCHK(hipSetDevice(c->dev));
     k_set_int<<<1, 64, 0, c->stream>>>(c->d_active, active);
+    c->active = active;
     return check_launch("k_set_int");
+}
+
+int swe_hip_batch_create(const swe_hip_static *s, const swe_hip_options *o, long long room,
+                         swe_hip_ctx **out, swe_hip_batch_bytes *bytes)
+{
+    *bytes = swe_hip_batch_bytes{};
+    const long long n = o->share ? o->share->n : s ? s->compute_size : 0;
+    const long long both = ensemble_bytes((int)n) + kMemberTileBytes * n;
+    if (o->tiled && !(o->flags & SWE_HIP_EXACT) && both <= room) {
+        swe_hip_options e = *o;
+        e.tiled = 0;   // its named member block takes no records by itself
+        swe_hip_ctx *c = nullptr;
+        if (int rc = swe_hip_create_ex(s, &e, &c))
+            return rc;
+        const long long before = c->bytes;
+        if (c->nnbr == 31 && ensemble_records(c)) {
+            bytes->records = c->bytes - before;
+            c->late_tiles = !ensemble_fills(c->n, c->B, c->ncu);
+            bytes->tiles = c->late_tiles ? kMemberTileBytes * n : 0;
+            *out = c;
+            return 0;
+        }
+        free_ctx(c);
+    }
+    return swe_hip_create_ex(s, o, out);
+}
+
+void swe_hip_batch_alone(swe_hip_ctx *c, int alone)
+{
+    if (c)
+        c->alone = alone != 0;
 }
 
 int swe_hip_move_member(swe_hip_ctx *c, int from, int to)
@@ -1859,16 +1901,27 @@ int swe_hip_rk_steps(swe_hip_ctx *c, int nsteps)
                 launch_fused(c, s);
         return check_launch("stage kernels");
     }
-    // every graph is captured on the first call, so no later (timed) call
-    // pays for a capture
+    if (c->late_tiles && !ensemble_batch(c->n, c->B, c->active, c->alone, c->ncu)) {
+        c->late_tiles = false;
+        int e = SWE_HIP_ENOMEM;
+        try {
+            e = build_member_tiles(c);
+        } catch (const std::bad_alloc &) {
+        }
+        if (e)   // the records alone
+            (void)hipGetLastError();
+    }
+    // every graph is captured on the first call (of a batch context: on each
+    // form), so no later (timed) call pays for a capture
+    hipGraphExec_t *graphs = c->graphs[c->tiles.ntiles > 0 && ensemble_form(c)];
     for (int g = 0; g < kGraphCount; ++g)
-        if (!c->graphs[g])
-            if (int rc = capture_steps(c, kGraphSteps[g], &c->graphs[g]))
+        if (!graphs[g])
+            if (int rc = capture_steps(c, kGraphSteps[g], &graphs[g]))
                 return rc;
     int left = nsteps;
     for (int g = 0; g < kGraphCount; ++g)
         for (; left >= kGraphSteps[g]; left -= kGraphSteps[g])
-            HIPCHK(hipGraphLaunch(c->graphs[g], c->stream));
+            HIPCHK(hipGraphLaunch(graphs[g], c->stream));
     return 0;
 }
 

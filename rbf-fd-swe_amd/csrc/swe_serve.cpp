@@ -10,6 +10,7 @@
 // (min(chunk_steps, smallest remaining budget)); members join and leave only
 // at chunk boundaries, which never changes any member's arithmetic.
 #include "swe_serve.h"
+#include "swe_batch.h"
 
 #include <algorithm>
 #include <chrono>
@@ -42,6 +43,7 @@ struct Batch {
     bool busy = false;
     int chunk = 0;
     long long bytes = 0;
+    bool records = false;        // has the matrix-core kernel's records (swe_batch.h)
 };
 
 struct Mesh {
@@ -55,6 +57,8 @@ struct Mesh {
     std::vector<int> batches;
     long long static_bytes = 0;  // charged while resident
     bool resident = false;
+    int records = 0;             // batches with records: one copy, charged once
+    long long record_bytes = 0;
 };
 
 struct Request {
@@ -178,6 +182,9 @@ void evict(swe_srv *s, int batch_id)
     b.ctx = nullptr;
     s->hbm_in_use -= b.bytes;
     b.bytes = 0;
+    if (b.records && --m.records == 0)
+        s->hbm_in_use -= m.record_bytes;
+    b.records = false;
     m.batches.erase(std::find(m.batches.begin(), m.batches.end(), batch_id));
     if (m.batches.empty() && m.resident) {
         s->hbm_in_use -= m.static_bytes;
@@ -223,22 +230,12 @@ int new_batch(swe_srv *s, int mesh_id, int *batch_id)
                       owner, 0, 0, m.tiled ? SWE_HIP_ORDER_HILBERT : SWE_HIP_ORDER_HOST,
                       m.tiled ? 1 : 0, 0, 0, 0};
     swe_hip_ctx *ctx = nullptr;
-    int rc = 0;
-    if (m.tiled && !(s->cfg.flags & SWE_HIP_EXACT)) {
-        // a batch is seldom full, so the kernel with blocks of 16 members serves
-        // it better than the one with 32 (20 mixed requests 98 against 118 ms);
-        // a context without its records has fallen back to another kernel
-        swe_hip_options e = o;
-        e.member_block = e.tiled = 0;
-        rc = swe_hip_create_ex(owner ? nullptr : &m.desc, &e, &ctx);
-        if (!rc && swe_hip_device_bytes(ctx) < m.slot_state_est * s->cfg.slots_per_batch
-                                                   + 1024LL * m.desc.compute_size) {
-            swe_hip_destroy(ctx);
-            ctx = nullptr;
-        }
-    }
-    if (!ctx)
-        rc = swe_hip_create_ex(owner ? nullptr : &m.desc, &o, &ctx);
+    // chunks that are not full run faster on a second kernel (20 mixed requests
+    // 107 against 200 ms); what both kernels need beyond the admission's estimate
+    // stays out of the last half of the budget
+    swe_hip_batch_bytes extra{};
+    int rc = swe_hip_batch_create(owner ? nullptr : &m.desc, &o,
+                                  s->cfg.hbm_cap_bytes / 2 - s->hbm_in_use - need(), &ctx, &extra);
     if (rc == SWE_HIP_ENOMEM)   // the device itself is full: wait while work
         return will_free() ? 1 : SWE_HIP_ENOMEM;   // is in flight, else fail
     if (rc)
@@ -247,12 +244,19 @@ int new_batch(swe_srv *s, int mesh_id, int *batch_id)
     b.ctx = ctx;
     b.mesh = mesh_id;
     b.slots.assign(s->cfg.slots_per_batch, Slot{});
-    b.bytes = swe_hip_device_bytes(ctx);
+    b.bytes = swe_hip_device_bytes(ctx) - extra.records + extra.tiles;
     charge(s, b.bytes);
     if (!m.resident) {
         m.resident = true;
         m.static_bytes = swe_hip_static_bytes(ctx);
         charge(s, m.static_bytes);
+    }
+    if (extra.records > 0) {
+        b.records = true;
+        if (m.records++ == 0) {
+            m.record_bytes = extra.records;
+            charge(s, extra.records);
+        }
     }
     s->batches.push_back(std::move(b));
     *batch_id = (int)s->batches.size() - 1;
@@ -320,6 +324,10 @@ int launch(swe_srv *s, Batch &b, int *progress)
     int chunk = s->cfg.chunk_steps;
     for (int i = 0; i < b.active; ++i)
         chunk = std::min(chunk, b.slots[i].remaining);
+    swe_hip_batch_alone(b.ctx, std::none_of(s->batches.begin(), s->batches.end(),
+                                            [&](const Batch &o) {
+                                                return &o != &b && o.ctx && o.active > 0;
+                                            }));
     int rc = swe_hip_set_active(b.ctx, b.active);
     if (!rc && chunk > 0)
         rc = swe_hip_rk_steps(b.ctx, chunk);

@@ -290,23 +290,29 @@ static int build(swe_hip_ctx *c, std::vector<std::vector<int>> *nbr_tiles, std::
     return rc;
 }
 
+// The context's form of the records (tiles, plan and contents depend on no more).
+static int form_of(const swe_hip_ctx *c)
+{
+    return c->B > 8 ? 2 : c->B > 1 ? 1 : exact(c) ? 3 : 0;
+}
+
 // Contexts of one mesh share the records of the form they run: N = 655362 in
 // FP64 holds 0.75 GB of them.
 static int share_or_build(swe_hip_ctx *c, std::vector<std::vector<int>> *nbr_tiles,
                           std::string *err)
 {
-    const int form = c->B > 8 ? 2 : c->B > 1 ? 1 : exact(c) ? 3 : 0;
     std::vector<SweUnitRecords *> &all = c->mesh->unit_records;
     std::lock_guard<std::mutex> lock(g_records);
-    auto at = std::find_if(all.begin(), all.end(),
-                           [&](const SweUnitRecords *r) { return r->form == form; });
+    const auto at = std::find_if(all.begin(), all.end(), [&](const SweUnitRecords *r) {
+        return r->form == form_of(c);
+    });
     if (at == all.end()) {
         if (int rc = build(c, nbr_tiles, err))
             return rc;
         auto r = std::make_unique<SweUnitRecords>();
         r->u = c->units;
         r->reads = *nbr_tiles;
-        r->form = form;
+        r->form = form_of(c);
         r->refs = 1;
         all.push_back(r.get());
         c->units.shared = r.release();
