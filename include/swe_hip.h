@@ -229,15 +229,19 @@ int swe_hip_create_ex(const swe_hip_static *s, const swe_hip_options *o, swe_hip
  * steps of a `members`-slot context on the static data of `base` for every
  * admissible member block (powers of two 2..64 dividing members) and
  * returns the fastest in *best_mb with its time per step in
- * *best_ms_per_step.  Timing uses HIP events on the candidates' streams. */
+ * *best_ms_per_step.  Timing uses HIP events on the candidates' streams.
+ * Named blocks only: the library's choice (member_block 0), which in fast
+ * mode runs the matrix-core kernel where that is the faster one (N = 10242 x
+ * 16: 14.5 against 42 us per stage), is among swe_hip_tune_ex's candidates. */
 int swe_hip_tune_member_block(swe_hip_ctx *base, int members, unsigned flags, int steps,
                               int *best_mb, double *best_ms_per_step);
 
 /* The same over the LDS-tiled ensemble kernel too (member block 32,
- * member-lane tiles, 31-point stencils, tiled = 1).  Returns the fastest (member block, tiled) pair; tiles follow
- * the node order of base's device copy (create base with
- * SWE_HIP_ORDER_HILBERT for compact tiles).  No counterpart in the
- * reference (its ensemble runs are separate processes). */
+ * member-lane tiles, 31-point stencils, tiled = 1), named blocks only as
+ * well.  Returns the fastest (member block, tiled) pair; tiles follow the
+ * node order of base's device copy (create base with SWE_HIP_ORDER_HILBERT
+ * for compact tiles).  No counterpart in the reference (its ensemble runs
+ * are separate processes). */
 int swe_hip_tune_ensemble(swe_hip_ctx *base, int members, unsigned flags, int steps,
                           int *best_mb, int *best_tiled, double *best_ms_per_step);
 
@@ -252,7 +256,8 @@ int swe_hip_tune_ensemble(swe_hip_ctx *base, int members, unsigned flags, int st
  *     256 nodes per compute unit (the streaming form);
  *   members > 1: every member block untiled, member block 32 on
  *     member-lane tiles of tile_nodes 8 or 6 x tile_rows 70 or 56, and in
- *     fast mode the matrix-core ensemble kernel (member_block 0);
+ *     fast mode the matrix-core ensemble kernel once (member_block 0, or a
+ *     tiled candidate where only those run it);
  *   SWE_HIP_FP32 contexts (flags must carry SWE_HIP_FP32, members == 1):
  *     LANE, TILE with 64, 128 and 256 nodes, and in fast mode PAIR, QUAD
  *     and OCT (lanes per node), and RESIDENT and AUTO as above.

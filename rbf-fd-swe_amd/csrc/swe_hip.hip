@@ -830,7 +830,8 @@ namespace {
 // Milliseconds per fused RK step of one candidate configuration on the
 // static data of `base`: one warm-up step (graph capture), then `steps`
 // timed with HIP events on the candidate's stream.
-int time_options(swe_hip_ctx *base, const swe_hip_options &opt, int steps, double *per_step)
+int time_options(swe_hip_ctx *base, const swe_hip_options &opt, int steps, double *per_step,
+                 bool *ensemble = nullptr)
 {
     swe_hip_options o = opt;
     o.share = base;
@@ -839,6 +840,8 @@ int time_options(swe_hip_ctx *base, const swe_hip_options &opt, int steps, doubl
     int rc = swe_hip_create_ex(nullptr, &o, &c);
     if (rc)
         return rc;
+    if (ensemble)   // whether it ran the matrix-core ensemble kernel
+        *ensemble = ensemble_form(c);
     hipEvent_t e0 = nullptr, e1 = nullptr;
     float ms = 0.0f;
     rc = swe_hip_rk_steps(c, 1);
@@ -1342,6 +1345,9 @@ int swe_hip_tune_ex(swe_hip_ctx *base, int members, unsigned flags, int steps,
                 for (int pf : {0, 4, 8})
                     add(0, SWE_HIP_KERNEL_TILE, pf, 0, tn, 0);
     } else {
+        if (fast31 && ensemble_default(base->n, members, base->ncu))
+            add(0, 0, 0, 0, 0, 0);   // the matrix-core kernel (16 members at N =
+                                     // 10242: 14.5 against 42 us per stage)
         for (int mb = 64; mb >= 2; mb >>= 1) {
             if (members % mb)
                 continue;
@@ -1351,14 +1357,19 @@ int swe_hip_tune_ex(swe_hip_ctx *base, int members, unsigned flags, int steps,
                     for (int tr : {kTmemRows, 56})
                         add(mb, 0, 0, 1, tn, tr);
         }
-        if (fast31)   // the matrix-core kernel (16 members at N = 10242: 14.5
-            add(0, 0, 0, 0, 0, 0);   // against 42 us per stage)
     }
     double best_t = 1e300;
     int found = -1;
+    bool timed_ensemble = false;
     for (size_t k = 0; k < cand.size(); ++k) {
+        // one candidate of those that run the matrix-core ensemble kernel: it
+        // cuts tiles of its own whatever shape they name
+        if (timed_ensemble && cand[k].tiled && ensemble_fills(base->n, members, base->ncu))
+            continue;
         double per = 0.0;
-        const int rc = time_options(base, cand[k], steps, &per);
+        bool ensemble = false;
+        const int rc = time_options(base, cand[k], steps, &per, &ensemble);
+        timed_ensemble |= ensemble;
         if (rc == SWE_HIP_EINVAL)
             continue;   // not possible on this mesh and node order (e.g. the
                         // resident kernel's tiles of a scattered order)
