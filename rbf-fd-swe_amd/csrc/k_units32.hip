@@ -375,8 +375,10 @@ bool units_plan32(SweUnits &u)
 template <int CHAINS>
 static void *streaming32(const SweUnits &u)
 {
-    if (u.mode == UM_GLOBAL && u.stream_nt)
-        return reinterpret_cast<void *>(&k_steps_units32<kUnits32Kept, UM_GLOBAL, CHAINS, true>);
+    // two chains end at 262144 nodes (151 MB of records), before stream_nt
+    if constexpr (CHAINS == 1)
+        if (u.mode == UM_GLOBAL && u.stream_nt)
+            return reinterpret_cast<void *>(&k_steps_units32<kUnits32Kept, UM_GLOBAL, 1, true>);
     return u.mode == UM_STREAM
                ? reinterpret_cast<void *>(&k_steps_units32<kUnits32Kept, UM_STREAM, CHAINS>)
                : reinterpret_cast<void *>(&k_steps_units32<kUnits32Kept, UM_GLOBAL, CHAINS>);
