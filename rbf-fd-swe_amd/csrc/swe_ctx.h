@@ -21,9 +21,6 @@ constexpr int kBlock = 256;            // threads per workgroup, stage kernels
 constexpr int kSingleBlock = 64;
 constexpr int kRingSlots = 4;          // pinned staging ring of a context
 constexpr size_t kRingBytes = 512 << 10;
-// States that the host reorders itself (swe_hip.hip, to_device).
-constexpr size_t kHostOrderMinBytes = 16 << 10;
-constexpr int kHostOrderMaxNodes = 4096;
 constexpr int kGraphCount = 4;         // captured step graphs per context
 // Resident whole-step kernel (k_resident.hip): one tile of <= 32 x
 // kResMaxWaves nodes per compute unit, whose stencils touch <= kResMaxRows

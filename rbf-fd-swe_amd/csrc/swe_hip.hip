@@ -1568,32 +1568,10 @@ static HostOrder host_order(const swe_hip_ctx *c, int member)
     return HostOrder{c->mesh->d_inv, c->lay.cfdl, c->lay.S, member, c->B};
 }
 
-static bool host_orders(const swe_hip_ctx *c, size_t bytes)
-{
-    return c->B == 1 && bytes >= kHostOrderMinBytes && c->n <= kHostOrderMaxNodes;
-}
-
-// f(element of the host layout, element of the single device state) for all.
-template <typename F>
-static void for_each_element(const swe_hip_ctx *c, F f)
-{
-    const std::vector<int> &perm = c->mesh->perm;
-    for (int d = 0; d < c->n; ++d) {
-        const int i = perm.empty() ? d : perm[d];
-        for (int v = 0; v < 4; ++v)
-            f(c->lay.svm(i, v), 4L * d + v);
-    }
-}
-
 // A state that needs reordering and fits the ring is reordered by a kernel
-// that reads or writes the pinned ring itself: 15 us for 10 KB, 18 for 140 KB,
-// 42 for 800 KB, where a DMA takes 8 to 21 and the kernel that has to wait for
-// it (or that it waits for) about 8 more.  A single state from 16 KB to 4096
-// nodes is reordered by the host on its way through the ring: 10.9 us in and
-// 11.1 out against 15.1 and 14.8 for 642 nodes in FP64, 13.2 and 15.0 against
-// 16.0 and 16.4 for 2562.  Below 16 KB a DMA takes longer (642 nodes in FP32:
-// 15.5 against 15.0), beyond 4096 nodes the loop (7292 in FP32 17.3 and 19.7
-// against 18.0 and 18.4; 10242 in FP64 23 and 33 against 24 and 26).
+// that reads or writes the pinned ring itself: 13 us for 20 KB, 19 for 328 KB,
+// 42 for 1.3 MB, where a DMA takes 8, 13 and 47 and the kernel that has to
+// wait for it (or that it waits for) about 8 more.
 template <typename T>
 static int to_device(swe_hip_ctx *c, int member, const T *host, T *dst)
 {
@@ -1603,12 +1581,6 @@ static int to_device(swe_hip_ctx *c, int member, const T *host, T *dst)
     if (same_order(c)) {
         if (int rc = ring_upload(c, dst, host, bytes))
             return rc;
-    } else if (host_orders(c, bytes)) {
-        if (int rc = stage_ring(c, bytes))
-            return rc;
-        T *ring = reinterpret_cast<T *>(c->ring);
-        for_each_element(c, [&](long h, long d) { ring[d] = host[h]; });
-        HIPCHK(hipMemcpyAsync(dst, ring, bytes, hipMemcpyHostToDevice, c->stream));
     } else {
         const T *from = static_cast<const T *>(c->d_stage);
         if (bytes <= kRingSlots * kRingBytes) {
@@ -1637,15 +1609,6 @@ static int from_device(swe_hip_ctx *c, int member, const T *src, T *host)
     if (same_order(c)) {
         if (int rc = ring_download(c, host, src, bytes))
             return rc;
-    } else if (host_orders(c, bytes)) {
-        if (int rc = stage_ring(c, bytes))
-            return rc;
-        const T *ring = reinterpret_cast<const T *>(c->ring);
-        HIPCHK(hipMemcpyAsync(c->ring, src, bytes, hipMemcpyDeviceToHost, c->stream));
-        HIPCHK(hipStreamSynchronize(c->stream));
-        if (int rc = check_resident(c))
-            return rc;
-        for_each_element(c, [&](long h, long d) { host[h] = ring[d]; });
     } else {
         const bool direct = bytes <= kRingSlots * kRingBytes;
         if (direct)
