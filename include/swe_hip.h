@@ -118,7 +118,8 @@ int swe_hip_eval_rhs32(swe_hip_ctx *ctx, int member, const float *K, float *F);
  * (a power of two 2..64 dividing members; 0 = the library's choice: in fast
  * mode with a 31-point stencil the matrix-core ensemble kernel, which keeps
  * weight and geometry records of 1.3 KB per node, else the largest such value;
- * 64 with a 31-point stencil = the member-pair kernel, two members per lane);
+ * 64 with a 31-point stencil = the member-pair kernel, two members per lane,
+ * also the library's choice where 64 divides the members of a small mesh);
  * share, when not NULL, is a context of the same mesh whose device copy of
  * the static data is reused (s may then be NULL): the static data stay
  * resident until the last context using them is destroyed.  Out-of-range
@@ -130,7 +131,15 @@ int swe_hip_eval_rhs32(swe_hip_ctx *ctx, int member, const float *K, float *F);
                                    form beyond that as far as a tile's rows
                                    fit the LDS (about 4000 nodes per compute
                                    unit), else PAIR with a 31-point
-                                   stencil, else QUADW (FP32: see below)     */
+                                   stencil, else QUADW (FP32: see below).
+                                   Both forms are cooperative launches that
+                                   need every compute unit at once: a launch
+                                   that is refused falls back to the stage
+                                   kernels, but one that starts beside
+                                   another process's work on the same device
+                                   can time out (SWE_HIP_EDEVICE, see
+                                   RESIDENT).  Name PAIR (FP32: LANE, PAIR)
+                                   to share a device between processes    */
 #define SWE_HIP_KERNEL_QUAD 1   /* FP32 single state: 4 lanes per node
                                    splitting the stencil slots (fast mode)   */
 #define SWE_HIP_KERNEL_LANE 2   /* FP32 single state: 1 lane per node        */
@@ -281,8 +290,9 @@ int swe_hip_get_state(swe_hip_ctx *ctx, int member, double *H);
 int swe_hip_rk_substep(swe_hip_ctx *ctx, int substep_id);
 
 /* Fast path: nsteps full RK4 steps (4 fused stage kernels per step, the RHS
- * never stored, K double-buffered), replayed from captured HIP graphs.
- * Same arithmetic per node as swe_hip_rk_substep. */
+ * never stored, K double-buffered), replayed from captured HIP graphs, or in
+ * one cooperative launch (SWE_HIP_KERNEL_AUTO, _RESIDENT).  Same arithmetic
+ * per node as swe_hip_rk_substep. */
 int swe_hip_rk_steps(swe_hip_ctx *ctx, int nsteps);
 
 /* No-allocation variant of swe_hip_rk_steps.  No counterpart in the

@@ -12,15 +12,19 @@
 // the RHS and the update need no exchange.
 //
 // A tile's distinct rows (4.2 per node at 32 nodes, against 8.9 for the 8-node
-// tiles of k_stage_tspec) go straight to LDS; the next member block's are on
-// their way while the RHS and the update run, and H and D are asked for before
-// the rows are waited for.  Two workgroups per compute unit overlap the rest.
-// 16 members make every access a whole 128-byte line: with 8 a launch fetched
-// 2.5 GB instead of 1.4 at N = 163842 x 64 (531 against 465 us).
+// tiles of k_stage_tspec) go straight to LDS; the next member block's are asked
+// for before the RHS runs.  What the compiler makes of it overlaps less than that
+// order promises: it drains the wave's memory counter before H and D are asked
+// for (their addresses and registers depend on loads and branches of the item
+// before), so every row copy and store has ended by then, and again before the
+// update, since the row copies after H and D are not a fixed number.  Across
+// tiles nothing is asked for early.  The two workgroups of a compute unit overlap
+// each other.  16 members make every access a whole 128-byte line: with 8 a
+// launch fetched 2.5 GB instead of 1.4 at N = 163842 x 64 (531 against 465 us).
 //
-// us per launch: N = 163842 x 64 465 against 495 (k_stage_tspec); of that the
-// traffic alone takes 354 (2.05 GB), the arithmetic alone 283 (221 without LDS
-// bank conflicts).  Against k_stage_members, the default before: N = 10242 x
+// us per launch: N = 163842 x 64 461 against 474 (k_stage_tspec, one box); of
+// that the traffic alone takes 354 (2.05 GB), the arithmetic alone 283 (221
+// without LDS bank conflicts).  Against k_stage_members, the default before: N = 10242 x
 // 2, 8, 16: 9.2, 9.8, 14.5 against 15, 22.6, 41.8; 40962 x 8, 32: 27, 67
 // against 80, 257; 642 x 2: 8.7 against 15.
 #include "units.h"
@@ -159,7 +163,7 @@ __global__ __launch_bounds__(256, 2) void k_stage_ensemble(DevEnsemble p, DevSta
             const int mem = MEMBERS * mb + 8 * half + 2 * j;   // this lane's two members
             const bool live = nl < tcount && mem < B;
             const long e = 4L * dn * B + (mem < B ? mem : 0);
-            // H and D on their way before the rows are waited for
+            // H and D on their way before the rows' barrier
             double2 hv[4], dv[4];
             constexpr int OWN = STAGE == ST_RHS || STAGE == ST_0 ? 0 : 8;
             __builtin_amdgcn_sched_barrier(0);
@@ -171,8 +175,8 @@ __global__ __launch_bounds__(256, 2) void k_stage_ensemble(DevEnsemble p, DevSta
                 }
             }
             __builtin_amdgcn_sched_barrier(0);
-            // this wave's rows are in LDS: at most the OWN loads after them
-            // (and the previous item's stores) are still out
+            // this wave's rows are in LDS: at most the OWN loads after them are
+            // still out (the compiler has already waited for all before those)
             wait_vm<OWN>();
             __syncthreads();
             // operator sums: acc[g][v] in lane (operator i, node b of group g,

@@ -18,7 +18,8 @@
 // The data.  One workgroup per compute unit and tile, 4 to 12 waves (streaming:
 // 8, two per SIMD with 256 registers): every wave keeps R units' weights (64
 // registers each) for the whole launch; what the registers do not hold is read again every
-// stage, RING 16-byte loads per lane in flight (nothing beyond the L2 moves
+// stage (UM_STREAM spills 23 registers, none inside the streamed loop), RING
+// 16-byte loads per lane in flight (nothing beyond the L2 moves
 // faster than 7.0 TB/s here, last-level cache or HBM, so a stage costs what it
 // re-reads).  UM_GLOBAL loads the weights non-temporally: the rest, 330 bytes a
 // node, then stays in the last-level cache (N = 655362 170 -> 133 us per stage;
@@ -323,8 +324,7 @@ void k_steps_units(DevUnits64 p)
                         constexpr int AHEAD = RING / 4;   // groups in flight
                         acc[q] = group(ring + 4 * (q % AHEAD), pv[q]);
 #pragma unroll
-                        for (int i = 0; i < 4; ++i)
-{
+                        for (int i = 0; i < 4; ++i) {
                             const double2 *from = q + AHEAD < 4
                                                       ? wc + 64 * (4 * (q + AHEAD) + i)
                                                       : wn + 64 * (4 * (q + AHEAD - 4) + i);

@@ -7,8 +7,9 @@
 // order: CHAINS == 1 the bits of k_stage_lane32, CHAINS == 2 (even and odd
 // slots apart, then added) those of k_stage_split32<2>, whichever AUTO used at
 // that size; two chains also halve the distance between dependent products.
-// A unit's weights take 32 registers: 4 units per wave stay (5 spill: 11.4
-// against 7.55 us at N = 163842).
+// A unit's weights take 32 registers: 4 units per wave stay (UM_GLOBAL spills 6
+// to 8 registers with them, UM_STREAM none; 5 spill: 11.4 against 7.55 us at N =
+// 163842).
 //
 // us per RK stage over 100 to 30 steps, against one lane per node resident up
 // to 65536 nodes and the stage kernels above:

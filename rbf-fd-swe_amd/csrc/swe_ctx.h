@@ -44,7 +44,7 @@ constexpr int kExactMaxPerCu = 64;
 // 642 to 163842 nodes).
 constexpr long long kMemberTileBytes = 2048;
 constexpr int kResMaxNbrs = 64;           // tiles one tile exchanges rows with (one wave)
-constexpr int kResAutoMinSteps = 4;       // AUTO contexts: shorter calls replay stage graphs
+constexpr int kResAutoMinSteps = 4;       // AUTO contexts: shorter calls launch the stage kernels
 
 // Host index macros of the reference (swe_config.h:21-54) at run time.
 struct HostLayout {
@@ -174,7 +174,7 @@ struct swe_hip_ctx {
     void *d_res_sync = nullptr;       // abort word + per-tile stage counts
     unsigned *h_res_abort = nullptr;  // pinned: wait time-out flag of the resident launches
     unsigned *d_res_abort = nullptr;  // its device address
-    bool res_auto = false;            // chosen by AUTO: short calls use the stage graphs
+    bool res_auto = false;            // chosen by AUTO: short calls launch the stage kernels
     long long res_stages = 0;         // stages counted since the counts were cleared
     int *d_res_nbrs = nullptr;        // [ntiles][kResMaxNbrs] tiles each tile waits for
     bool res_pending = false;         // a launch's flag is not checked yet

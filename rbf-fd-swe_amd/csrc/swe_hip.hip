@@ -1148,29 +1148,30 @@ int swe_hip_create_ex(const swe_hip_static *s, const swe_hip_options *o, swe_hip
             if (!rc)
                 rc = upload_waits(c, waits);
         } else {
-        // one tile of <= ceil(n / CUs) consecutive nodes per compute unit;
-        // two lanes per node in FP64, one in FP32
-        const int tmax = (c->n + c->ncu - 1) / c->ncu;
-        const int waves = fp32 ? (tmax + 63) / 64 : (tmax + 31) / 32;
-        if (c->nnbr != 31 || tmax > 32 * kResMaxWaves)
-            rc = fail(SWE_HIP_EINVAL, "the resident kernel takes 31-point stencils and at most "
-                                      + std::to_string(32 * kResMaxWaves)
-                                      + " nodes per compute unit");
-        std::vector<int> ts, us, ul;
-        if (!rc) {
-            c->res_block = 64 * waves;
-            rc = build_tiles(c, tmax, kResMaxRows, &ts, &us, &ul);
-        }
-        if (!rc && c->tiles.ntiles > c->ncu)
-            rc = fail(SWE_HIP_EINVAL, "the resident kernel's tiles exceed one per compute unit");
-        std::vector<int> waits;
-        if (!rc)
-            rc = resident_neighbours(tile_reads(c->n, ts, us, ul), &waits);
-        if (!rc)
-            rc = upload_waits(c, waits);
-        if (!rc)
-            c->res_lds = c->tiles.umax_used * (fp32 ? (int)(sizeof(float4) + sizeof(int))
-                                                    : 2 * (int)(sizeof(double2) + sizeof(int)));
+            // one tile of <= ceil(n / CUs) consecutive nodes per compute unit;
+            // two lanes per node in FP64, one in FP32
+            const int tmax = (c->n + c->ncu - 1) / c->ncu;
+            const int waves = fp32 ? (tmax + 63) / 64 : (tmax + 31) / 32;
+            if (c->nnbr != 31 || tmax > 32 * kResMaxWaves)
+                rc = fail(SWE_HIP_EINVAL, "the resident kernel takes 31-point stencils and at most "
+                                          + std::to_string(32 * kResMaxWaves)
+                                          + " nodes per compute unit");
+            std::vector<int> ts, us, ul;
+            if (!rc) {
+                c->res_block = 64 * waves;
+                rc = build_tiles(c, tmax, kResMaxRows, &ts, &us, &ul);
+            }
+            if (!rc && c->tiles.ntiles > c->ncu)
+                rc = fail(SWE_HIP_EINVAL,
+                          "the resident kernel's tiles exceed one per compute unit");
+            std::vector<int> waits;
+            if (!rc)
+                rc = resident_neighbours(tile_reads(c->n, ts, us, ul), &waits);
+            if (!rc)
+                rc = upload_waits(c, waits);
+            if (!rc)
+                c->res_lds = c->tiles.umax_used * (fp32 ? (int)(sizeof(float4) + sizeof(int))
+                                                        : 2 * (int)(sizeof(double2) + sizeof(int)));
         }
         if (!rc) {
             rc = dev_alloc(&c->bytes, &c->d_res_sync,
@@ -1477,10 +1478,12 @@ int swe_hip_move_member(swe_hip_ctx *c, int from, int to)
 
 }  // extern "C"
 
-// Host <-> device copies through a pinned ring of the context, 1 MB a slot:
-// the host copy of one slot runs beside the DMA of the others.  A pageable
-// copy of 64 KB to 1 MB costs the runtime 40 to 137 us, memcpy and DMA 8 to 21
-// (1.3 MB: 53 and 61 us in, 79 and 71 out; 5.2 MB: 159 and 183, 312 and 275).
+// Host <-> device copies through a pinned ring of the context, 512 KB a slot:
+// the host copy of one slot runs beside the DMA of the others.  set_state and
+// get_state in the host's node order, pageable copies against the ring: N = 40962
+// (1.3 MB) 93 and 121 us against 61 and 78, 163842 (5.2 MB) 254 and 440 against 242
+// and 256, 655362 (21 MB) 1449 and 1889 against 989 and 981; 82 KB 14 or 43 (by
+// where the buffer lies) against 12 and 14.
 static int stage_ring(swe_hip_ctx *c, size_t bytes)
 {
     if (c->ring_slots)
@@ -1569,9 +1572,11 @@ static HostOrder host_order(const swe_hip_ctx *c, int member)
 }
 
 // A state that needs reordering and fits the ring is reordered by a kernel
-// that reads or writes the pinned ring itself: 13 us for 20 KB, 19 for 328 KB,
-// 42 for 1.3 MB, where a DMA takes 8, 13 and 47 and the kernel that has to
-// wait for it (or that it waits for) about 8 more.
+// that reads or writes the pinned ring itself: 15 us for 20 KB, 24 for 328 KB,
+// 69 for 1.3 MB, memcpy included.  For 20 KB a host loop and a DMA take 11 with
+// nothing else on the stream, but a kernel that has to wait for a DMA (or that
+// it waits for) costs about 8 more: N = 642, one step, state in and out 48 us
+// against 50 (DMA in and out) and 64 (in only).
 template <typename T>
 static int to_device(swe_hip_ctx *c, int member, const T *host, T *dst)
 {
@@ -1838,9 +1843,9 @@ int swe_hip_rk_steps(swe_hip_ctx *c, int nsteps)
     if (!c || nsteps < 0)
         return fail(SWE_HIP_EINVAL, "rk_steps: bad ctx or nsteps");
     HIPCHK(hipSetDevice(c->dev));
-    // a resident context chosen by AUTO replays the stage graphs for calls
-    // too short to repay a launch (same arithmetic, bitwise); above 256 nodes
-    // per compute unit one step already does
+    // a resident context chosen by AUTO launches the stage kernels for calls
+    // too short to repay a cooperative launch (same arithmetic, bitwise); above
+    // 256 nodes per compute unit one step already does
     if (c->kernel == SWE_HIP_KERNEL_RESIDENT
         && (!c->res_auto || nsteps >= kResAutoMinSteps
             || c->n > 32 * kResMaxWaves * c->ncu)) {
