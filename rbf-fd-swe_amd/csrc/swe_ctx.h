@@ -8,6 +8,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -83,6 +84,7 @@ struct SweMesh {
     std::vector<int> perm;        // device node -> host node (empty: identity)
     int *d_inv = nullptr;         // host node -> device node, on the device
     std::vector<struct SweUnitRecords *> unit_records;   // those contexts use (swe_units.hip)
+    std::mutex records_mutex;     // guards them: contexts may live on several threads
     std::vector<double> h_xyz;    // node coordinates, device order, [3][n]
     std::vector<int> h_nbr;       // host copy of nbr, device order, [nnbr][n]
 };

@@ -7,7 +7,6 @@
 #include <cmath>
 #include <cstring>
 #include <memory>
-#include <mutex>
 #include <new>
 #include <numeric>
 
@@ -39,10 +38,6 @@ int prec_at(bool by_node, int m, int slot)
 
 }  // namespace
 
-// Guards the meshes' lists of records: contexts of one mesh may be destroyed by
-// different threads.
-static std::mutex g_records;
-
 static void free_records(SweUnits &u)
 {
     void *ptrs[] = {u.d_wrec, u.d_grec, u.d_tables};
@@ -57,7 +52,7 @@ void units_free(swe_hip_ctx *c)
     if (u.d_hd)
         (void)hipFree(u.d_hd);
     if (u.shared) {
-        std::lock_guard<std::mutex> lock(g_records);
+        std::lock_guard<std::mutex> lock(c->mesh->records_mutex);
         if (--u.shared->refs == 0) {
             std::vector<SweUnitRecords *> &all = c->mesh->unit_records;
             all.erase(std::find(all.begin(), all.end(), u.shared));
@@ -302,7 +297,7 @@ static int share_or_build(swe_hip_ctx *c, std::vector<std::vector<int>> *nbr_til
                           std::string *err)
 {
     std::vector<SweUnitRecords *> &all = c->mesh->unit_records;
-    std::lock_guard<std::mutex> lock(g_records);
+    std::lock_guard<std::mutex> lock(c->mesh->records_mutex);
     const auto at = std::find_if(all.begin(), all.end(), [&](const SweUnitRecords *r) {
         return r->form == form_of(c);
     });
