@@ -22,7 +22,7 @@
 // each other.  16 members make every access a whole 128-byte line: with 8 a
 // launch fetched 2.5 GB instead of 1.4 at N = 163842 x 64 (531 against 465 us).
 //
-// us per launch: N = 163842 x 64 461 against 474 (k_stage_tspec, one box); of
+// us per launch: N = 163842 x 64 461 against 474 (k_stage_tspec, side by side); of
 // that the traffic alone takes 354 (2.05 GB), the arithmetic alone 283 (221
 // without LDS bank conflicts).  Against k_stage_members, the default before: N = 10242 x
 // 2, 8, 16: 9.2, 9.8, 14.5 against 15, 22.6, 41.8; 40962 x 8, 32: 27, 67
