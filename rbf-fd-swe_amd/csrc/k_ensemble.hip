@@ -397,13 +397,14 @@ static void *ensemble_kernel(int stage)
     case ST_1: return reinterpret_cast<void *>(&k_stage_ensemble<ST_1, HALVES>);
     case ST_2: return reinterpret_cast<void *>(&k_stage_ensemble<ST_2, HALVES>);
     case ST_3: return reinterpret_cast<void *>(&k_stage_ensemble<ST_3, HALVES>);
+    case ST_3D: return reinterpret_cast<void *>(&k_stage_ensemble<ST_3D, HALVES>);
     default: return reinterpret_cast<void *>(&k_stage_ensemble<ST_RHS, HALVES>);
     }
 }
 
 int ensemble_prepare(swe_hip_ctx *c, std::string *err)
 {
-    for (int stage = 0; stage < 5; ++stage) {
+    for (int stage : {ST_0, ST_1, ST_2, ST_3, ST_RHS, ST_3D}) {
         void *fn = c->units.halves == 2 ? ensemble_kernel<2>(stage) : ensemble_kernel<1>(stage);
         if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, kUnitsMaxLds / 2)
             != hipSuccess) {

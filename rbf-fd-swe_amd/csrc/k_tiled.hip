@@ -44,6 +44,7 @@ void launch_tiled_stage(const swe_hip_ctx *c, int stage, const DevStage &st)
     case ST_1: by_flags<ST_1>(c, st); break;
     case ST_2: by_flags<ST_2>(c, st); break;
     case ST_3: by_flags<ST_3>(c, st); break;
+    case ST_3D: by_flags<ST_3D>(c, st); break;
     default: by_flags<ST_RHS>(c, st); break;
     }
 }

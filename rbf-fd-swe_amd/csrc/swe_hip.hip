@@ -204,13 +204,12 @@ void launch_fused_k(const swe_hip_ctx *c, int s, const T *kin, T *kout, bool kee
         DevStage32 st{};
         st.h = c->f_H;
         st.d = c->f_D;
-        st.keep_d = keep_d;
         st.src = s == 0 ? c->f_H : kin;
         st.out = s == 3 ? c->f_H : kout;
         st.c = s == 2 ? dt : (float)(dt / 2.0);
         st.c6 = dt / 6.0;
         st.dcoef = s == 0 ? 0.0f : (s == 3 ? 1.0f : 2.0f);
-        launch_fp32_stage(c, s, st);
+        launch_fp32_stage(c, keep_d && s == 3 ? ST_3D : s, st);
     } else {
         const double dt = c->dt;
         DevStage st{};
@@ -218,12 +217,11 @@ void launch_fused_k(const swe_hip_ctx *c, int s, const T *kin, T *kout, bool kee
         st.active = c->d_active;
         st.h = c->d_H;
         st.d = c->d_D;
-        st.keep_d = keep_d;
         st.src = s == 0 ? c->d_H : kin;
         st.out = s == 3 ? c->d_H : kout;
         st.c = s == 3 ? dt / 6.0 : (s == 2 ? dt : dt / 2.0);
         st.dcoef = s == 0 ? 0.0 : (s == 3 ? 1.0 : 2.0);
-        launch_stage(c, s, st);
+        launch_stage(c, keep_d && s == 3 ? ST_3D : s, st);
     }
 }
 

@@ -38,7 +38,6 @@ struct DevStage32 {
     float c;            // K = H + c*F (float dt/2.0, dt/2.0, dt)
     double c6;          // stage 3: H += (dt/6.0)*D in double
     float dcoef;        // D += dcoef*F (2, 2, 1)
-    int keep_d;         // stage 3 stores D too (drop-in substeps)
     int nblk;
 };
 
@@ -124,8 +123,8 @@ __device__ __forceinline__ void stage_update32(const DevStage32 &st, long e, con
                                           axpy32<EXACT>(d0.y, st.dcoef, F[1]),
                                           axpy32<EXACT>(d0.z, st.dcoef, F[2]),
                                           axpy32<EXACT>(d0.w, st.dcoef, F[3]));
-            if constexpr (STAGE == ST_3) {
-                if (st.keep_d)
+            if constexpr (STAGE == ST_3 || STAGE == ST_3D) {
+                if constexpr (STAGE == ST_3D)
                     *dp = dv;
                 *out = make_float4(update_h32<EXACT>(hv.x, st.c6, dv.x),
                                    update_h32<EXACT>(hv.y, st.c6, dv.y),
